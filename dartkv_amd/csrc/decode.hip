@@ -31,52 +31,6 @@ constexpr int kMaxGroup = 16;   // query heads per KV head
 constexpr int kMaxDim = 512;    // head_dim
 constexpr int kChanPerThread = kMaxDim / kThreads;
 
-__device__ __forceinline__ float key_value(const dkv_segment& s, int64_t bh, int c, int t, int D, const int32_t* inv,
-                                           int cache_dt, int meta) {
-  if (s.key_kind == DKV_KEY_DENSE) {
-    return dev_load((const void*)s.key[0], bh * s.key_bh[0] + (int64_t)t * D + c, cache_dt);
-  }
-  const int kg = s.key_group;
-  const int G = (s.tokens + kg - 1) / kg;
-  const int g = t / kg;
-  uint32_t code;
-  if (s.key_kind == DKV_KEY_UNIFORM) {
-    const int per_byte = 8 / s.key_bits;
-    const int pk = (G * kg + per_byte - 1) / per_byte;
-    const uint8_t byte = ((const uint8_t*)s.key[0])[bh * s.key_bh[0] + (int64_t)c * pk + t / per_byte];
-    code = (byte >> ((t % per_byte) * s.key_bits)) & ((1u << s.key_bits) - 1u);
-  } else {
-    const int nb = (kg + 3) / 4;
-    const int w = t % kg;
-    const uint8_t lo = ((const uint8_t*)s.key[0])[bh * s.key_bh[0] + ((int64_t)c * G + g) * nb + w / 4];
-    code = (lo >> ((w % 4) * 2)) & 3u;
-    const int slot = inv[c];
-    if (slot >= 0) {
-      const uint8_t hi = ((const uint8_t*)s.key[1])[bh * s.key_bh[1] + ((int64_t)slot * G + g) * nb + w / 4];
-      code |= ((hi >> ((w % 4) * 2)) & 3u) << 2;
-    }
-  }
-  const int64_t mi = (int64_t)c * G + g;
-  return dev_dequant(code, dev_load_meta((const void*)s.key[3], bh * s.key_bh[3] + mi, meta),
-                     dev_load_meta((const void*)s.key[4], bh * s.key_bh[4] + mi, meta), meta, cache_dt);
-}
-
-__device__ __forceinline__ float value_value(const dkv_segment& s, int64_t bh, int t, int c, int D, int cache_dt,
-                                             int meta) {
-  if (s.value_kind == DKV_VALUE_DENSE) {
-    return dev_load((const void*)s.value[0], bh * s.value_bh[0] + (int64_t)t * D + c, cache_dt);
-  }
-  const int vg = s.value_group;
-  const int Gv = (D + vg - 1) / vg;
-  const int per_byte = 8 / s.value_bits;
-  const int pv = (Gv * vg + per_byte - 1) / per_byte;
-  const uint8_t byte = ((const uint8_t*)s.value[0])[bh * s.value_bh[0] + (int64_t)t * pv + c / per_byte];
-  const uint32_t code = (byte >> ((c % per_byte) * s.value_bits)) & ((1u << s.value_bits) - 1u);
-  const int64_t mi = (int64_t)t * Gv + c / vg;
-  return dev_dequant(code, dev_load_meta((const void*)s.value[1], bh * s.value_bh[1] + mi, meta),
-                     dev_load_meta((const void*)s.value[2], bh * s.value_bh[2] + mi, meta), meta, cache_dt);
-}
-
 // MG is a compile-time bound on the query heads per KV head, so the per-head
 // state below stays in registers: DKV_FOR_HEAD unrolls over MG heads and skips
 // heads >= G.
@@ -156,7 +110,7 @@ __global__ void __launch_bounds__(kThreads) decode_split_general(DecodeParams p)
           }
         } else {
           for (int c = 0; c < D; ++c) {
-            const float kv = key_value(seg, bh, c, t, D, inv_s, cache_dt, meta);
+            const float kv = key_value(seg, bh, c, t, D, seg.key_kind == DKV_KEY_MIXED ? inv_s[c] : -1, cache_dt, meta);
             DKV_FOR_HEAD(h) logit[h] = fmaf(q_s[h * D + c], kv, logit[h]);
           }
         }
@@ -622,13 +576,17 @@ extern "C" int dkv_decode_attention(const dkv_decode_args* args, void* stream) {
     int rc = dkv_check_launch("dkv_decode_attention(dense)");
     if (rc) return rc;
   } else if (general_splits > 0) {
+    bool taken = false;
+    int rc = dkv::launch_tile_decode(p, s, &taken);
+    if (rc) return rc;
     const dim3 grid((unsigned)general_splits, (unsigned)a.Hkv, (unsigned)a.B);
-    if (p.group <= 1) hipLaunchKernelGGL(decode_split_general<1>, grid, dim3(kThreads), 0, s, p);
+    if (taken) {
+    } else if (p.group <= 1) hipLaunchKernelGGL(decode_split_general<1>, grid, dim3(kThreads), 0, s, p);
     else if (p.group <= 2) hipLaunchKernelGGL(decode_split_general<2>, grid, dim3(kThreads), 0, s, p);
     else if (p.group <= 4) hipLaunchKernelGGL(decode_split_general<4>, grid, dim3(kThreads), 0, s, p);
     else if (p.group <= 8) hipLaunchKernelGGL(decode_split_general<8>, grid, dim3(kThreads), 0, s, p);
     else hipLaunchKernelGGL(decode_split_general<16>, grid, dim3(kThreads), 0, s, p);
-    int rc = dkv_check_launch("dkv_decode_attention(split)");
+    rc = dkv_check_launch("dkv_decode_attention(split)");
     if (rc) return rc;
   }
   const int merge_threads = (int)(a.D < 64 ? 64 : (a.D > kThreads ? kThreads : ((a.D + 63) / 64) * 64));

@@ -34,6 +34,10 @@ int launch_fast_decode(const dkv_decode_args& a, int first, int count, int np, i
 int uniform_decode_max_loads(int kb, int vb, int gv);
 int launch_uniform_decode(const dkv_decode_args& a, int first, int count, int kb, int vb, int vg, int splits,
                           int split_stride, hipStream_t stream, const FusedRest* fused = nullptr);
+// The segments of a decode call outside the page kernels' run, for 16-bit
+// caches (decode_tiles.hip); *taken is false, and nothing is launched, when
+// they are not of the forms that kernel reads.
+int launch_tile_decode(const DecodeParams& d, hipStream_t stream, bool* taken);
 // LDS bytes of one wave of the uniform page kernel.
 size_t uniform_decode_wave_lds_bytes(int kb, int vb, int gv);
 

@@ -1,0 +1,124 @@
+"""The tile decode kernel (16-bit caches outside the page kernels' forms) against the oracle, at the edges of its
+tiles and of its dispatch.
+
+Its weights stay fp32 and its products are exact, so its error is that of fp32 logits and sums: a logit of size L
+carries about L 2^-24 (L below 50 here: 3e-6 relative in its weight) and the sums over at most 1,200 tokens the
+same order, under the 1e-5 that fp32 caches are held to.
+"""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda"
+BF, FP = torch.bfloat16, torch.float16
+
+
+def _rel_err(a, b):
+    a, b = a.detach().float().cpu().flatten(2), b.detach().float().cpu().flatten(2)
+    return float(((a - b).abs().amax(-1) / b.abs().amax(-1).clamp_min(1e-30)).max())
+
+
+def _run(B, Hkv, G, D, T, dtype, cfg, updates=(), n_splits=None):
+    import dartkv_amd as dart
+    from dartkv_amd import synthetic
+    from oracle import dart_oracle as O
+    cfg = dict(dict(bits=2, page_size=128, key_group_size=128, value_group_size=64, sink_tokens=32,
+                    hold_partial_pages=True, metadata_dtype=torch.float16), **cfg)
+    k, v, q = synthetic.outlier_kv(B, Hkv, T, D, query_heads=Hkv * G, dtype=dtype, seed=7 + T + G, outliers=D // 16)
+    oc, cache = O.OracleCache(O.OracleConfig(**cfg)), dart.DartKVCache(dart.DartKVCacheConfig(**cfg))
+    start = 0
+    for n in (*updates, T - sum(updates)):
+        part = slice(start, start + n)
+        oc.append(k[..., part, :], v[..., part, :])
+        cache.append(k[..., part, :].to(DEV), v[..., part, :].to(DEV))
+        start += n
+    ref = O.streamed_attention(q, oc, return_fp32=True)[1]
+    out = torch.empty(B, Hkv * G, D, dtype=torch.float32, device=DEV)
+    print("case", B, Hkv, G, D, T, dtype, cfg, n_splits, flush=True)
+    dart.decode_attention(q.to(DEV), cache, out_f32=out, fast=False, n_splits=n_splits)
+    torch.cuda.synchronize()
+    return _rel_err(out.unsqueeze(2), ref)
+
+
+@pytest.mark.parametrize("G,D,T,dtype,cfg", [
+    # head ratios: the padded rows of 4, 8 and 16, on Dart pages
+    (1, 128, 700, BF, dict(promote_ratio=0.25)),
+    (3, 128, 700, FP, dict(promote_ratio=0.25)),
+    (5, 64, 700, BF, dict(promote_ratio=0.25)),
+    (8, 128, 700, FP, dict(promote_ratio=0.25)),
+    (9, 64, 700, FP, dict(promote_ratio=0.25)),
+    (16, 128, 700, BF, dict(promote_ratio=0.25)),
+    # promoted counts: one, not a multiple of 8 or 32, more than one block of 32, every channel
+    (4, 128, 500, BF, dict(promote_ratio=0.008)),
+    (4, 64, 500, FP, dict(promote_ratio=0.3)),
+    (6, 128, 500, BF, dict(promote_ratio=0.3, key_group_size=64)),
+    (4, 128, 500, FP, dict(promote_ratio=0.6, key_group_size=32)),
+    (4, 128, 500, BF, dict(promote_ratio=1.0)),
+    # code widths, key groups (several per tile, a padded one, one wider than the page), value groups
+    (4, 128, 500, BF, dict(key_group_size=32, value_group_size=32)),
+    (4, 64, 500, FP, dict(key_group_size=256, value_group_size=16)),
+    (7, 128, 500, BF, dict(bits=4, key_group_size=64, value_group_size=48)),
+    (2, 64, 500, BF, dict(bits=4, key_group_size=32, value_group_size=64)),
+    (4, 128, 500, FP, dict(bits=8, key_group_size=64, value_group_size=128)),
+    (12, 64, 500, BF, dict(bits=8, key_group_size=32, value_group_size=32)),
+    # segments that are not one full tile: short pages, pages of 256 tokens (two and four tiles), partial pages
+    (4, 128, 333, BF, dict(page_size=40, key_group_size=32, promote_ratio=0.25)),
+    (4, 128, 1200, FP, dict(page_size=256, key_group_size=128, promote_ratio=0.25)),
+    (4, 64, 1200, BF, dict(page_size=256, key_group_size=64, bits=8)),
+    (4, 128, 1000, BF, dict(hold_partial_pages=False, promote_ratio=0.25)),
+    (3, 128, 1000, FP, dict(hold_partial_pages=False, bits=4, key_group_size=64)),
+    (3, 64, 33, BF, dict(hold_partial_pages=False)),                 # one packed token
+    # dense tokens only, none, and more than a tile of them
+    (3, 64, 20, BF, {}),
+    (9, 128, 160, FP, {}),
+    (4, 64, 400, BF, dict(sink_tokens=0)),
+    (4, 128, 900, BF, dict(sink_tokens=300, local_tokens=200, promote_ratio=0.25)),
+])
+def test_tile_kernel_vs_oracle(G, D, T, dtype, cfg):
+    assert _run(2, 2, G, D, T, dtype, cfg) <= 1e-5
+
+
+@pytest.mark.parametrize("n_splits", [1, 2, 5, 64])
+def test_tile_kernel_split_counts(n_splits):
+    """Splits that hold several pages, a page and the dense pieces, or nothing but a dense piece."""
+    assert _run(1, 2, 6, 128, 900, BF, dict(promote_ratio=0.25), n_splits=n_splits) <= 1e-5
+
+
+def test_rest_of_a_page_run_takes_the_tile_kernel():
+    """A short last page beside a run the page kernel takes: the run's records and the tile kernel's meet in one merge
+    (the page kernel's bar, its weights are 16-bit)."""
+    import dartkv_amd as dart
+    from dartkv_amd import synthetic
+    from oracle import dart_oracle as O
+    cfg = dict(bits=2, page_size=128, key_group_size=128, value_group_size=64, sink_tokens=32, promote_ratio=0.25,
+               hold_partial_pages=False, metadata_dtype=torch.float16)
+    k, v, q = synthetic.outlier_kv(2, 4, 1000, 128, query_heads=16, dtype=BF, seed=3)
+    oc, cache = O.OracleCache(O.OracleConfig(**cfg)), dart.DartKVCache(dart.DartKVCacheConfig(**cfg))
+    oc.append(k, v)
+    cache.append(k.to(DEV), v.to(DEV))
+    ref = O.streamed_attention(q, oc, return_fp32=True)[1]
+    out = torch.empty(2, 16, 128, dtype=torch.float32, device=DEV)
+    dart.decode_attention(q.to(DEV), cache, out_f32=out)
+    torch.cuda.synchronize()
+    assert _rel_err(out.unsqueeze(2), ref) <= 2e-3
+
+
+@pytest.mark.parametrize("dtype", [BF, FP])
+def test_tile_kernel_keeps_infinite_dense_values(dtype):
+    """A dense tail token with an infinite value gives infinities where fp32 attention does, and no NaN from the
+    positions past the tail."""
+    import dartkv_amd as dart
+    g = torch.Generator().manual_seed(1)
+    k, v = (torch.randn(1, 2, 300, 64, generator=g).to(dtype) for _ in range(2))
+    v[0, 1, 299, 5] = float("inf")
+    q = torch.randn(1, 6, 1, 64, generator=g).to(dtype)
+    cache = dart.DartKVCache(dart.DartKVCacheConfig(bits=4, page_size=128, key_group_size=64, value_group_size=64,
+                                                    hold_partial_pages=True))
+    cache.append(k.to(DEV), v.to(DEV))
+    out = dart.fused_dart_attention(q.to(DEV), cache).cpu()
+    torch.cuda.synchronize()
+    expected = torch.zeros(1, 6, 1, 64, dtype=torch.bool)
+    expected[0, 3:, 0, 5] = True
+    assert torch.equal(torch.isinf(out), expected) and not torch.isnan(out).any()
