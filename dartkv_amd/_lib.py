@@ -26,7 +26,7 @@ KEY_DENSE, KEY_UNIFORM, KEY_MIXED = 0, 1, 2
 VALUE_DENSE, VALUE_UNIFORM = 0, 1
 SELECT_MAGNITUDE, SELECT_VARIANCE, SELECT_GIVEN = 0, 1, 2
 
-ABI_VERSION = 13
+ABI_VERSION = 14
 
 _DTYPE_CODES = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2, torch.float64: 3}
 # element types the kernels read and write (sources, outputs, metadata)
@@ -107,6 +107,19 @@ class DecodeArgs(ctypes.Structure):
 assert ctypes.sizeof(Segment) == 160
 
 
+class MaterializeArgs(ctypes.Structure):
+    _fields_ = [
+        ("segments", ctypes.c_void_p), ("chunks", ctypes.c_void_p), ("n_chunks", ctypes.c_int64),
+        ("tail", Segment), ("tail_start", ctypes.c_int64),
+        ("B", ctypes.c_int64), ("H", ctypes.c_int64), ("D", ctypes.c_int64), ("tokens", ctypes.c_int64),
+        ("dtype", ctypes.c_int64), ("meta_dtype", ctypes.c_int64),
+        ("keys", ctypes.c_void_p), ("values", ctypes.c_void_p),
+    ]
+
+
+MATERIALIZE_CHUNK = 128
+
+
 class DecodePrepArgs(ctypes.Structure):
     _fields_ = [
         ("qkv", ctypes.c_void_p), ("qkv_sb", ctypes.c_int64),
@@ -134,7 +147,7 @@ EXPORTED = (
     "dkv_quantize_key_pages",
     "dkv_dequantize_rows",
     "dkv_dequantize_mixed", "dkv_decode_workspace_bytes", "dkv_decode_attention", "dkv_decode_attention_noalloc",
-    "dkv_decode_scratch_bytes", "dkv_decode_prep", "dkv_copy_token_blocks",
+    "dkv_decode_scratch_bytes", "dkv_decode_prep", "dkv_copy_token_blocks", "dkv_materialize",
 )
 
 _lib: Optional[ctypes.CDLL] = None
@@ -170,11 +183,12 @@ def load() -> ctypes.CDLL:
         lib.dkv_decode_scratch_bytes.argtypes = []
         lib.dkv_decode_scratch_bytes.restype = i64
         lib.dkv_decode_prep.argtypes = [ctypes.POINTER(DecodePrepArgs), vp]
+        lib.dkv_materialize.argtypes = [ctypes.POINTER(MaterializeArgs), vp]
         lib.dkv_copy_token_blocks.argtypes = [ctypes.POINTER(CopyBlock), i64, vp]
         for name in ("dkv_quantize_rows", "dkv_quantize_row_blocks", "dkv_quantize_value_rows", "dkv_quantize_key_pages",
                      "dkv_dequantize_rows",
                      "dkv_dequantize_mixed", "dkv_decode_attention", "dkv_decode_attention_noalloc",
-                     "dkv_decode_prep", "dkv_copy_token_blocks"):
+                     "dkv_decode_prep", "dkv_copy_token_blocks", "dkv_materialize"):
             getattr(lib, name).restype = ctypes.c_int
         if lib.dkv_abi_version() != ABI_VERSION:
             raise RuntimeError("libdartkv_hip.so ABI version mismatch; rebuild it")

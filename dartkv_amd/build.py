@@ -21,7 +21,7 @@ PKG = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(PKG, "csrc")
 LIB = os.path.join(PKG, "libdartkv_hip.so")
 SOURCES = ["capi.hip", "quantize.hip", "decode.hip", "decode_fast.hip", "decode_uniform.hip", "decode_tiles.hip",
-           "prep.hip", "copy.hip"]
+           "materialize.hip", "prep.hip", "copy.hip"]
 ARCH = os.environ.get("DKV_OFFLOAD_ARCH", "gfx950")
 
 

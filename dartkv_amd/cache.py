@@ -377,7 +377,23 @@ class _DecodePlan:
          self.fast_value_bits) = fast
         self.rest_dense = rest_dense
         self.host_table = None  # the descriptors in host memory (dkv_decode_args.segments_host)
+        self._chunks: Optional[torch.Tensor] = None
         self.call_layouts: dict = {}  # decode call shape -> (DecodeArgs template, workspace bytes)
+
+    def chunks(self) -> torch.Tensor:
+        """int32 [n, 3] on the device: dkv_materialize's chunks (entry, first token, output token) of the table;
+        made on the first read-back of this layout."""
+        if self._chunks is None:
+            rows, start = [], 0
+            for i in range(self.count):
+                n = self.host_table[i].tokens
+                rows += [(i, t, start + t) for t in range(0, n, _lib.MATERIALIZE_CHUNK)]
+                start += n
+            self._chunks = torch.tensor(rows, dtype=torch.int32).reshape(len(rows), 3).to(self.device)
+        return self._chunks
+
+    def chunks_ready(self) -> bool:
+        return self._chunks is not None or self.table is None
 
 
 class DartKVCache:
@@ -590,6 +606,9 @@ class DartKVCache:
     def get(self) -> Tuple[torch.Tensor, torch.Tensor]:
         if self._seen_tokens == 0:
             raise RuntimeError("DartKVCache is empty; call update() before get()")
+        dense = self._materialize_all()
+        if dense is not None:
+            return dense
         keys = [_materialize(s) for s in self._keys]
         values = [_materialize(s) for s in self._values]
         if self._pending_key is not None:
@@ -597,6 +616,43 @@ class DartKVCache:
         if self._pending_value is not None:
             values.append(self._pending_value)
         return torch.cat(keys, dim=-2), torch.cat(values, dim=-2)
+
+    def _materialize_all(self) -> Optional[Tuple[torch.Tensor, torch.Tensor]]:
+        """The contents as dense tensors from one launch over the descriptor table (dkv_materialize), or None
+        where the segments are dequantized one by one: a cache on the host, Kitty value windows (the two
+        tracks are not cut alike), and under capture a table that is not built yet (its upload cannot be
+        captured)."""
+        device, c = self._device, self.config
+        if device is None or device.type != "cuda" or c.value_local_tokens:
+            return None
+        plan = self._decode_plan_cache
+        ready = plan is not None and plan.version == self._sealed_version and plan.device == device
+        if not (ready and plan.chunks_ready()) and torch.cuda.is_current_stream_capturing():
+            return None
+        plan = self.decode_plan(device)
+        B, H, D = self._shape
+        a = _lib.MaterializeArgs()
+        if plan.table is not None:
+            chunks = plan.chunks()
+            a.segments, a.chunks, a.n_chunks = plan.table.data_ptr(), chunks.data_ptr(), chunks.shape[0]
+            stream = torch.cuda.current_stream(device)
+            plan.table.record_stream(stream)
+            chunks.record_stream(stream)
+        pk, pv = self._pending_key, self._pending_value
+        if plan.tail_is_pending and pk is not None:
+            keep: list = []
+            a.tail.tokens = pk.shape[-2]
+            a.tail.key_kind, a.tail.value_kind = _lib.KEY_DENSE, _lib.VALUE_DENSE
+            a.tail.key[0], a.tail.key_bh[0] = _dense_block(pk, keep)
+            a.tail.value[0], a.tail.value_bh[0] = _dense_block(pv, keep)
+            a.tail_start = plan.n_tokens
+        a.B, a.H, a.D, a.tokens = B, H, D, self._seen_tokens
+        a.dtype, a.meta_dtype = _lib.dtype_code(self._dtype), _lib.dtype_code(c.metadata_dtype)
+        keys = torch.empty(B, H, self._seen_tokens, D, dtype=self._dtype, device=device)
+        values = torch.empty_like(keys)
+        a.keys, a.values = keys.data_ptr(), values.data_ptr()
+        _lib.check(_lib.load().dkv_materialize(a, _lib.stream_ptr(device)), "dkv_materialize")
+        return keys, values
 
     @property
     def key_states(self) -> torch.Tensor:

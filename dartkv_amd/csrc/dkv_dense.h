@@ -38,14 +38,17 @@ __device__ __forceinline__ dkv_segment general_segment(const DecodeParams& p, in
   return p.a.segments[v < p.skip_first ? v : v + p.skip_count];
 }
 
-// Key element (token t, channel c) of a segment of any kind, dequantized with
-// the reference's chain, as fp32.  `slot`: c's slot among the promoted channels
-// of a Dart page (-1: none).
-__device__ __forceinline__ float key_value(const dkv_segment& s, int64_t bh, int c, int t, int D, int slot,
-                                           int cache_dt, int meta) {
-  if (s.key_kind == DKV_KEY_DENSE) {
-    return dev_load((const void*)s.key[0], bh * s.key_bh[0] + (int64_t)t * D + c, cache_dt);
-  }
+// One packed element: its code, and the place of its scale and zero point
+// within their (batch, kv head) blocks.
+struct PackedElem {
+  uint32_t code;
+  const void *scale, *zero;
+  int64_t at;
+};
+
+// Key element (token t, channel c) of a packed segment.  `slot`: c's slot among
+// the promoted channels of a Dart page (-1: none).
+__device__ __forceinline__ PackedElem key_code(const dkv_segment& s, int64_t bh, int c, int t, int D, int slot) {
   const int kg = s.key_group;
   const int G = (s.tokens + kg - 1) / kg;
   const int g = t / kg;
@@ -66,24 +69,37 @@ __device__ __forceinline__ float key_value(const dkv_segment& s, int64_t bh, int
     }
   }
   const int64_t mi = (int64_t)c * G + g;
-  return dev_dequant(code, dev_load_meta((const void*)s.key[3], bh * s.key_bh[3] + mi, meta),
-                     dev_load_meta((const void*)s.key[4], bh * s.key_bh[4] + mi, meta), meta, cache_dt);
+  return PackedElem{code, (const void*)s.key[3], (const void*)s.key[4], mi};
 }
 
-__device__ __forceinline__ float value_value(const dkv_segment& s, int64_t bh, int t, int c, int D, int cache_dt,
-                                             int meta) {
-  if (s.value_kind == DKV_VALUE_DENSE) {
-    return dev_load((const void*)s.value[0], bh * s.value_bh[0] + (int64_t)t * D + c, cache_dt);
-  }
+__device__ __forceinline__ PackedElem value_code(const dkv_segment& s, int64_t bh, int t, int c, int D) {
   const int vg = s.value_group;
   const int Gv = (D + vg - 1) / vg;
   const int per_byte = 8 / s.value_bits;
   const int pv = (Gv * vg + per_byte - 1) / per_byte;
   const uint8_t byte = ((const uint8_t*)s.value[0])[bh * s.value_bh[0] + (int64_t)t * pv + c / per_byte];
   const uint32_t code = (byte >> ((c % per_byte) * s.value_bits)) & ((1u << s.value_bits) - 1u);
-  const int64_t mi = (int64_t)t * Gv + c / vg;
-  return dev_dequant(code, dev_load_meta((const void*)s.value[1], bh * s.value_bh[1] + mi, meta),
-                     dev_load_meta((const void*)s.value[2], bh * s.value_bh[2] + mi, meta), meta, cache_dt);
+  return PackedElem{code, (const void*)s.value[1], (const void*)s.value[2], (int64_t)t * Gv + c / vg};
+}
+
+// The same elements of a segment of any kind, dequantized with the reference's
+// chain, as fp32.
+__device__ __forceinline__ float key_value(const dkv_segment& s, int64_t bh, int c, int t, int D, int slot,
+                                           int cache_dt, int meta) {
+  if (s.key_kind == DKV_KEY_DENSE)
+    return dev_load((const void*)s.key[0], bh * s.key_bh[0] + (int64_t)t * D + c, cache_dt);
+  const PackedElem e = key_code(s, bh, c, t, D, slot);
+  return dev_dequant(e.code, dev_load_meta(e.scale, bh * s.key_bh[3] + e.at, meta),
+                     dev_load_meta(e.zero, bh * s.key_bh[4] + e.at, meta), meta, cache_dt);
+}
+
+__device__ __forceinline__ float value_value(const dkv_segment& s, int64_t bh, int t, int c, int D, int cache_dt,
+                                             int meta) {
+  if (s.value_kind == DKV_VALUE_DENSE)
+    return dev_load((const void*)s.value[0], bh * s.value_bh[0] + (int64_t)t * D + c, cache_dt);
+  const PackedElem e = value_code(s, bh, t, c, D);
+  return dev_dequant(e.code, dev_load_meta(e.scale, bh * s.value_bh[1] + e.at, meta),
+                     dev_load_meta(e.zero, bh * s.value_bh[2] + e.at, meta), meta, cache_dt);
 }
 
 constexpr int kDenseWaves = 4;

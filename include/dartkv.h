@@ -344,6 +344,33 @@ typedef struct dkv_decode_args {
 } dkv_decode_args;
 
 /*
+ * A cache's contents as dense tensors: every segment dequantized (or copied)
+ * to its tokens of keys and values, both [B][H][tokens][D] in `dtype` (the
+ * cache's; dense segments hold it).  `chunks` is a device array of n_chunks
+ * triples (segment index, first token, output token): tokens [first, min(first
+ * + 128, segment tokens)) of that segment go to output tokens [output token,
+ * ...); first is a multiple of 128.  The tail (by value, tokens 0: none) goes
+ * to output tokens from tail_start.  D up to 16384.
+ *
+ * Replaces reference src/dart/cache.py:192-204 (`get`), which dequantizes and
+ * concatenates segment by segment (src/dart/quantization.py:96-109,
+ * src/dart/mixed.py:72-94).
+ */
+typedef struct dkv_materialize_args {
+  const dkv_segment* segments;
+  const int32_t* chunks;
+  int64_t n_chunks;
+  dkv_segment tail;
+  int64_t tail_start;
+  int64_t B, H, D, tokens;
+  int64_t dtype, meta_dtype;
+  void* keys;
+  void* values;
+} dkv_materialize_args;
+
+int dkv_materialize(const dkv_materialize_args* args, void* stream);
+
+/*
  * Decode-step preparation for the Qwen3 adapter, one new token per sequence:
  * qkv[b] holds the projected query heads, key heads and value heads of
  * sequence b (Hq + 2 Hkv rows of D = 128 elements, row stride qkv_sb elements,

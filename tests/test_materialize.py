@@ -1,0 +1,46 @@
+"""The one-launch read-back of a cache (dkv_materialize) against its segments dequantized one by one, bit for bit, over
+its load forms (octets of 2-, 4- and 8-bit codes, Dart pages, dense pieces) and the element-wise form of every other
+layout and type, at partial chunks."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda"
+BF, FP, F32, F64 = torch.bfloat16, torch.float16, torch.float32, torch.float64
+
+
+@pytest.mark.parametrize("T,D,dtype,cfg", [
+    (1000, 128, BF, dict(promote_ratio=0.25, sink_tokens=32, hold_partial_pages=True)),
+    (1001, 64, FP, dict(promote_ratio=0.3, key_group_size=64, value_group_size=32)),
+    (517, 128, FP, dict(bits=4, key_group_size=32, sink_tokens=3, hold_partial_pages=True)),
+    (300, 64, BF, dict(bits=8, value_group_size=24)),
+    (256, 128, F32, dict(key_group_size=32, value_group_size=32, sink_tokens=2)),
+    (700, 128, BF, dict(page_size=300, key_group_size=104, bits=4, sink_tokens=200)),   # chunks inside a page
+    (130, 8, F32, dict(page_size=16, key_group_size=8, value_group_size=8, promote_ratio=0.25)),
+    # element by element: group sizes that are not octets, other metadata, float64, an odd head_dim
+    (90, 32, BF, dict(page_size=8, key_group_size=3, value_group_size=6, promote_ratio=0.25)),
+    (200, 64, FP, dict(metadata_dtype=BF, bits=4)),
+    (200, 64, F64, dict(metadata_dtype=F64, bits=2, promote_ratio=0.25)),
+    (60, 20, F32, dict(page_size=16, key_group_size=8, value_group_size=8, bits=4)),
+    (140, 64, BF, dict(local_tokens=4, page_size=32, key_group_size=32)),
+])
+def test_get_equals_the_segments(T, D, dtype, cfg):
+    import dartkv_amd as dart
+    from dartkv_amd.cache import _materialize
+    g = torch.Generator().manual_seed(T)
+    k, v = (torch.randn(2, 3, T, D, generator=g, dtype=F32).to(dtype).to(DEV) for _ in range(2))
+    cache = dart.DartKVCache(dart.DartKVCacheConfig(**cfg))
+    cache.append(k[..., :T - 1, :], v[..., :T - 1, :])
+    cache.append(k[..., T - 1:, :], v[..., T - 1:, :])
+    print("case", T, D, dtype, cfg, flush=True)
+    segments = cache.iter_segments()
+    keys = torch.cat([_materialize(ks) for ks, _ in segments], dim=-2)
+    values = torch.cat([_materialize(vs) for _, vs in segments], dim=-2)
+    got_k, got_v = cache.get()
+    torch.cuda.synchronize()
+    assert got_k.is_contiguous() and got_k.dtype == dtype and got_k.shape == (2, 3, T, D)
+    bits = torch.int64 if dtype == F64 else torch.int32 if dtype == F32 else torch.int16
+    assert torch.equal(got_k.view(bits), keys.contiguous().view(bits))
+    assert torch.equal(got_v.view(bits), values.contiguous().view(bits))
