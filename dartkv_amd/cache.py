@@ -24,8 +24,6 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
-import threading
-import time
 from dataclasses import dataclass, fields as dataclass_fields
 from itertools import accumulate
 from typing import TYPE_CHECKING, List, Optional, Tuple, Union
@@ -33,6 +31,7 @@ from typing import TYPE_CHECKING, List, Optional, Tuple, Union
 import torch
 
 from . import _lib
+from .finite import drain as _drain, nonfinite_flags as _nonfinite_flags
 from .mixed import MixedQuantizedKey, launch_key_pages, promoted_count, random_channels
 from .pool import PagePool, PoolKeys, PoolMixedKey, PoolValues
 from .quantization import QuantizedTensor
@@ -131,47 +130,6 @@ class DartKVCacheConfig:
     @property
     def resolved_value_group_size(self) -> int:
         return self.value_group_size if self.value_group_size is not None else self.group_size
-
-
-_flag_store = threading.local()
-
-
-def _nonfinite_flags(device: torch.device) -> torch.Tensor:
-    """int32 [2] flags (keys, values) for the quantizers' non-finite reports on ``device``, one pair per
-    thread and device and shared by that thread's caches (an append's scope reads them before the next
-    append can start on the thread).  They live in pinned host memory, which the kernels write directly:
-    reading them after the append's launches takes a stream synchronization and no device-to-host copy.
-    They are zero between appends."""
-    flags = getattr(_flag_store, "flags", None)
-    if flags is None:
-        flags = _flag_store.flags = {}
-    t = flags.get(device)
-    if t is None:
-        with torch.inference_mode(False):  # updated in place whatever mode a later append runs in
-            t = flags[device] = torch.zeros(2, dtype=torch.int32, pin_memory=True)
-    return t
-
-
-_DRAIN_SPIN_S = 1e-3  # poll this long, then block (a long append does not keep a CPU core busy)
-
-
-def _drain(device: torch.device) -> None:
-    """Wait until the device's current stream has run everything enqueued so far, by polling an event
-    recorded on it: the wait ends within a few microseconds of the GPU finishing, where a blocking
-    stream synchronization returns about 10-15 µs later (measured on MI355X).  Work still running
-    after ``_DRAIN_SPIN_S`` of polling is waited for with a blocking synchronization."""
-    events = getattr(_flag_store, "events", None)
-    if events is None:
-        events = _flag_store.events = {}
-    ev = events.get(device)
-    if ev is None:
-        ev = events[device] = torch.cuda.Event()
-    ev.record(torch.cuda.current_stream(device))
-    t0 = time.perf_counter()
-    while not ev.query():
-        if time.perf_counter() - t0 > _DRAIN_SPIN_S:
-            ev.synchronize()
-            return
 
 
 def _storage(shape, dtype: torch.dtype, device) -> torch.Tensor:

@@ -892,6 +892,128 @@ __global__ void __launch_bounds__(kThreads) quantize_key_pages_tiled(KeyParams k
   }
 }
 
+// Uniform keys straight from registers: groups of 32, 64 or 128 tokens,
+// head_dims that fill whole 128-byte row pieces, pages of any token count.  A
+// wave takes a block of 128 tokens x 128 bytes of channels: lane (half, cl)
+// reads 64 tokens of NCH channels, one dword each (32 lanes read one 128-byte
+// piece of a row), all 64 loads in flight; the two halves of a 128-token group
+// meet with one shuffle, narrower groups lie inside a lane.  Every source byte
+// is read once and nothing goes through LDS, where the tiled kernel has
+// barriers between its phases and divides per element.  Bound by the reads.
+//
+// Tokens past the page repeat its last one, as the padding does
+// (quantization.py:174-177).
+struct ColumnParams {
+  const void* src;
+  int64_t sb, sh, st;      // element strides (channels are contiguous)
+  int H, D, T, G, pk;      // heads, head_dim, tokens per page, groups per page, packed bytes per channel
+  int blocks, chunks;      // 128-token blocks per page, 128-byte channel pieces per row
+  int64_t items;           // waves of work: pages x batch x heads x blocks x chunks
+  int64_t bhs;
+  uint8_t* low;
+  void *scale, *zero;
+  int64_t low_page_stride, scale_page_stride, zero_page_stride;
+  int meta_dtype;
+  uint32_t* nonfinite;
+};
+
+constexpr int kColumnTokens = 128;
+
+template <int SRC, int BITS, int KG>
+__global__ void __launch_bounds__(kThreads, 4) quantize_key_columns(ColumnParams p) {
+  constexpr int NCH = SRC == kF32 ? 1 : 2;
+  constexpr int SG = KG < 64 ? KG : 64;  // tokens of a group in one lane
+  constexpr float qmax = (float)((1 << BITS) - 1), inv_qmax = 1.0f / (float)((1 << BITS) - 1);
+  const int64_t item = (int64_t)blockIdx.x * (kThreads / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (item >= p.items) return;
+  const int lane = threadIdx.x & 63, half = lane >> 5;
+  // channel pieces of one block are neighbouring waves: they read the same rows
+  const int chunk = (int)(item % p.chunks);
+  const int64_t r0 = item / p.chunks;
+  const int block = (int)(r0 % p.blocks);
+  const int64_t r1 = r0 / p.blocks, bh = r1 % p.bhs, page = r1 / p.bhs;
+  const int c0 = (chunk * 32 + (lane & 31)) * NCH;
+  const int t0 = block * kColumnTokens + 64 * half;
+  // the block's rows from a wave-uniform base; a lane's offset is 32 bits
+  constexpr int kSize = SRC == kF32 ? 4 : 2;
+  const uint8_t* base = (const uint8_t*)p.src +
+                        kSize * ((bh / p.H) * p.sb + (bh % p.H) * p.sh + (page * p.T + block * kColumnTokens) * p.st);
+  uint32_t w[64];
+  if ((block + 1) * kColumnTokens <= p.T) {
+    const uint32_t off = (uint32_t)kSize * (64u * half * (uint32_t)p.st + c0);
+#pragma unroll
+    for (int j = 0; j < 64; ++j) w[j] = *(const uint32_t*)(base + kSize * j * p.st + off);
+  } else {
+    const int last = p.T - 1 - block * kColumnTokens;
+#pragma unroll
+    for (int j = 0; j < 64; ++j) {
+      w[j] = *(const uint32_t*)(base + (uint32_t)kSize * ((uint32_t)min(64 * half + j, last) * (uint32_t)p.st + c0));
+      if (j % 8 == 7) __builtin_amdgcn_sched_barrier(0);  // eight addresses at a time
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < NCH; ++k) {
+    auto x = [&](int j) -> float {
+      if (SRC == kF32) return __builtin_bit_cast(float, w[j]);
+      if (SRC == kBF16) return __builtin_bit_cast(float, k ? w[j] & 0xffff0000u : w[j] << 16);
+      return (float)__builtin_bit_cast(_Float16, (uint16_t)(w[j] >> (16 * k)));
+    };
+    const int64_t channel = bh * p.D + c0 + k;
+#pragma unroll
+    for (int s = 0; s < 64 / SG; ++s) {
+      float mn = x(s * SG), mx = mn;
+#pragma unroll
+      for (int j = 1; j < SG; ++j) {
+        mn = nmin(mn, x(s * SG + j));
+        mx = nmax(mx, x(s * SG + j));
+      }
+      if (KG == 128) {
+        mn = nmin(mn, __shfl_xor(mn, 32, 64));
+        mx = nmax(mx, __shfl_xor(mx, 32, 64));
+      }
+      const int g = (t0 + s * SG) / KG;
+      if (g >= p.G) continue;  // (both halves of a 128-token group agree)
+      // the codes convert the tokens again: kept, the conversions would take 64 more registers
+#pragma unroll
+      for (int j = 0; j < SG; ++j) asm volatile("" : "+v"(w[s * SG + j]));
+      const float sc = rows_group_scale<SRC>(mn, mx, qmax, inv_qmax);
+      const float y = __fdiv_rn(1.0f, sc);
+      if (KG < 128 || half == 0) {
+        flag_nonfinite(p.nonfinite, mn, mx);
+        dev_store_meta((char*)p.scale + page * p.scale_page_stride, channel * p.G + g, sc, p.meta_dtype);
+        dev_store_meta((char*)p.zero + page * p.zero_page_stride, channel * p.G + g, mn, p.meta_dtype);
+      }
+      constexpr int kWords = SG * BITS / 32;
+      uint32_t out[kWords];
+#pragma unroll
+      for (int d = 0; d < kWords; ++d) {
+        constexpr int per = 32 / BITS;
+        uint32_t plane[4] = {0u, 0u, 0u, 0u}, plane4[2] = {0u, 0u};
+#pragma unroll
+        for (int h = 0; h < per / 4; ++h) {
+          float xs[4], q[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) xs[i] = x(s * SG + per * d + 4 * h + i);
+          chain_quotients4<SRC>(xs, mn, sc, y, q);
+          if (BITS == 2) codes_to_planes2(q, h, plane);
+          else if (BITS == 4) codes_to_planes4(q, h, plane4);
+          else out[d] = codes_as_bytes(q);
+        }
+        if (BITS == 2) out[d] = pack2(plane);
+        if (BITS == 4) out[d] = pack4(plane4);
+      }
+      uint8_t* dst = p.low + page * p.low_page_stride + channel * p.pk + (t0 + s * SG) * BITS / 8;
+      if constexpr (kWords == 2) {
+        *(uint2*)dst = make_uint2(out[0], out[1]);
+      } else {
+#pragma unroll
+        for (int d = 0; d < kWords; d += 4)
+          ((uint4*)dst)[d / 4] = make_uint4(out[d], out[d + 1], out[d + 2], out[d + 3]);
+      }
+    }
+  }
+}
+
 // Single-pass key page kernel for the common shape: head_dim 128, at most 128
 // tokens per page, one key group per page, 16-bit source with unit channel
 // stride.  One workgroup per (batch * head, page), 256 threads:
@@ -1316,6 +1438,51 @@ __global__ void __launch_bounds__(kThreads) dequantize_rows_kernel(const uint8_t
                     dev_load_meta(zero, r * groups + g, meta), meta, out_dt);
 }
 
+// Eight elements of one group per lane: one load of 2, 4 or 8 bytes of codes,
+// one scale and zero point, one store of 16 (fp32: 32) bytes.  Bound by the
+// stores; the form above spends a 64-bit division and a store per element.
+// n8: lanes per row (shift: its log2, or -1).
+template <int BITS, int META, int OUT>
+__global__ void __launch_bounds__(kThreads) dequantize_rows_vec(const uint8_t* values, const void* scale,
+                                                                const void* zero, uint32_t items, uint32_t n8,
+                                                                int shift, uint32_t group8, uint32_t groups,
+                                                                int64_t packed_bytes, void* out, int64_t out_stride) {
+  constexpr int kItems = 2;
+  const uint32_t first = (uint32_t)blockIdx.x * (kThreads * kItems) + threadIdx.x;
+#pragma unroll
+  for (int u = 0; u < kItems; ++u) {
+    const uint32_t item = first + u * kThreads;
+    if (item >= items) return;
+    const uint32_t r = shift >= 0 ? item >> shift : item / n8, i8 = item - r * n8;
+    const uint8_t* src = values + (int64_t)r * packed_bytes + i8 * BITS;
+    uint64_t w;
+    if (BITS == 2) w = *(const uint16_t*)src;
+    else if (BITS == 4) w = *(const uint32_t*)src;
+    else w = *(const uint64_t*)src;
+    const int64_t g = (int64_t)r * groups + i8 / group8;
+    const float s = dev_load(scale, g, META), z = dev_load(zero, g, META);
+    float x[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const uint32_t code = (uint32_t)(w >> (BITS * j)) & ((1u << BITS) - 1u);
+      x[j] = src_round<META>(src_round<META>((float)code * s) + z);  // -ffp-contract=off: one rounding each
+    }
+    if (OUT == kF32) {
+      float4* o = (float4*)((float*)out + (int64_t)r * out_stride + 8 * i8);
+      o[0] = make_float4(x[0], x[1], x[2], x[3]);
+      o[1] = make_float4(x[4], x[5], x[6], x[7]);
+    } else {
+      uint16_t h[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        h[j] = OUT == kBF16 ? __builtin_bit_cast(uint16_t, (__bf16)x[j]) : __builtin_bit_cast(uint16_t, (_Float16)x[j]);
+      uint4 o;
+      __builtin_memcpy(&o, h, 16);
+      *(uint4*)((uint16_t*)out + (int64_t)r * out_stride + 8 * i8) = o;
+    }
+  }
+}
+
 __global__ void __launch_bounds__(kThreads) dequantize_mixed_kernel(const uint8_t* low, const uint8_t* high,
                                                                     const int32_t* idx, const void* scale,
                                                                     const void* zero, int meta, int64_t B,
@@ -1574,6 +1741,53 @@ extern "C" int dkv_quantize_key_pages(const dkv_key_pages_args* args, void* stre
                          ((int64_t)a.D * row_bytes) % 16 == 0 &&
                          (Kp == 0 || (((uintptr_t)a.high % 16) == 0 && (a.high_page_stride % 16) == 0 &&
                                       ((int64_t)Kp * row_bytes) % 16 == 0));
+  // uniform keys from registers; the single-pass kernel below keeps its shape
+  // (one 128-token group per page of head_dim 128)
+  const int row_piece = a.src_dtype == kF32 ? 32 : 64;  // channels of a 128-byte piece
+  const int col_store = std::min<int>(16, (int)std::min<int64_t>(a.group, 64) * (int)a.bits / 8);
+  const bool use_columns =
+      a.key_mode == DKV_KEY_UNIFORM && (a.group == 32 || a.group == 64 || a.group == 128) &&
+      (a.src_dtype == kBF16 || a.src_dtype == kF16 || a.src_dtype == kF32) && a.sd == 1 && a.D % row_piece == 0 &&
+      a.page_tokens < (1 << 28) && a.st >= 0 && a.st < (1 << 21) && ((uintptr_t)a.src % 4) == 0 &&
+      (a.src_dtype == kF32 || (a.st % 2 == 0 && a.sb % 2 == 0 && a.sh % 2 == 0)) &&
+      ((uintptr_t)a.low % col_store) == 0 && (a.low_page_stride % col_store) == 0 &&
+      !(a.src_dtype != kF32 && a.D == kFastKeyD && a.page_tokens <= kFastKeyT && a.group == kFastKeyT);
+  if (use_columns) {
+    ColumnParams c;
+    c.src = a.src;
+    c.sb = a.sb; c.sh = a.sh; c.st = a.st;
+    c.H = (int)a.H; c.D = (int)a.D; c.T = (int)a.page_tokens; c.G = (int)k.G; c.pk = (int)k.pk;
+    c.blocks = (int)((a.page_tokens + kColumnTokens - 1) / kColumnTokens);
+    c.chunks = (int)(a.D / row_piece);
+    c.bhs = a.B * a.H;
+    c.items = a.n_pages * c.bhs * c.blocks * c.chunks;
+    c.low = a.low; c.scale = a.scale; c.zero = a.zero;
+    c.low_page_stride = a.low_page_stride; c.scale_page_stride = a.scale_page_stride;
+    c.zero_page_stride = a.zero_page_stride;
+    c.meta_dtype = (int)a.meta_dtype;
+    c.nonfinite = a.nonfinite;
+    const int64_t waves = kThreads / 64, wgs = (c.items + waves - 1) / waves;
+    DKV_CHECK(wgs < (int64_t)1 << 31, DKV_ERR_UNSUPPORTED, "too many pages for one launch");
+    const dim3 grid((unsigned)wgs);
+#define DKV_COL(T, B)                                                                                           \
+  do {                                                                                                          \
+    if (a.group == 32) hipLaunchKernelGGL((quantize_key_columns<T, B, 32>), grid, dim3(kThreads), 0, s, c);     \
+    else if (a.group == 64) hipLaunchKernelGGL((quantize_key_columns<T, B, 64>), grid, dim3(kThreads), 0, s, c); \
+    else hipLaunchKernelGGL((quantize_key_columns<T, B, 128>), grid, dim3(kThreads), 0, s, c);                  \
+  } while (0)
+#define DKV_COL_BITS(T)                 \
+  do {                                  \
+    if (a.bits == 2) DKV_COL(T, 2);     \
+    else if (a.bits == 4) DKV_COL(T, 4); \
+    else DKV_COL(T, 8);                 \
+  } while (0)
+    if (a.src_dtype == kBF16) DKV_COL_BITS(kBF16);
+    else if (a.src_dtype == kF16) DKV_COL_BITS(kF16);
+    else DKV_COL_BITS(kF32);
+#undef DKV_COL_BITS
+#undef DKV_COL
+    return finish();
+  }
   // the single-pass kernel: head_dim 128, one group of up to 128 tokens per page
   const int fast_bits = a.key_mode == DKV_KEY_MIXED ? 2 : (int)a.bits;
   const bool use_fast = use_tiled && a.D == kFastKeyD && a.page_tokens <= kFastKeyT && a.group >= kFastKeyT &&
@@ -1683,6 +1897,37 @@ extern "C" int dkv_dequantize_rows(const uint8_t* values, const void* scale, con
   const int per_byte = 8 / bits;
   const int64_t packed_bytes = (groups * group + per_byte - 1) / per_byte;
   const int64_t items = rows * n;
+  // octets of one group with aligned codes and outputs
+  const int osize = out_dtype == kF32 ? 4 : 2;
+  if (meta_dtype != kF64 && out_dtype != kF64 && n % 8 == 0 && group % 8 == 0 && items / 8 < (int64_t)1 << 31 &&
+      ((uintptr_t)values % bits) == 0 && ((uintptr_t)out % 16) == 0 && (out_row_stride * osize) % 16 == 0) {
+    const uint32_t n8 = (uint32_t)(n / 8), lanes = (uint32_t)(items / 8);
+    const int shift = (n8 & (n8 - 1)) == 0 ? __builtin_ctz(n8) : -1;
+    const dim3 grid((lanes + 2 * kThreads - 1) / (2 * kThreads));
+    const uint32_t group8 = (uint32_t)std::min<int64_t>(group / 8, (int64_t)1 << 30);
+#define DKV_DQ(B, M, O)                                                                                              \
+  hipLaunchKernelGGL((dequantize_rows_vec<B, M, O>), grid, dim3(kThreads), 0, (hipStream_t)stream, values, scale, zero, \
+                     lanes, n8, shift, group8, (uint32_t)groups, packed_bytes, out, out_row_stride)
+#define DKV_DQ_OUT(B, M)                     \
+  do {                                       \
+    if (out_dtype == kBF16) DKV_DQ(B, M, kBF16); \
+    else if (out_dtype == kF16) DKV_DQ(B, M, kF16); \
+    else DKV_DQ(B, M, kF32);                 \
+  } while (0)
+#define DKV_DQ_META(B)                       \
+  do {                                       \
+    if (meta_dtype == kF16) DKV_DQ_OUT(B, kF16); \
+    else if (meta_dtype == kBF16) DKV_DQ_OUT(B, kBF16); \
+    else DKV_DQ_OUT(B, kF32);                \
+  } while (0)
+    if (bits == 2) DKV_DQ_META(2);
+    else if (bits == 4) DKV_DQ_META(4);
+    else DKV_DQ_META(8);
+#undef DKV_DQ_META
+#undef DKV_DQ_OUT
+#undef DKV_DQ
+    return dkv_check_launch("dkv_dequantize_rows");
+  }
   hipLaunchKernelGGL(dequantize_rows_kernel, dim3((unsigned)((items + kThreads - 1) / kThreads)), dim3(kThreads), 0,
                      (hipStream_t)stream, values, scale, zero, meta_dtype, rows, n, bits, group, groups, packed_bytes,
                      out, out_dtype, out_row_stride);

@@ -13,6 +13,7 @@ from typing import Optional, Tuple
 import torch
 
 from . import _lib
+from .finite import drain, nonfinite_flags
 
 _SUPPORTED_BITS = (2, 4, 8)
 
@@ -123,6 +124,15 @@ def _check_finite(data: torch.Tensor, message: str) -> None:
         raise ValueError(message)
 
 
+def _columns_apply(data: torch.Tensor, axis: int, group_size: int) -> bool:
+    """Whether ``dkv_quantize_key_pages`` reads ``data`` in place along its last but one axis (its register
+    kernel: groups of 32, 64 or 128, rows of whole 128-byte pieces); otherwise the axis is moved last by a copy."""
+    return (data.ndim >= 2 and axis == data.ndim - 2 and group_size in (32, 64, 128) and data.is_contiguous()
+            and data.dtype in (torch.bfloat16, torch.float16, torch.float32) and data.data_ptr() % 4 == 0
+            and data.shape[-1] % (128 // data.element_size()) == 0 and data.shape[-1] < (1 << 21)
+            and data.shape[-2] < (1 << 28) and data.numel() // (data.shape[-1] * data.shape[-2]) < (1 << 31))
+
+
 def quantize(
     data: torch.Tensor,
     *,
@@ -146,31 +156,54 @@ def quantize(
         raise TypeError(f"quantize expects a floating-point tensor, got {data.dtype}")
     if data.shape[-1] == 0:
         raise ValueError("quantize does not support an empty final dimension")
-    _check_finite(data, "quantize expects all values to be finite")
     original_shape = tuple(data.shape)
-    if not isinstance(axis, int) or not -data.ndim <= axis < data.ndim:
+    message = "quantize expects all values to be finite"
+    bad_axis = not isinstance(axis, int) or not -data.ndim <= axis < data.ndim
+    # the kernels report non-finite values themselves; checked ahead where another error would come first
+    # or none of their launches runs
+    ahead = (bad_axis or data.device.type != "cuda" or data.dtype not in _lib.FLOAT_DTYPES or data.numel() == 0
+             or torch.cuda.is_current_stream_capturing())
+    if ahead:
+        _check_finite(data, message)
+    if bad_axis:
         raise ValueError(f"axis must be in [-{data.ndim}, {data.ndim}), got {axis}")
     axis = axis % data.ndim
     _lib.require_device(data)
-    moved = data.movedim(axis, -1).contiguous()
-    n = moved.shape[-1]
+    n = original_shape[axis]
+    outer = original_shape[:axis] + original_shape[axis + 1:]
     groups = (n + group_size - 1) // group_size
     padded = groups * group_size
     per_byte = 8 // bits
     packed_dim = ((padded + per_byte - 1) // per_byte) * per_byte
-    meta = _metadata_dtype(moved, metadata_dtype)
-    outer = moved.shape[:-1]
+    meta = _metadata_dtype(data, metadata_dtype)
     rows = _numel(outer)
     dev = data.device
     values = torch.empty(*outer, packed_dim // per_byte, dtype=torch.uint8, device=dev)
     scale = torch.empty(*outer, groups, dtype=meta, device=dev)
     zero = torch.empty(*outer, groups, dtype=meta, device=dev)
     if rows:
-        lib = _lib.load()
-        rc = lib.dkv_quantize_rows(moved.data_ptr(), _lib.dtype_code(moved.dtype), rows, n, n, 1, bits, group_size,
-                                   values.data_ptr(), scale.data_ptr(), zero.data_ptr(), _lib.dtype_code(meta),
-                                   _lib.stream_ptr(dev))
-        _lib.check(rc, "dkv_quantize_rows")
+        flags = None if ahead else nonfinite_flags(dev)
+        flag = None if flags is None else flags.data_ptr()
+        lib, stream = _lib.load(), _lib.stream_ptr(dev)
+        if n and _columns_apply(data, axis, group_size):
+            T, D = original_shape[-2], original_shape[-1]
+            a = _lib.KeyPagesArgs(src=data.data_ptr(), src_dtype=_lib.dtype_code(data.dtype), B=1, H=rows // D, D=D,
+                                  page_tokens=T, n_pages=1, sb=0, sh=T * D, st=D, sd=1, key_mode=_lib.KEY_UNIFORM,
+                                  bits=bits, group=group_size, meta_dtype=_lib.dtype_code(meta), low=values.data_ptr(),
+                                  scale=scale.data_ptr(), zero=zero.data_ptr(), nonfinite=flag)
+            _lib.check(lib.dkv_quantize_key_pages(a, stream), "dkv_quantize_key_pages")
+        else:
+            moved = data.movedim(axis, -1).contiguous()
+            a = _lib.ValueRowsArgs(src=moved.data_ptr(), src_dtype=_lib.dtype_code(moved.dtype), blocks=1,
+                                   block_rows=rows, n=n, row_stride=n, bits=bits, group=group_size,
+                                   meta_dtype=_lib.dtype_code(meta), values=values.data_ptr(), scale=scale.data_ptr(),
+                                   zero=zero.data_ptr(), nonfinite=flag)
+            _lib.check(lib.dkv_quantize_value_rows(a, stream), "dkv_quantize_value_rows")
+        if flags is not None:
+            drain(dev)
+            if any(flags.tolist()):
+                flags.zero_()
+                raise ValueError(message)
     return QuantizedTensor(values=values, scale=scale, zero_point=zero, original_shape=original_shape,
                            original_dim=n, padded_dim=padded, packed_dim=packed_dim, group_size=group_size,
                            bits=bits, output_dtype=data.dtype, axis=axis)
