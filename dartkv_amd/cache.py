@@ -28,6 +28,7 @@ from dataclasses import dataclass, fields as dataclass_fields
 from itertools import accumulate
 from typing import TYPE_CHECKING, List, Optional, Tuple, Union
 
+import numpy as np
 import torch
 
 from . import _lib
@@ -853,10 +854,11 @@ class DartKVCache:
 
     def _pools(self) -> list:
         pools = {id(p): p for p in (self._key_pool, self._value_pool) if p is not None}
-        for seg in (*self._keys, *self._values):
-            pool = getattr(seg, "_pool", None)
-            if pool is not None:
-                pools[id(pool)] = pool
+        for track, usual in ((self._keys, self._key_pool), (self._values, self._value_pool)):
+            for seg in track:
+                pool = getattr(seg, "_pool", None)
+                if pool is not usual and pool is not None:
+                    pools[id(pool)] = pool
         return list(pools.values())
 
     def _invalidate_page_descriptors(self) -> None:
@@ -1354,20 +1356,18 @@ class DartKVCache:
         sealed = self._sealed_pairs()
         tail_is_pending = self._tail_resident() or self._tail_count_dev is not None
         keepalive: list = [dict(p.tensors) for p in self._pools()]  # storage outlives the table
-        descs = (_lib.Segment * max(1, len(sealed)))()
-        n_tokens = 0
-        for i, (kseg, vseg) in enumerate(sealed):
-            fill_segment(descs[i], kseg, vseg, keepalive)
-            n_tokens += descs[i].tokens
-        table = None
+        rows = np.zeros(len(sealed), dtype=_SEGMENT_ROW)
+        table = descs = None
+        runs: list = []
         if sealed:
-            raw = torch.frombuffer(bytearray(bytes(descs)), dtype=torch.uint8)
-            table = raw.to(device)
-        fast = _fast_run(self, descs, len(sealed))
-        rest_dense = _rest_dense(self, descs, len(sealed), fast)
-        plan = _DecodePlan(self._sealed_version, device, table, len(sealed), keepalive, tail_is_pending, n_tokens,
-                           fast, rest_dense)
-        plan.host_table = descs if sealed else None
+            descs = (_lib.Segment * len(sealed)).from_buffer(rows)
+            runs = _fill_table(descs, rows, sealed, keepalive)
+            table = torch.from_numpy(rows.view(np.uint8)).to(device)
+        fast = _fast_run(self, descs, runs)
+        rest_dense = _rest_dense(self, descs, runs, fast)
+        plan = _DecodePlan(self._sealed_version, device, table, len(sealed), keepalive, tail_is_pending,
+                           int(rows["tokens"].sum()), fast, rest_dense)
+        plan.host_table = descs
         self._decode_plan_cache = plan
         return plan
 
@@ -1385,6 +1385,8 @@ def _union_pairs(keys: list, values: list) -> list:
     v_len = [_segment_tokens(s) for s in values]
     if min(k_len + v_len) <= 0:
         raise RuntimeError("DartKVCache contains an empty logical segment")
+    if k_len == v_len:
+        return list(zip(keys, values))
     k_ends, v_ends = list(accumulate(k_len)), list(accumulate(v_len))
     if k_ends[-1] != v_ends[-1]:
         raise RuntimeError("DartKVCache key/value logical lengths diverged")
@@ -1504,6 +1506,11 @@ def _materialize(segment: Segment) -> torch.Tensor:
 
 
 def _segment_tokens(segment: Segment) -> int:
+    kind = type(segment)
+    if kind is PoolValues:
+        return segment._rows
+    if kind is PoolMixedKey:
+        return segment._tokens
     return segment.shape[-2] if isinstance(segment, torch.Tensor) else segment.original_shape[-2]
 
 
@@ -1606,6 +1613,58 @@ def fill_segment(desc, kseg: Segment, vseg: Segment, keepalive: list) -> None:
         desc.value[2], desc.value_bh[2] = _field_block(vseg, "zero_point", keepalive)
 
 
+# _lib.Segment as a numpy row: runs of pages differ by constant steps, so their descriptors are made and checked as
+# arrays (one at a time, the 127 pages of a 16,384-token prompt took 1.5 ms after every prefill and page seal)
+_SEGMENT_ROW = np.dtype([(name, np.int32 if ctypes.sizeof(kind) == 4 else np.uint64 if name in ("key", "value")
+                          else np.int64, *([(kind._length_,)] if hasattr(kind, "_length_") else []))
+                         for name, kind in _lib.Segment._fields_])
+assert _SEGMENT_ROW.itemsize == ctypes.sizeof(_lib.Segment)
+
+_KEY_SLOTS = {PoolMixedKey: ("low_values", "high_values", "channel_indices", "scale", "zero_point"),
+              PoolKeys: ("values", None, None, "scale", "zero_point")}
+
+
+def _run_length(pairs: list, i: int) -> int:
+    """How many pairs from ``i`` on are consecutive pages of one key pool over consecutive equal runs of one value
+    pool's rows (at least 1)."""
+    k, v = pairs[i]
+    kind = type(k)
+    if kind not in _KEY_SLOTS or type(v) is not PoolValues:
+        return 1
+    kpool, vpool, rows, n = k._pool, v._pool, v._rows, 1
+    at, row, tokens = k._at + 1, v._at + rows, _segment_tokens(k)
+    for k, v in pairs[i + 1:]:
+        if (type(k) is not kind or k._pool is not kpool or k._at != at or type(v) is not PoolValues
+                or v._pool is not vpool or v._at != row or v._rows != rows or _segment_tokens(k) != tokens):
+            break
+        n, at, row = n + 1, at + 1, row + rows
+    return n
+
+
+def _fill_table(descs, rows: np.ndarray, pairs: list, keepalive: list) -> list:
+    """The descriptors of ``pairs`` (``descs`` and ``rows`` are one memory): the first page of a run by
+    ``fill_segment``, the others by the pools' steps.  Returns the runs' lengths."""
+    runs, i = [], 0
+    while i < len(pairs):
+        kseg, vseg = pairs[i]
+        fill_segment(descs[i], kseg, vseg, keepalive)
+        n = _run_length(pairs, i)
+        if n > 1:
+            keepalive.extend(pairs[i + 1:i + n])
+            kref, vref = kseg._pool.ref, vseg._pool.ref
+            keys = [kref(name) if name is not None else None for name in _KEY_SLOTS[type(kseg)]]
+            ksteps = [0 if f is None or not a else f.stride(0) * f.element_size() for f, a in zip(keys, descs[i].key)]
+            values = [vref(name) for name in ("values", "scale", "zero_point")]
+            vsteps = [vseg._rows * f.stride(2) * f.element_size() for f in values]
+            run, at = rows[i:i + n], np.arange(n, dtype=np.uint64)[:, None]
+            run[1:] = run[0]
+            run["key"] += at * np.array(ksteps, dtype=np.uint64)
+            run["value"] += at * np.array(vsteps, dtype=np.uint64)
+        runs.append(n)
+        i += n
+    return runs
+
+
 def _dense_block(t: torch.Tensor, keepalive: list) -> Tuple[int, int]:
     """Dense [B,H,T,D] block: rows of D contiguous elements, token stride D."""
     B, H, T, D = t.shape
@@ -1619,7 +1678,7 @@ def _dense_block(t: torch.Tensor, keepalive: list) -> Tuple[int, int]:
     return c.data_ptr(), T * D
 
 
-def _fast_run(cache: DartKVCache, descs, count: int) -> Tuple[int, int, int, int, int, int]:
+def _fast_run(cache: DartKVCache, descs, runs: list) -> Tuple[int, int, int, int, int, int]:
     """Longest run of descriptors a page kernel handles:
     (first, count, promoted, value group, key bits, value bits).
 
@@ -1628,7 +1687,8 @@ def _fast_run(cache: DartKVCache, descs, count: int) -> Tuple[int, int, int, int
     2/4/8-bit keys along the tokens in one group per page, 2/4/8-bit values)
     to the arithmetic one.  Both need full 128-token pages, head_dim 128, fp16
     metadata, value groups that are multiples of 16 dividing 128, and every
-    block 16-byte aligned per (batch, head)."""
+    block 16-byte aligned per (batch, head).  ``runs``: lengths of the table's
+    runs, whose descriptors differ by constant steps."""
     none = (0, 0, 0, 0, 0, 0)
     if cache.shape is None or cache.dtype not in (torch.bfloat16, torch.float16):
         return none
@@ -1651,12 +1711,12 @@ def _fast_run(cache: DartKVCache, descs, count: int) -> Tuple[int, int, int, int
         key_blocks = ((0, 1), (3, 2), (4, 2))
     key_kind = _lib.KEY_MIXED if K else _lib.KEY_UNIFORM
 
-    def ok(d) -> bool:
-        if not (d.tokens == 128 and d.key_kind == key_kind and d.value_kind == _lib.VALUE_UNIFORM
-                and d.key_group == 128 and d.value_bits == vbits and d.value_group == vg):
-            return False
-        if (d.promoted != K) if K else (d.key_bits != kbits):
-            return False
+    def layout(d) -> bool:
+        return (d.tokens == 128 and d.key_kind == key_kind and d.value_kind == _lib.VALUE_UNIFORM
+                and d.key_group == 128 and d.value_bits == vbits and d.value_group == vg
+                and ((d.promoted == K) if K else (d.key_bits == kbits)))
+
+    def aligned(d) -> bool:
         for i, size in key_blocks:
             if d.key[i] % 16 or (d.key_bh[i] * size) % 16:
                 return False
@@ -1665,21 +1725,22 @@ def _fast_run(cache: DartKVCache, descs, count: int) -> Tuple[int, int, int, int
                 return False
         return True
 
-    best = (0, 0)
-    i = 0
-    while i < count:
-        if not ok(descs[i]):
-            i += 1
-            continue
-        j = i
-        while j < count and ok(descs[j]):
-            j += 1
-        if j - i > best[1]:
-            best = (i, j - i)
-        i = j
-    if best[1] == 0:
+    best, first, count, start = 0, 0, 0, 0  # best run so far, and the one that ends at `start`
+    for n in runs:
+        if not layout(descs[start]):
+            ok = [False] * n
+        elif aligned(descs[start]) and (n == 1 or aligned(descs[start + 1])):
+            ok = [True] * n  # steps of whole 16-byte units
+        else:
+            ok = [aligned(descs[i]) for i in range(start, start + n)]
+        for i, good in enumerate(ok, start):
+            count = count + 1 if good else 0
+            if count > best:
+                best, first = count, i + 1 - count
+        start += n
+    if best == 0:
         return none
-    return (best[0], best[1], K, vg, kbits, vbits)
+    return (first, best, K, vg, kbits, vbits)
 
 
 def _dense16_ok(d) -> bool:
@@ -1688,14 +1749,17 @@ def _dense16_ok(d) -> bool:
             and d.value[0] % 16 == 0 and (d.key_bh[0] * 2) % 16 == 0 and (d.value_bh[0] * 2) % 16 == 0)
 
 
-def _rest_dense(cache: DartKVCache, descs, count: int, fast: Tuple[int, ...]) -> int:
+def _rest_dense(cache: DartKVCache, descs, runs: list, fast: Tuple[int, ...]) -> int:
     """Most tokens of any sealed entry outside the fast run when all of them are
     dense 16-bit with aligned rows and head_dim is 128 (0 if there are none);
     -1 when the dense decode kernel cannot take them."""
     if cache.shape is None or cache.dtype not in (torch.bfloat16, torch.float16) or cache.shape[-1] != 128:
         return -1
-    first, n = fast[0], fast[1]
-    rest = [descs[i] for i in range(count) if not first <= i < first + n]
+    first, stop = fast[0], fast[0] + fast[1]
+    rest, start = [], 0
+    for n in runs:  # (runs of several entries are pages: one outside the fast run tells)
+        rest += [descs[i] for i in ((start,) if n == 1 else (start, start + n - 1)) if not first <= i < stop]
+        start += n
     if not all(_dense16_ok(d) for d in rest):
         return -1
     return max((d.tokens for d in rest), default=0)
