@@ -14,6 +14,7 @@
 // attention sees (attention.py:74-77).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <mutex>
 #include <math.h>
 
@@ -504,13 +505,49 @@ extern "C" int dkv_decode_attention(const dkv_decode_args* args, void* stream) {
               "rest_dense_tokens needs n_splits == non-page segments * ceil(rest_dense_tokens / %d)", kDenseChunk);
     DKV_CHECK(a.cache_dtype == dkv::kBF16 || a.cache_dtype == dkv::kF16, DKV_ERR_UNSUPPORTED,
               "rest_dense_tokens needs a bf16 or fp16 cache");
-    // up to kDenseMaxGroup heads per KV head in the dense kernels of their own; 16 only as waves of the
-    // Dart page kernel's launch
-    const int max_group = fast_count > 0 && a.fast_promoted > 0 ? kDenseFusedMaxGroup : kDenseMaxGroup;
+    // up to kDenseMaxGroup heads per KV head, or 16 where the tile kernel takes a Dart page run
+    const int max_group = fast_count > 0 && a.fast_promoted > 0 ? kMaxGroup : kDenseMaxGroup;
     DKV_CHECK(a.D == kDenseDim && p.group <= max_group, DKV_ERR_UNSUPPORTED,
               "rest_dense_tokens needs head_dim %d and at most %d query heads per KV head", kDenseDim, max_group);
   }
-  if (fast_count > 0) {
+  const int merge_threads = (int)(a.D < 64 ? 64 : (a.D > kThreads ? kThreads : ((a.D + 63) / 64) * 64));
+  bool run_done = false;
+  if (fast_count > 0 && dkv::tiles_take_run(a, p.group)) {
+    // The tile kernel takes the run: sixteen rows per KV head on Dart pages,
+    // and uniform pages of one width where the launch fills the device or has
+    // eight rows (one layer with its merge, MI355X, tile against page kernel: sixteen
+    // rows, 8 x 8 heads x 64 pages: 38 against 71 µs; 16 x 8 x 256 pages at 2 bits: 119
+    // against 172 µs; 16 x 8 x 128 pages at 4 bits, four rows: 94 against 99, eight rows:
+    // 105 against 127 µs, at 8 bits 148 against 156; one sequence x 8 heads x 8 pages:
+    // four rows at 2 bits 15.6 against 14.3 µs, eight rows at 2 bits 14.7 against 17.8,
+    // at 8 bits 19.1 against 17.9).
+    DecodeParams t = p;
+    t.skip_first = t.skip_count = 0;
+    const bool all = rest == 0 || dense_rest;  // the dense pieces ride in the same launch
+    t.n_total = (int)(all ? a.n_segments + (a.tail.tokens > 0 ? 1 : 0) : fast_count);
+    // one page per split: one dense piece per split too (there is a record for each)
+    const int splits = (int)(fast_splits >= fast_count ? t.n_total : fast_splits);
+    t.split_offset = 0;
+    if (all) t.split_stride = splits;
+    else if (splits != fast_splits) t.split_stride = splits + (int)general_splits;
+    int rc = record_event(a.fast_events[0], s);
+    if (rc) return rc;
+    const dkv::TileLayout layout{a.fast_promoted > 0 ? 2 : (int)a.fast_key_bits, 128, (int)a.fast_value_group,
+                                 (int)a.fast_promoted};
+    rc = dkv::launch_tile_run(t, (int)a.fast_first, (int)fast_count, splits, layout, s);
+    if (rc) return rc;
+    rc = record_event(a.fast_events[1], s);
+    if (rc) return rc;
+    if (all) {
+      hipLaunchKernelGGL(decode_merge, dim3((unsigned)(a.B * a.Hq)), dim3(merge_threads),
+                         (size_t)2 * splits * sizeof(float), s, t);
+      return dkv_check_launch("dkv_decode_attention(merge)");
+    }
+    p.split_offset = splits;
+    p.split_stride = t.split_stride;
+    run_done = true;
+  }
+  if (fast_count > 0 && !run_done) {
     // With a dense rest, the page kernel's launch also runs the dense chunks
     // (extra waves beside the page waves, so their latency hides behind the
     // pages), and one merge launch follows.  Merging in the page launch itself
@@ -589,8 +626,7 @@ extern "C" int dkv_decode_attention(const dkv_decode_args* args, void* stream) {
     rc = dkv_check_launch("dkv_decode_attention(split)");
     if (rc) return rc;
   }
-  const int merge_threads = (int)(a.D < 64 ? 64 : (a.D > kThreads ? kThreads : ((a.D + 63) / 64) * 64));
   hipLaunchKernelGGL(decode_merge, dim3((unsigned)(a.B * a.Hq)), dim3(merge_threads),
-                     (size_t)2 * stride * sizeof(float), s, p);
+                     (size_t)2 * p.split_stride * sizeof(float), s, p);
   return dkv_check_launch("dkv_decode_attention(merge)");
 }

@@ -3,11 +3,11 @@
 // Scope: head_dim 128, 128-token pages, keys with Dart promotion (2-bit codes
 // for every channel plus the upper 2 bits of NP promoted channels, one key
 // group per page), 2-bit values with groups of vg (16 | vg, vg | 128)
-// channels, fp16 metadata, bf16 or fp16 cache, 1, 2, 4, 8 or 16 query rows per
-// KV head (8 or 16 rows: two or four row groups of 4, each with its own Q K
-// MFMAs on the same dequantized B operands; the multi-token path maps two or
-// four tokens of a 4-head group here).  Everything else goes through the general kernel
-// (decode.hip).
+// channels, fp16 metadata, bf16 or fp16 cache, 1, 2, 4 or 8 query rows per KV
+// head (8 rows: two row groups of 4, each with its own Q K MFMAs on the same
+// dequantized B operands; the multi-token path maps two tokens of a 4-head
+// group here).  Sixteen rows and everything else go to the tile kernel
+// (decode_tiles.hip) or the general one (decode.hip).
 //
 // One wave owns one split: a contiguous range of pages of one (batch, kv
 // head).  (Launches that leave most of the GPU idle give a split four waves,
@@ -63,8 +63,8 @@ struct LdsMap {
   int kl, vc, kh, ki, ks, kz, vs, vz, klut, klut16, vlut, pidx, q16, qp, pt, zero, bytes;
 };
 
-// rg: row groups of 4 query rows (1, or 2 / 4 for 8 / 16 rows per KV head).
-// With several, the promoted channels' query rows live in the softmax-weight
+// rg: row groups of 4 query rows (1, or 2 for 8 rows per KV head).  With two,
+// the promoted channels' query rows live in the softmax-weight
 // region (which is free from the weights' last read in P V until the softmax
 // writes them) and the query takes 4 rg rows.
 __host__ __device__ inline LdsMap lds_map(int np, int gv, int rg) {
@@ -261,39 +261,36 @@ __host__ __device__ constexpr int xchg_bytes(int rg) { return kSplitWaves * rg *
 // Outstanding page copies stay in flight.
 __device__ __forceinline__ void block_lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// Row groups of 4 query rows for GQ rows per KV head, and waves per workgroup:
-// one-wave workgroups for 16 rows, whose LDS region (about 24 KB) leaves room
-// for six waves per CU but not for two four-wave workgroups.
+// Row groups of 4 query rows for GQ rows per KV head.
 __host__ __device__ constexpr int fast_row_groups(int gq) { return gq > 4 ? gq / 4 : 1; }
-__host__ __device__ constexpr int fast_waves_per_block(int gq) { return gq > 8 ? 1 : kWaves; }
 
-// GQ: query rows per KV head (1, 2, 4, 8 or 16); NP: promoted channels (16,
+// GQ: query rows per KV head (1, 2, 4 or 8); NP: promoted channels (16,
 // 32, 48 or 64); BF16: cache dtype bf16 (else fp16).  All compile-time, so
 // every block loop unrolls with immediate offsets and the table builds carry
 // no dtype tests.  Rows come in RG groups of GH: each group has its own Q K
-// MFMAs (the slot layout holds 4 rows), with 8 or 16 rows the groups' A
+// MFMAs (the slot layout holds 4 rows), with 8 rows the groups' A
 // operands are formed per MFMA from one 2-byte LDS read each (several register
 // sets would not fit; four reads per operand, three of zeros, stalled on LDS
 // issue), as are the promoted pass's for any row count, and P V takes all rows
 // in one MFMA (rows 4g + i: lane group kq = g holds group g's outputs).
 //
-// W: waves per split, 1 or kSplitWaves (channel-split pages, GQ <= 8).
+// W: waves per split, 1 or kSplitWaves (channel-split pages).
 template <int GQ, int NP, bool BF16, int W>
-__global__ void __launch_bounds__(64 * fast_waves_per_block(GQ), 2)
+__global__ void __launch_bounds__(64 * kWaves, 2)
     decode_pages_fast(FastParams p) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = lane & 15, kq = lane >> 4;
-  static_assert(W == 1 || (W == kSplitWaves && fast_waves_per_block(GQ) == W), "one split per workgroup");
+  static_assert(W == 1 || (W == kSplitWaves && kWaves == W), "one split per workgroup");
   const int mw = W > 1 ? wave : 0;  // this wave's quarter of a channel-split page
   const int total_workers = p.B * p.Hkv * p.splits;
   // page workers first (W waves each), then the dense-rest workers (one wave each)
-  const int worker = W > 1 ? (int)blockIdx.x : (int)blockIdx.x * fast_waves_per_block(GQ) + wave;
+  const int worker = W > 1 ? (int)blockIdx.x : (int)blockIdx.x * kWaves + wave;
   constexpr int np = NP;
   constexpr bool bf16 = BF16;
   constexpr int RG = fast_row_groups(GQ), GH = GQ > 4 ? 4 : GQ;
-  static_assert(GQ == 1 || GQ == 2 || GQ == 4 || GQ == 8 || GQ == 16, "1, 2, 4, 8 or 16 query rows per KV head");
+  static_assert(GQ == 1 || GQ == 2 || GQ == 4 || GQ == 8, "1, 2, 4 or 8 query rows per KV head");
   const int gv = p.gv;
   const LdsMap M = lds_map(np, gv, RG);
   uint8_t* lds = smem + wave * M.bytes;
@@ -729,7 +726,7 @@ namespace dkv {
 int fast_decode_max_loads(int np, int gv) { return n_small_loads(np, gv) + n_key_loads(np); }
 
 size_t fast_decode_lds_bytes(int np, int gv, int gq) {
-  return (size_t)fast_waves_per_block(gq) * lds_map(np, gv, fast_row_groups(gq)).bytes;
+  return (size_t)kWaves * lds_map(np, gv, fast_row_groups(gq)).bytes;
 }
 
 // Compute units of the current device (read once per device; threads that
@@ -771,7 +768,6 @@ int launch_fast_decode(const dkv_decode_args& a, int first, int count, int np, i
   p.ws = (float*)a.workspace;
   set_fused(p, fused);
   const int64_t page_workers = (int64_t)p.B * p.Hkv * splits;
-  const int wpb = fast_waves_per_block(p.GQ);
   // Channel-split pages when every workgroup of that launch (one split each,
   // then the dense-rest waves four to a workgroup) has a compute unit to
   // itself: the launch leaves most of the GPU idle, and a page's latency
@@ -780,24 +776,22 @@ int launch_fast_decode(const dkv_decode_args& a, int first, int count, int np, i
   const int64_t split_blocks = page_workers + (p.dense_workers + kSplitWaves - 1) / kSplitWaves;
   const char* force = getenv("DKV_SPLIT_PAGES");
   bool split_pages = false;
-  if (wpb == kSplitWaves) {
-    if (force != nullptr && force[0] != '\0') {
-      split_pages = force[0] != '0';
-    } else {
-      const int cus = device_cus();
-      split_pages = cus > 0 && split_blocks <= cus;
-    }
+  if (force != nullptr && force[0] != '\0') {
+    split_pages = force[0] != '0';
+  } else {
+    const int cus = device_cus();
+    split_pages = cus > 0 && split_blocks <= cus;
   }
   const unsigned blocks =
-      (unsigned)(split_pages ? split_blocks : (page_workers + p.dense_workers + wpb - 1) / wpb);
+      (unsigned)(split_pages ? split_blocks : (page_workers + p.dense_workers + kWaves - 1) / kWaves);
   const size_t lds = fast_decode_lds_bytes(np, p.gv, p.GQ) +
                      (split_pages ? (size_t)2 * xchg_bytes(fast_row_groups(p.GQ)) : 0);
-  const dim3 grid(blocks), block(64 * wpb);
+  const dim3 grid(blocks), block(64 * kWaves);
 #define DKV_FAST_LAUNCH(G, N)                                                                             \
   do {                                                                                                    \
-    if (split_pages && G <= 8) {                                                                          \
-      if (p.bf16) hipLaunchKernelGGL((decode_pages_fast<G, N, true, G <= 8 ? kSplitWaves : 1>), grid, block, lds, stream, p); \
-      else hipLaunchKernelGGL((decode_pages_fast<G, N, false, G <= 8 ? kSplitWaves : 1>), grid, block, lds, stream, p);      \
+    if (split_pages) {                                                                                    \
+      if (p.bf16) hipLaunchKernelGGL((decode_pages_fast<G, N, true, kSplitWaves>), grid, block, lds, stream, p); \
+      else hipLaunchKernelGGL((decode_pages_fast<G, N, false, kSplitWaves>), grid, block, lds, stream, p); \
     } else {                                                                                              \
       if (p.bf16) hipLaunchKernelGGL((decode_pages_fast<G, N, true, 1>), grid, block, lds, stream, p);    \
       else hipLaunchKernelGGL((decode_pages_fast<G, N, false, 1>), grid, block, lds, stream, p);          \
@@ -819,9 +813,8 @@ int launch_fast_decode(const dkv_decode_args& a, int first, int count, int np, i
     case 2: DKV_FAST_NP(2); break;
     case 4: DKV_FAST_NP(4); break;
     case 8: DKV_FAST_NP(8); break;
-    case 16: DKV_FAST_NP(16); break;
     default:
-      set_error("fast decode supports 1, 2, 4, 8 or 16 query rows per KV head");
+      set_error("fast decode supports 1, 2, 4 or 8 query rows per KV head");
       return DKV_ERR_UNSUPPORTED;
   }
 #undef DKV_FAST_NP

@@ -43,8 +43,8 @@
 // Arithmetic.  K and V hold the reference's dequantized values exactly (its
 // rounding chain), the query is exact in the operand type, and the softmax
 // weights stay fp32: a weight is the exact sum of three 16-bit parts (8 + 8 +
-// 8 bits for bf16; 11 + 11 + 2 for fp16), the parts of 4 heads fill the 16
-// rows of one MFMA (those of 8 heads two MFMAs, of 16 heads three), and their
+// 8 bits for bf16; 11 + 11 + 2 for fp16), the parts of 4 heads take 12 of the
+// 16 rows of one MFMA (those of 8 heads two MFMAs, of 16 heads three), and their
 // products meet in the fp32 accumulators when the split ends.
 #include <hip/hip_runtime.h>
 #include <math.h>
@@ -76,8 +76,9 @@ struct TileParams {
   int packed_first, n_packed, splits;
   // what every packed segment shares
   int key_group, value_group, promoted;
-  // LDS of one wave (bytes): key tables, value tables, weights, then what Dart
-  // pages need (scale/zero pairs by channel, the query rows)
+  // LDS of one wave (bytes): the key tables, and after Q K the value tables in
+  // their place; the weights, before them the scale/zero pairs of a Dart page's
+  // channels; the query rows
   int kt, vt, pw, sz, q, wave_bytes;
 };
 
@@ -115,6 +116,10 @@ __device__ __forceinline__ Packed packed_segment(const_segment& s, int64_t bh) {
   return t;
 }
 
+// A product below 2^32 of factors below 2^24, in one full-rate instruction (a
+// 32-bit product takes four).
+__device__ __forceinline__ uint32_t mul24(uint32_t a, uint32_t b) { return __umul24(a, b); }
+
 __device__ __forceinline__ int groups_of(int n, int group) { return (n + group - 1) / group; }
 
 // fp16 pair -> the pair in the operand type.
@@ -149,45 +154,69 @@ __device__ __forceinline__ uint2 table4(uint32_t sz) {
 }
 
 // ---- codes: NP consecutive positions (tokens of a key channel, channels of a
-// value row) of K index k are one load of NP * BITS / 8 bytes ----
-
+// value row) of one K index are NP * BITS / 8 bytes ----
+//
+// Where that is one or two bytes, neighbouring lanes share their loads: of the
+// pair of K indices (k0, k1) the even lane loads k0's and the odd lane k1's
+// codes of both lanes' positions, and they exchange halves when the codes are
+// used.  (A load each, packed into one register, waits for its data where it is
+// issued: the packing cannot leave the load's block.)
 template <int BITS, int NP>
 struct Codes {
-  static constexpr int kBytes = NP * BITS / 8;                     // 1, 2, 4 or 8
-  static constexpr int kPairRegs = kBytes <= 2 ? 1 : kBytes / 2;   // registers of two K indices
+  static constexpr int kBytes = NP * BITS / 8;                    // 1, 2, 4 or 8
+  static constexpr bool kShared = kBytes <= 2;
+  static constexpr int kPairRegs = kShared ? 1 : kBytes / 2;      // registers of two K indices
+  static constexpr int kSpan = kShared ? 2 * NP : NP;             // positions of one load
 };
 
-// Codes of K indices 0 .. NK - 1 of the lane into regs, two per pair: index k's
-// are at base(k) (wave-uniform) + off(k) bytes.
+// Codes of K indices 0 .. NK - 1 of the lane into regs: index k's are at
+// base(k) (wave-uniform) + off(k) bytes; a shared load asks for the pair's
+// first index, and off adds the odd lane's step.
 template <int BITS, int NP, int NK, int N, class Base, class Off>
 __device__ __forceinline__ void load_codes(uint32_t (&regs)[N], Base base, Off off) {
   typedef Codes<BITS, NP> C;
   static_assert(N == NK / 2 * C::kPairRegs, "one tile's codes");
 #pragma unroll
   for (int p = 0; p < NK / 2; ++p) {
-    const uint8_t *a = base(2 * p), *b = base(2 * p + 1);
-    const uint32_t oa = off(2 * p), ob = off(2 * p + 1);
+    const uint8_t* a = base(2 * p);
+    const uint32_t oa = off(2 * p);
     if constexpr (C::kBytes == 1) {
-      regs[p] = (uint32_t)gload<uint8_t>(a, oa) | ((uint32_t)gload<uint8_t>(b, ob) << 16);
+      regs[p] = gload<uint16_t>(a, oa);
     } else if constexpr (C::kBytes == 2) {
-      regs[p] = (uint32_t)gload<uint16_t>(a, oa) | ((uint32_t)gload<uint16_t>(b, ob) << 16);
+      regs[p] = gload<uint32_t>(a, oa);
     } else if constexpr (C::kBytes == 4) {
       regs[2 * p] = gload<uint32_t>(a, oa);
-      regs[2 * p + 1] = gload<uint32_t>(b, ob);
+      regs[2 * p + 1] = gload<uint32_t>(base(2 * p + 1), off(2 * p + 1));
     } else {
-      const u32x2 x = gload<u32x2>(a, oa), y = gload<u32x2>(b, ob);
+      const u32x2 x = gload<u32x2>(a, oa), y = gload<u32x2>(base(2 * p + 1), off(2 * p + 1));
       regs[4 * p] = x.x; regs[4 * p + 1] = x.y;
       regs[4 * p + 2] = y.x; regs[4 * p + 3] = y.y;
     }
   }
 }
 
-// Operand dwords of a pair of K indices at every position j, from 2-bit codes
-// in byte planes: y's bytes are (k0, k1, k0, k1) at positions j and j + NP / 2.
+// The other lane's register of a lane pair.
+__device__ __forceinline__ uint32_t swap_pair(uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0xb1, 0xf, 0xf, true);  // quad_perm 1, 0, 3, 2
+}
+
+// Selector of unshare() for this lane: its own positions of (k0, k1) as bytes
+// (k0, k1, k0, k1), or (k0, k1, 0, 0) where a lane has one byte of each.
+template <int BYTES>
+__device__ __forceinline__ uint32_t unshare_sel(int lane) {
+  if (BYTES == 2) return lane & 1 ? 0x03070206u : 0x05010400u;
+  return lane & 1 ? 0x0c0c0105u : 0x0c0c0400u;
+}
+__device__ __forceinline__ uint32_t unshare(uint32_t x, uint32_t sel) { return perm(swap_pair(x), x, sel); }
+
+// Bytes (k0, k1, k0, k1) at positions j and j + NP / 2 of unshared 2-bit codes.
 template <int NP>
-__device__ __forceinline__ void lookup_pair(uint32_t codes, uint32_t lo0, uint32_t hi0, uint32_t lo1, uint32_t hi1,
+__device__ __forceinline__ uint32_t two_bit_bytes(uint32_t y) { return NP == 8 ? y : perm(y >> 4, y, 0x05040100u); }
+
+// Operand dwords of a pair of K indices at every position j, from 2-bit codes.
+template <int NP>
+__device__ __forceinline__ void lookup_pair(uint32_t y, uint32_t lo0, uint32_t hi0, uint32_t lo1, uint32_t hi1,
                                             uint32_t m3, uint32_t sel2, uint32_t (&op)[NP]) {
-  const uint32_t y = NP == 8 ? perm(0u, codes, 0x03010200u) : perm(codes >> 4, codes, 0x06040200u);
 #pragma unroll
   for (int j = 0; j < NP / 2; ++j) {
     const uint32_t e = ((y >> (2 * j)) & m3) | sel2;
@@ -197,6 +226,9 @@ __device__ __forceinline__ void lookup_pair(uint32_t codes, uint32_t lo0, uint32
   }
 }
 
+// (m & a) | (~m & b), one v_bfi_b32
+__device__ __forceinline__ uint32_t bit_select(uint32_t m, uint32_t a, uint32_t b) { return (m & a) | (~m & b); }
+
 // Two code bytes (values below 16) of word half W as an fp16 pair.
 template <bool HI>
 __device__ __forceinline__ half2v codes16(uint32_t e) {
@@ -204,9 +236,10 @@ __device__ __forceinline__ half2v codes16(uint32_t e) {
 }
 
 // The same from 4- or 8-bit codes by the arithmetic chain; s, z hold the two
-// indices' scales and zero points.
+// indices' scales and zero points, sel is the unshare selector.
 template <bool BF, int BITS, int NP>
-__device__ __forceinline__ void chain_pair(const uint32_t* codes, uint32_t s, uint32_t z, uint32_t (&op)[NP]) {
+__device__ __forceinline__ void chain_pair(const uint32_t* codes, uint32_t s, uint32_t z, uint32_t sel,
+                                           uint32_t (&op)[NP]) {
   const half2v sv = __builtin_bit_cast(half2v, s), zv = __builtin_bit_cast(half2v, z);
   auto value = [&](half2v c) {
     const half2v prod = c * sv;  // -ffp-contract=off: one rounding each
@@ -215,7 +248,7 @@ __device__ __forceinline__ void chain_pair(const uint32_t* codes, uint32_t s, ui
   if constexpr (BITS == 4) {
 #pragma unroll
     for (int q = 0; q < NP / 4; ++q) {  // four positions: bytes (k0, k1, k0, k1), two positions per byte
-      const uint32_t y = NP == 8 ? perm(codes[1], codes[0], q ? 0x07030602u : 0x05010400u) : perm(0u, codes[0], 0x03010200u);
+      const uint32_t y = NP == 8 ? perm(codes[1], codes[0], q ? 0x07030602u : 0x05010400u) : unshare(codes[0], sel);
       const uint32_t even = y & 0x0f0f0f0fu, odd = (y >> 4) & 0x0f0f0f0fu;
       op[4 * q] = value(codes16<false>(even));
       op[4 * q + 1] = value(codes16<false>(odd));
@@ -238,11 +271,6 @@ __device__ __forceinline__ void chain_pair(const uint32_t* codes, uint32_t s, ui
   }
 }
 
-// Scale (low half) and zero point (high half) of item lane_at + at.
-__device__ __forceinline__ uint32_t load_sz(const uint16_t* s, const uint16_t* z, uint32_t lane_at, int at) {
-  return (uint32_t)gload<uint16_t>(s + at, 2 * lane_at) | ((uint32_t)gload<uint16_t>(z + at, 2 * lane_at) << 16);
-}
-
 // Item `i` of a table region: a byte-plane table (2-bit codes) or its place in
 // the pair (s0, s1), (z0, z1) of the arithmetic chain.
 template <bool BF>
@@ -256,11 +284,41 @@ __device__ __forceinline__ void put_table(uint8_t* region, int i, uint32_t sz, b
   }
 }
 
+// The leading 16-bit parts of two values (rounded toward zero) as operands,
+// and what is left of them, exactly: three parts hold an fp32 value (8 + 8 + 8
+// bits in bf16, 11 + 11 + 2 in fp16 within its range).
+template <bool BF>
+__device__ __forceinline__ uint32_t take_part(float x0, float x1, float& r0, float& r1) {
+  if constexpr (BF) {
+    const uint32_t b0 = __builtin_bit_cast(uint32_t, x0), b1 = __builtin_bit_cast(uint32_t, x1);
+    r0 = x0 - __builtin_bit_cast(float, b0 & 0xffff0000u);
+    r1 = x1 - __builtin_bit_cast(float, b1 & 0xffff0000u);
+    return perm(b1, b0, 0x07060302u);
+  } else {
+    const auto h = __builtin_amdgcn_cvt_pkrtz(x0, x1);
+    r0 = x0 - (float)h[0];
+    r1 = x1 - (float)h[1];
+    return __builtin_bit_cast(uint32_t, h);
+  }
+}
+
+// A pair of weight parts, none of them zero: an infinite value times a zero
+// part would be NaN where the weight itself is not zero (a zero weight keeps its
+// zero first part).  The smallest step, 2^-126 (bf16) or 2^-24 of weights
+// scaled by 2^7 (fp16), is below what the sums resolve.
+template <bool BF>
+__device__ __forceinline__ uint32_t at_least_tiny(uint32_t x) {
+  typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+  const uint16_t tiny = BF ? 0x0080 : 0x0001;
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, x), u16x2{tiny, tiny}));
+}
+
 // The softmax state and accumulators of a wave, and the steps both kinds of
 // tile share.  GP: query rows per KV head rounded up to 4, 8 or 16.  S[j] row 4
 // kq + i = head (4 kq + i) % GP, column n = token NJ n + j; O[j] row 4 kq + i =
 // weight part and head of that row (head % GP), column n = channel NC n + j.
-template <int D, bool BF, int GP, int TILE>
+// PARTS: the query comes in three parts.
+template <int D, bool BF, int GP, int TILE, bool PARTS>
 struct TileState {
   static constexpr int NJ = TILE / 16;          // tokens of a lane
   static constexpr int NC = D / 16;             // channels of a lane
@@ -276,9 +334,24 @@ struct TileState {
   float scale;
   int n, kq;
 
+  const uint8_t* q;  // query rows in LDS: part p of head h at row p GP + h (Dart pages, or more than one part)
+
+  // The lane's A operand of query part `part`, channel block kb.
+  __device__ __forceinline__ u32x4 q_part(int part, int kb) const {
+    return *(const u32x4*)((const uint16_t*)q + (part * GP + n % GP) * D + 32 * kb + 8 * kq);
+  }
+
   __device__ __forceinline__ void q_products(int kb, const uint32_t (&op)[4][NJ], float4v (&S)[NJ]) const {
 #pragma unroll
     for (int j = 0; j < NJ; ++j) S[j] = mfma<BF>(qa[kb], u32x4{op[0][j], op[1][j], op[2][j], op[3][j]}, S[j]);
+    if constexpr (PARTS) {
+#pragma unroll
+      for (int part = 1; part < 3; ++part) {
+        const u32x4 a = q_part(part, kb);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) S[j] = mfma<BF>(a, u32x4{op[0][j], op[1][j], op[2][j], op[3][j]}, S[j]);
+      }
+    }
   }
 
   // Row 16 pass + r of the weights = part (16 pass + r) / GP of head r % GP.
@@ -335,7 +408,8 @@ struct TileState {
         for (int j = 0; j < NC; ++j) O[j][i] *= alpha;
       }
     }
-    // weights (fp16 operands: times 2^7, undone in the record) and their parts
+    // weights (fp16 operands: times 2^7, undone in the record) and their parts;
+    // with 8 heads the last part takes two rows, half of it each
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int head = GP == 4 ? i : GP == 8 ? 4 * (kq & 1) + i : 4 * kq + i;
@@ -351,27 +425,23 @@ struct TileState {
         uint32_t part[U > 1 ? U / 2 : 1];
 #pragma unroll
         for (int u = 0; u < U; u += 2) {
-          const float w0 = w[u], w1 = U > 1 ? w[(u + 1) % U] : 0.f;
+          float w0 = w[u], w1 = U > 1 ? w[(u + 1) % U] : 0.f;
+          if (GP == 8 && k == 2) w0 *= 0.5f, w1 *= 0.5f;
           float r0, r1;
-          if constexpr (BF) {
-            const uint32_t b0 = __builtin_bit_cast(uint32_t, w0), b1 = __builtin_bit_cast(uint32_t, w1);
-            part[u / 2] = perm(b1, b0, 0x07060302u);
-            r0 = w0 - __builtin_bit_cast(float, b0 & 0xffff0000u);
-            r1 = w1 - __builtin_bit_cast(float, b1 & 0xffff0000u);
-          } else {
-            const auto h = __builtin_amdgcn_cvt_pkrtz(w0, w1);
-            part[u / 2] = __builtin_bit_cast(uint32_t, h);
-            r0 = w0 - (float)h[0];
-            r1 = w1 - (float)h[1];
-          }
+          part[u / 2] = take_part<BF>(w0, w1, r0, r1);
           w[u] = r0;
           if (U > 1) w[(u + 1) % U] = r1;
+          if (k > 0) part[u / 2] = at_least_tiny<BF>(part[u / 2]);
         }
-        uint8_t* dst = pw + (k * GP + head) * kPRow + 2 * (NJ * n + start);
-        if constexpr (U == 1) *(uint16_t*)dst = (uint16_t)part[0];
-        else if constexpr (U == 2) *(uint32_t*)dst = part[0];
-        else if constexpr (U == 4) *(uint2*)dst = make_uint2(part[0], part[1]);
-        else *(uint4*)dst = make_uint4(part[0], part[1], part[2], part[3]);
+        auto put = [&](int row) {
+          uint8_t* dst = pw + row * kPRow + 2 * (NJ * n + start);
+          if constexpr (U == 1) *(uint16_t*)dst = (uint16_t)part[0];
+          else if constexpr (U == 2) *(uint32_t*)dst = part[0];
+          else if constexpr (U == 4) *(uint2*)dst = make_uint2(part[0], part[1]);
+          else *(uint4*)dst = make_uint4(part[0], part[1], part[2], part[3]);
+        };
+        put(k * GP + head);
+        if (GP == 8 && k == 2) put(3 * GP + head);
       }
     }
   }
@@ -384,10 +454,17 @@ struct TileState {
       S[j] = float4v{0.f, 0.f, 0.f, 0.f};
       const uint32_t off = 2 * ((t0 + min(NJ * n + j, nt - 1)) * D + 8 * kq);
 #pragma unroll
-      for (int kb = 0; kb < KB; ++kb) S[j] = mfma<BF>(qa[kb], gload<u32x4>(k, off + 64 * kb), S[j]);
+      for (int kb = 0; kb < KB; ++kb) {
+        const u32x4 row = gload<u32x4>(k, off + 64 * kb);
+        S[j] = mfma<BF>(qa[kb], row, S[j]);
+        if constexpr (PARTS) {
+          S[j] = mfma<BF>(q_part(1, kb), row, S[j]);
+          S[j] = mfma<BF>(q_part(2, kb), row, S[j]);
+        }
+      }
     }
     softmax(S, nt);
-    lds_sync();
+    lds_order();
 #pragma unroll 1
     for (int kb = 0; kb < VB; ++kb) {
       if (32 * kb >= nt) break;  // the weights of later tokens are zero
@@ -411,76 +488,22 @@ struct TileState {
         }
       }
     }
-    lds_sync();
+    lds_order();
   }
 };
 
-// Rest entries s0 .. s1 - 1 (in this kernel's numbering) of one (batch, kv
-// head) element by element in fp32, by one wave: lane = channels lane, lane +
-// 64.  Only for splits with non-finite sums.
-template <int D>
-__device__ __forceinline__ void scalar_split(const TileParams& p, int bhi, int split, int s0, int s1, int lane) {
-  const DecodeParams& d = p.d;
-  const dkv_decode_args& a = d.a;
-  const int64_t b = bhi / (int)a.Hkv, kvh = bhi % (int)a.Hkv;
-  const int cache_dt = (int)a.cache_dtype, meta = (int)a.meta_dtype;
-  constexpr int R = D / 64;
-#pragma unroll 1
-  for (int h = 0; h < d.group; ++h) {
-    const int64_t hq = kvh * d.group + h;
-    float q[R], acc[R], m = -INFINITY, l = 0.f;
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      q[r] = dev_load(a.query, b * a.q_sb + hq * a.q_sh + lane + 64 * r, (int)a.q_dtype);
-      acc[r] = 0.f;
-    }
-#pragma unroll 1
-    for (int i = s0; i < s1; ++i) {
-      const int j = i - p.n_packed;
-      const dkv_segment seg = general_segment(d, i < p.n_packed ? p.packed_first + i : j < p.packed_first ? j : j + p.n_packed);
-      int slot[R];
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        slot[r] = -1;
-        if (seg.key_kind != DKV_KEY_MIXED) continue;
-        for (int k = 0; k < seg.promoted; ++k)
-          if (((const int32_t*)seg.key[2])[bhi * seg.key_bh[2] + k] == lane + 64 * r) slot[r] = k;
-      }
-#pragma unroll 1
-      for (int t = 0; t < seg.tokens; ++t) {
-        float x = 0.f;
-#pragma unroll
-        for (int r = 0; r < R; ++r)
-          x = fmaf(q[r], key_value(seg, bhi, lane + 64 * r, t, D, slot[r], cache_dt, meta), x);
-        x = wave_sum(x) * (float)a.scale;
-        const float m_new = fmaxf(m, x), old = expf(m - m_new), w = expf(x - m_new);
-        l = l * old + w;
-        m = m_new;
-#pragma unroll
-        for (int r = 0; r < R; ++r)
-          acc[r] = acc[r] * old + w * value_value(seg, bhi, t, lane + 64 * r, D, cache_dt, meta);
-      }
-    }
-    float* rec = (float*)a.workspace + ((b * a.Hq + hq) * d.split_stride + d.split_offset + split) * (D + 2);
-    if (lane == 0) {
-      rec[0] = m;
-      rec[1] = l;
-    }
-#pragma unroll
-    for (int r = 0; r < R; ++r) rec[2 + lane + 64 * r] = acc[r];
-  }
-}
-
-// KBITS: key code width; MIXED: Dart pages (KBITS 2); VBITS: value code width.
-template <int D, bool BF, int GP, int KBITS, bool MIXED, int VBITS>
+// KBITS: key code width; MIXED: Dart pages (KBITS 2); VBITS: value code width;
+// PARTS: the query is of another type than the cache.
+template <int D, bool BF, int GP, int KBITS, bool MIXED, int VBITS, bool PARTS>
 __global__ void __launch_bounds__(64 * kTileWaves, 2) decode_tiles(TileParams p) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   constexpr int TILE = KBITS == 8 || VBITS == 8 ? 64 : 128;
-  typedef TileState<D, BF, GP, TILE> St;
+  typedef TileState<D, BF, GP, TILE, PARTS> St;
   constexpr int NJ = St::NJ, NC = St::NC, KB = St::KB, VB = St::VB, PASSES = St::PASSES;
   constexpr int KK = D / 4, VK = TILE / 4;  // K indices of a lane
-  constexpr int KIT = kMaxGroups * D / 64, VIT = kMaxGroups * TILE / 64;  // table items of a lane
-  constexpr int KSTEP = D / 64, VSTEP = TILE / 64;                       // items per group
+  constexpr int KSTEP = D / 64, VSTEP = TILE / 64;       // table items of a lane per group
+  constexpr int KIT = 2 * KSTEP, VIT = 2 * VSTEP;        // ... that wait in registers: two groups' (the others
+                                                         // are loaded when their tables are made)
   constexpr int kTabK = D * 8 + 16, kTabV = TILE * 8 + 16;
   typedef Codes<KBITS, NJ> KC;
   typedef Codes<VBITS, NC> VC;
@@ -499,33 +522,66 @@ __global__ void __launch_bounds__(64 * kTileWaves, 2) decode_tiles(TileParams p)
   const int s0 = uni((int)(((int64_t)split * d.n_total) / p.splits));
   const int s1 = uni((int)(((int64_t)(split + 1) * d.n_total) / p.splits));
   const uint32_t m3 = in_sgpr(0x03030303u), sel2 = in_vgpr(0x04000400u);
+  const uint32_t ksel = unshare_sel<KC::kBytes>(lane), vsel = unshare_sel<VC::kBytes>(lane);
+  const int odd = lane & 1;
   const int kgroup = p.key_group, vgroup = p.value_group, promoted = p.promoted;
   const int Gv = groups_of(D, vgroup), vrow = Gv * vgroup * VBITS / 8;
 
   // ---- the query: A operands of row n (head n % GP, zero past G), and its
-  // rows in LDS for the promoted channels ----
+  // rows in LDS for the promoted channels and for further parts ----
   St st;
   st.n = n;
   st.kq = kq;
   st.pw = lds + p.pw;
+  st.q = lds + p.q;
   st.scale = (float)a.scale;
   {
     const int head = n % GP;
-    const uint16_t* q = (const uint16_t*)a.query + (int64_t)b * a.q_sb + (int64_t)(kvh * G + (head < G ? head : 0)) * a.q_sh;
+    const int64_t at = (int64_t)b * a.q_sb + (int64_t)(kvh * G + (head < G ? head : 0)) * a.q_sh;
+    if constexpr (!PARTS) {
+      const uint16_t* q = (const uint16_t*)a.query + at;
 #pragma unroll
-    for (int kb = 0; kb < KB; ++kb) {
+      for (int kb = 0; kb < KB; ++kb) {
 #pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        const int c = 32 * kb + 8 * kq + 2 * w;
-        const uint32_t v = (uint32_t)gload<uint16_t>(q, 2 * c) | ((uint32_t)gload<uint16_t>(q, 2 * c + 2) << 16);
-        st.qa[kb][w] = head < G ? v : 0u;
+        for (int w = 0; w < 4; ++w) {
+          const int c = 32 * kb + 8 * kq + 2 * w;
+          const uint32_t v = (uint32_t)gload<uint16_t>(q, 2 * c) | ((uint32_t)gload<uint16_t>(q, 2 * c + 2) << 16);
+          st.qa[kb][w] = head < G ? v : 0u;
+        }
+        if (MIXED && n < GP) *(u32x4*)(lds + p.q + 2 * (n * D + 32 * kb + 8 * kq)) = st.qa[kb];
       }
-      if (MIXED && n < GP) *(u32x4*)(lds + p.q + 2 * (n * D + 32 * kb + 8 * kq)) = st.qa[kb];
+    } else {
+      // a query of another type as the exact sum of three parts; for fp16
+      // operands it is scaled by a power of two that the logit scale takes back
+      float x[8 * KB];
+#pragma unroll
+      for (int i = 0; i < 8 * KB; ++i) {
+        x[i] = dev_load(a.query, at + 32 * (i >> 3) + 8 * kq + (i & 7), (int)a.q_dtype);
+        x[i] = head < G ? x[i] : 0.f;
+      }
+      const int e = BF ? 0 : query_exponent(x);
+      st.scale = ldexpf(st.scale, e);
+#pragma unroll
+      for (int i = 0; i < 8 * KB; ++i) x[i] = ldexpf(x[i], -e);
+#pragma unroll
+      for (int part = 0; part < 3; ++part) {
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb) {
+          u32x4 row;
+#pragma unroll
+          for (int w = 0; w < 4; ++w) {
+            float &x0 = x[8 * kb + 2 * w], &x1 = x[8 * kb + 2 * w + 1];
+            float r0, r1;
+            row[w] = take_part<BF>(x0, x1, r0, r1);
+            x0 = r0;
+            x1 = r1;
+          }
+          if (part == 0) st.qa[kb] = row;
+          if (n < GP) *(u32x4*)(lds + p.q + 2 * ((part * GP + n) * D + 32 * kb + 8 * kq)) = row;
+        }
+      }
     }
   }
-  // the weight rows past the three parts stay zero
-  for (int i = lane; i < (16 * PASSES - 3 * GP) * St::kPRow / 4; i += 64)
-    *(uint32_t*)(st.pw + 3 * GP * St::kPRow + 4 * i) = 0u;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     st.m_run[i] = -INFINITY;
@@ -537,41 +593,61 @@ __global__ void __launch_bounds__(64 * kTileWaves, 2) decode_tiles(TileParams p)
   // ---- packed tiles ----
   {
     uint32_t kc[KK / 2 * KC::kPairRegs], vc[VK / 2 * VC::kPairRegs];  // the codes of the tile to come
-    uint32_t ksz[KIT], vsz[VIT];  // its scales and zero points
-    int kidx[8];                  // its promoted channels of this lane, first block (slots 8 kq ..)
+    uint16_t ks[KIT], kz[KIT], vs[VIT], vz[VIT];  // its scales and zero points
+    int kidx[4];  // its promoted channels: slots 8 kq + 2 w + odd of the first block
+    int zidx;     // ... and slot `lane`
     auto load_keys = [&](const Packed& t, int t0) {
       const int Gp = groups_of(t.tokens, kgroup), padded = Gp * kgroup;
       const int row = padded * KBITS / 8;  // bytes of a channel
-      const int first = min(t0 + NJ * n, padded - NJ);  // a lane past the page repeats its last tokens
-      const uint32_t off = (uint32_t)(first * KBITS / 8 + 8 * kq * row);
+      constexpr int span = KC::kSpan;
+      const int at = KC::kShared ? n >> 1 : n;
+      const int first = min(t0 + span * at, padded - span);  // a lane past the page repeats its last tokens
+      const uint32_t off = (uint32_t)(first * KBITS / 8) + mul24(8 * kq + (KC::kShared ? odd : 0), row);
       load_codes<KBITS, NJ, KK>(
           kc, [&](int k) { return t.k + (32 * (k >> 3) + (k & 7)) * row; }, [&](int) { return off; });
       const int g0 = t0 / kgroup, ng = min(Gp - g0, max(1, TILE / kgroup));
 #pragma unroll
-      for (int m = 0; m < KIT; ++m)
-        if (m / KSTEP < ng) ksz[m] = load_sz(t.ks, t.kz, lane * Gp, 64 * (m % KSTEP) * Gp + g0 + m / KSTEP);
+      for (int m = 0; m < KIT; ++m) {
+        if (m / KSTEP < ng) {
+          const int step = 64 * (m % KSTEP) * Gp + g0 + m / KSTEP;
+          ks[m] = gload<uint16_t>(t.ks + step, mul24(2 * lane, Gp));
+          kz[m] = gload<uint16_t>(t.kz + step, mul24(2 * lane, Gp));
+        }
+      }
       if constexpr (MIXED) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) kidx[i] = gload<int>(t.ki, 4 * min(8 * kq + i, promoted - 1));
+        for (int w = 0; w < 4; ++w) kidx[w] = gload<int>(t.ki, 4 * min(8 * kq + 2 * w + odd, promoted - 1));
+        zidx = gload<int>(t.ki, 4 * min(lane, promoted - 1));
       }
     };
     auto load_values = [&](const Packed& t, int t0) {
       const int last = t.tokens - 1;
-      const uint32_t col = (uint32_t)(NC * n * VBITS / 8);
+      const uint32_t col = (uint32_t)(VC::kSpan * (VC::kShared ? n >> 1 : n) * VBITS / 8);
+      const int step = VC::kShared ? odd : 0;
       if (t0 + TILE <= t.tokens) {  // a whole tile's addresses step by the row
-        const uint32_t off = col + (uint32_t)(8 * kq * vrow);
+        const uint32_t off = col + mul24(8 * kq + step, vrow);
         load_codes<VBITS, NC, VK>(
             vc, [&](int k) { return t.v + (t0 + 32 * (k >> 3) + (k & 7)) * vrow; }, [&](int) { return off; });
 #pragma unroll
-        for (int m = 0; m < VIT; ++m)
-          if (m / VSTEP < Gv) vsz[m] = load_sz(t.vs, t.vz, lane * Gv, (t0 + 64 * (m % VSTEP)) * Gv + m / VSTEP);
+        for (int m = 0; m < VIT; ++m) {
+          if (m / VSTEP < Gv) {
+            const int item = (t0 + 64 * (m % VSTEP)) * Gv + m / VSTEP;
+            vs[m] = gload<uint16_t>(t.vs + item, mul24(2 * lane, Gv));
+            vz[m] = gload<uint16_t>(t.vz + item, mul24(2 * lane, Gv));
+          }
+        }
       } else {  // a partial one repeats its last token
         load_codes<VBITS, NC, VK>(
             vc, [&](int) { return t.v; },
-            [&](int k) { return col + (uint32_t)(min(t0 + 32 * (k >> 3) + 8 * kq + (k & 7), last) * vrow); });
+            [&](int k) { return col + mul24(min(t0 + 32 * (k >> 3) + 8 * kq + (k & 7) + step, last), vrow); });
 #pragma unroll
-        for (int m = 0; m < VIT; ++m)
-          if (m / VSTEP < Gv) vsz[m] = load_sz(t.vs, t.vz, min(t0 + lane + 64 * (m % VSTEP), last) * Gv, m / VSTEP);
+        for (int m = 0; m < VIT; ++m) {
+          if (m / VSTEP < Gv) {
+            const uint32_t item = 2 * (mul24(min(t0 + lane + 64 * (m % VSTEP), last), Gv) + m / VSTEP);
+            vs[m] = gload<uint16_t>(t.vs, item);
+            vz[m] = gload<uint16_t>(t.vz, item);
+          }
+        }
       }
     };
     const uint8_t* vtab = lds + p.vt + (NC * n / vgroup) * kTabV;
@@ -602,40 +678,42 @@ __global__ void __launch_bounds__(64 * kTileWaves, 2) decode_tiles(TileParams p)
       const int ng = min(Gp - g0, max(1, TILE / kgroup));
       const int lane_group = min((cur0 + NJ * n) / kgroup - g0, ng - 1);
       const int row = Gp * kgroup * KBITS / 8;
-      const uint32_t tok_off = (uint32_t)(min(cur0 + NJ * n, Gp * kgroup - NJ) * KBITS / 8);
-      uint32_t pl[4], ph[4];  // promoted channels' codes of the lane
-      auto load_promoted = [&](int block, const int (&idx)[8]) {
+      // codes of the promoted slots 32 block + 8 kq + 2 w + odd, shared as the others are
+      const uint32_t tok_off = (uint32_t)(min(cur0 + 2 * NJ * (n >> 1), Gp * kgroup - 2 * NJ) / 4);
+      uint32_t pl[4], ph[4];
+      auto load_promoted = [&](int block, const int (&idx)[4]) {
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
-          uint32_t lo[2], hi[2];
-#pragma unroll
-          for (int e = 0; e < 2; ++e) {
-            const int slot = min(32 * block + 8 * kq + 2 * w + e, promoted - 1);
-            const uint32_t la = (uint32_t)((idx[2 * w + e] & (D - 1)) * row) + tok_off, ha = (uint32_t)(slot * row) + tok_off;
-            lo[e] = NJ == 8 ? (uint32_t)gload<uint16_t>(cur.k, la) : (uint32_t)gload<uint8_t>(cur.k, la);
-            hi[e] = NJ == 8 ? (uint32_t)gload<uint16_t>(cur.kh, ha) : (uint32_t)gload<uint8_t>(cur.kh, ha);
-          }
-          pl[w] = lo[0] | (lo[1] << 16);
-          ph[w] = hi[0] | (hi[1] << 16);
+          const int slot = min(32 * block + 8 * kq + 2 * w + odd, promoted - 1);
+          const uint32_t la = mul24(idx[w] & (D - 1), row) + tok_off, ha = mul24(slot, row) + tok_off;
+          pl[w] = NJ == 8 ? gload<uint32_t>(cur.k, la) : (uint32_t)gload<uint16_t>(cur.k, la);
+          ph[w] = NJ == 8 ? gload<uint32_t>(cur.kh, ha) : (uint32_t)gload<uint16_t>(cur.kh, ha);
         }
       };
       if constexpr (MIXED) load_promoted(0, kidx);
+      auto key_item = [&](int m, uint32_t sz) {
+        const int c = lane + 64 * (m % KSTEP), g = m / KSTEP;
+        put_table<BF>(lds + p.kt + g * kTabK, c, sz, KBITS == 2);
+        if (MIXED) *(uint32_t*)(lds + p.sz + 4 * (g * D + c)) = sz;
+      };
 #pragma unroll
-      for (int m = 0; m < KIT; ++m) {
-        if (m / KSTEP < ng) {
-          const int c = lane + 64 * (m % KSTEP), g = m / KSTEP;
-          put_table<BF>(lds + p.kt + g * kTabK, c, ksz[m], KBITS == 2);
-          if (MIXED) *(uint32_t*)(lds + p.sz + 4 * (g * D + c)) = ksz[m];
+      for (int m = 0; m < KIT; ++m)
+        if (m / KSTEP < ng) key_item(m, ks[m] | ((uint32_t)kz[m] << 16));
+#pragma unroll 1
+      for (int m = KIT; m < ng * KSTEP; ++m) {
+        const uint32_t at = 2 * ((lane + 64 * (m % KSTEP)) * Gp + g0 + m / KSTEP);
+        key_item(m, gload<uint16_t>(cur.ks, at) | ((uint32_t)gload<uint16_t>(cur.kz, at) << 16));
+      }
+      if constexpr (MIXED) {  // promoted channels take the 4-bit pass: their 2-bit tables become zero
+        lds_order();
+#pragma unroll 1
+        for (int j = lane; j < promoted; j += 64) {
+          const int c = (j == lane ? zidx : gload<int>(cur.ki, 4 * j)) & (D - 1);
+#pragma unroll 1
+          for (int g = 0; g < ng; ++g) *(uint2*)(lds + p.kt + g * kTabK + 8 * c) = make_uint2(0u, 0u);
         }
       }
-      if constexpr (MIXED) {
-        lds_sync();
-        for (int i = lane; i < promoted * ng; i += 64) {
-          const int g = i / promoted, c = gload<int>(cur.ki, 4 * (i % promoted)) & (D - 1);
-          *(uint2*)(lds + p.kt + g * kTabK + 8 * c) = make_uint2(0u, 0u);
-        }
-      }
-      lds_sync();
+      lds_order();
 
       // ---- S = Q K ----
       float4v S[NJ];
@@ -650,10 +728,11 @@ __global__ void __launch_bounds__(64 * kTileWaves, 2) decode_tiles(TileParams p)
         for (int w = 0; w < 4; ++w) {
           if constexpr (KBITS == 2) {
             const uint4 tt = tab[w];
-            lookup_pair<NJ>(kc[4 * kb + w], tt.x, tt.y, tt.z, tt.w, m3, sel2, op[w]);
+            lookup_pair<NJ>(two_bit_bytes<NJ>(unshare(kc[4 * kb + w], ksel)), tt.x, tt.y, tt.z, tt.w, m3, sel2, op[w]);
           } else {
             const uint4 tt = tab[w / 2];
-            chain_pair<BF, KBITS, NJ>(&kc[KC::kPairRegs * (4 * kb + w)], w % 2 ? tt.z : tt.x, w % 2 ? tt.w : tt.y, op[w]);
+            chain_pair<BF, KBITS, NJ>(&kc[KC::kPairRegs * (4 * kb + w)], w % 2 ? tt.z : tt.x, w % 2 ? tt.w : tt.y, ksel,
+                                      op[w]);
           }
         }
         st.q_products(kb, op, S);
@@ -664,53 +743,67 @@ __global__ void __launch_bounds__(64 * kTileWaves, 2) decode_tiles(TileParams p)
         for (int block = 0; 32 * block < promoted; ++block) {
           if (block) {
 #pragma unroll
-            for (int i = 0; i < 8; ++i) kidx[i] = gload<int>(cur.ki, 4 * min(32 * block + 8 * kq + i, promoted - 1));
+            for (int w = 0; w < 4; ++w) kidx[w] = gload<int>(cur.ki, 4 * min(32 * block + 8 * kq + 2 * w + odd, promoted - 1));
             load_promoted(block, kidx);
           }
-          u32x4 qp;
+          // slots past the last one: zero query, zero scale and zero point
+          const bool whole = 32 * block + 32 <= promoted;
           uint32_t op[4][NJ];
-          const uint16_t* q = (const uint16_t*)(lds + p.q) + (n % GP) * D;
+          u32x4 qp[PARTS ? 3 : 1];
           const uint32_t* sz = (const uint32_t*)(lds + p.sz) + lane_group * D;
 #pragma unroll
           for (int w = 0; w < 4; ++w) {
-            const int slot = 32 * block + 8 * kq + 2 * w;
-            const int c0 = kidx[2 * w] & (D - 1), c1 = kidx[2 * w + 1] & (D - 1);
-            // slots past the last one: zero query, zero scale and zero point
-            uint32_t q0 = q[c0], q1 = q[c1], sz0 = sz[c0], sz1 = sz[c1];
-            q0 = slot < promoted ? q0 : 0u;
-            q1 = slot + 1 < promoted ? q1 : 0u;
-            sz0 = slot < promoted ? sz0 : 0u;
-            sz1 = slot + 1 < promoted ? sz1 : 0u;
-            qp[w] = q0 | (q1 << 16);
-            const half2v s = __builtin_bit_cast(half2v, perm(sz1, sz0, 0x05040100u));
-            const half2v z = __builtin_bit_cast(half2v, perm(sz1, sz0, 0x07060302u));
-            const uint32_t yl = NJ == 8 ? perm(0u, pl[w], 0x03010200u) : perm(pl[w] >> 4, pl[w], 0x06040200u);
-            const uint32_t yh = NJ == 8 ? perm(0u, ph[w], 0x03010200u) : perm(ph[w] >> 4, ph[w], 0x06040200u);
+            const int own = kidx[w] & (D - 1), next = (int)swap_pair((uint32_t)own);
+            const int c0 = odd ? next : own, c1 = odd ? own : next, slot = 32 * block + 8 * kq + 2 * w;
+#pragma unroll
+            for (int part = 0; part < (PARTS ? 3 : 1); ++part) {
+              const uint16_t* q = (const uint16_t*)(lds + p.q) + (part * GP + n % GP) * D;
+              uint32_t v = q[c0] | ((uint32_t)q[c1] << 16);
+              if (!whole) v &= (slot < promoted ? 0xffffu : 0u) | (slot + 1 < promoted ? 0xffff0000u : 0u);
+              qp[part][w] = v;
+            }
+            uint32_t mine = sz[own];
+            if (!whole) mine = slot + odd < promoted ? mine : 0u;
+            const uint32_t other = swap_pair(mine);
+            // (s0, s1) and (z0, z1): the even lane's first
+            const half2v s = __builtin_bit_cast(half2v, perm(other, mine, odd ? 0x01000504u : 0x05040100u));
+            const half2v z = __builtin_bit_cast(half2v, perm(other, mine, odd ? 0x03020706u : 0x07060302u));
+            const uint32_t yl = two_bit_bytes<NJ>(unshare(pl[w], ksel)), yh = two_bit_bytes<NJ>(unshare(ph[w], ksel));
+            // nibbles of positions j and j + 2 (even) and j + 1 and j + 3 (odd) per byte, from both planes
+            const uint32_t even = bit_select(0x33333333u, yl, yh << 2), oddn = bit_select(0x33333333u, yl >> 2, yh);
 #pragma unroll
             for (int j = 0; j < NJ / 2; ++j) {
-              const uint32_t e = ((yl >> (2 * j)) & m3) | (((yh >> (2 * j)) & m3) << 2);
+              const uint32_t e = ((j & 1 ? oddn : even) >> (4 * (j >> 1))) & 0x0f0f0f0fu;
               const half2v x = codes16<false>(e) * s, y = codes16<true>(e) * s;
               op[w][j] = to_operand<BF>(x + z);
               op[w][j + NJ / 2] = to_operand<BF>(y + z);
             }
           }
 #pragma unroll
-          for (int j = 0; j < NJ; ++j) S[j] = mfma<BF>(qp, u32x4{op[0][j], op[1][j], op[2][j], op[3][j]}, S[j]);
+          for (int part = 0; part < (PARTS ? 3 : 1); ++part) {
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) S[j] = mfma<BF>(qp[part], u32x4{op[0][j], op[1][j], op[2][j], op[3][j]}, S[j]);
+          }
         }
       }
       if (live) load_keys(nxt, t0);
-
+      lds_order();
       st.softmax(S, nt);
 
       // ---- value tables (tokens past the tile's end: zero) ----
+      auto value_item = [&](int m, uint32_t sz) {
+        const int tok = lane + 64 * (m % VSTEP);
+        put_table<BF>(lds + p.vt + (m / VSTEP) * kTabV, tok, tok < nt ? sz : 0u, VBITS == 2);
+      };
 #pragma unroll
-      for (int m = 0; m < VIT; ++m) {
-        if (m / VSTEP < Gv) {
-          const int tok = lane + 64 * (m % VSTEP);
-          put_table<BF>(lds + p.vt + (m / VSTEP) * kTabV, tok, tok < nt ? vsz[m] : 0u, VBITS == 2);
-        }
+      for (int m = 0; m < VIT; ++m)
+        if (m / VSTEP < Gv) value_item(m, vs[m] | ((uint32_t)vz[m] << 16));
+#pragma unroll 1
+      for (int m = VIT; m < Gv * VSTEP; ++m) {
+        const uint32_t at = 2 * ((cur0 + min(lane + 64 * (m % VSTEP), nt - 1)) * Gv + m / VSTEP);
+        value_item(m, gload<uint16_t>(cur.vs, at) | ((uint32_t)gload<uint16_t>(cur.vz, at) << 16));
       }
-      lds_sync();
+      lds_order();
 
       // ---- O += P V ----
 #pragma unroll
@@ -721,16 +814,17 @@ __global__ void __launch_bounds__(64 * kTileWaves, 2) decode_tiles(TileParams p)
         for (int w = 0; w < 4; ++w) {
           if constexpr (VBITS == 2) {
             const uint4 tt = tab[w];
-            lookup_pair<NC>(vc[4 * kb + w], tt.x, tt.y, tt.z, tt.w, m3, sel2, op[w]);
+            lookup_pair<NC>(two_bit_bytes<NC>(unshare(vc[4 * kb + w], vsel)), tt.x, tt.y, tt.z, tt.w, m3, sel2, op[w]);
           } else {
             const uint4 tt = tab[w / 2];
-            chain_pair<BF, VBITS, NC>(&vc[VC::kPairRegs * (4 * kb + w)], w % 2 ? tt.z : tt.x, w % 2 ? tt.w : tt.y, op[w]);
+            chain_pair<BF, VBITS, NC>(&vc[VC::kPairRegs * (4 * kb + w)], w % 2 ? tt.z : tt.x, w % 2 ? tt.w : tt.y, vsel,
+                                      op[w]);
           }
         }
         st.p_products(kb, op);
       }
       if (live) load_values(nxt, t0);
-      lds_sync();
+      lds_order();
     }
   }
 
@@ -741,9 +835,11 @@ __global__ void __launch_bounds__(64 * kTileWaves, 2) decode_tiles(TileParams p)
     const int j = i - p.n_packed, e = uni(j < p.packed_first ? j : j + p.n_packed);
     int tokens;
     uint64_t k, v;
+    bool dense = true;
     if (e < n_rest) {
       const_segment& s = rest_entry(d, e);
       tokens = s.tokens;
+      dense = s.key_kind == DKV_KEY_DENSE && s.value_kind == DKV_VALUE_DENSE;
       k = s.key[0] + (uint64_t)(2 * bh * s.key_bh[0]);
       v = s.value[0] + (uint64_t)(2 * bh * s.value_bh[0]);
     } else {
@@ -756,6 +852,10 @@ __global__ void __launch_bounds__(64 * kTileWaves, 2) decode_tiles(TileParams p)
       v = a.tail.value[0] + (uint64_t)(2 * bh * a.tail.value_bh[0]);
     }
     tokens = uni(tokens);
+    if (!dense) {  // (a caller that passed no host copy of the descriptors to check): a NaN record
+      st.m_run[0] = st.m_run[1] = st.m_run[2] = st.m_run[3] = NAN;
+      tokens = 0;
+    }
 #pragma unroll 1
     for (int at = 0; at < tokens; at += TILE)
       st.dense_tile((const uint16_t*)uniform_u64(k), (const uint16_t*)uniform_u64(v), at, min(TILE, tokens - at));
@@ -764,7 +864,6 @@ __global__ void __launch_bounds__(64 * kTileWaves, 2) decode_tiles(TileParams p)
   // ---- partial state ----
   constexpr float unscale = BF ? 1.f : 0.0078125f;
   float* ws = (float*)a.workspace;
-  bool finite = true;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     float l = st.l_part[i];
@@ -780,21 +879,14 @@ __global__ void __launch_bounds__(64 * kTileWaves, 2) decode_tiles(TileParams p)
       rec[0] = st.m_run[i];
       rec[1] = l * unscale;
     }
-    float sum = l;
 #pragma unroll
     for (int j = 0; j < NC; ++j) {
-      float o = st.O[j][i];
+      float o = GP == 4 && kq == 3 ? 0.f : st.O[j][i];  // (the fourth part's rows hold nothing)
       if (GP == 4) o += __shfl_xor(o, 16, 64);
       if (GP <= 8) o += __shfl_xor(o, 32, 64);
       if (writes) rec[2 + NC * n + j] = o * unscale;
-      sum += fabsf(o);
     }
-    finite = finite && (!writes || __builtin_isfinite(sum));
   }
-  // An infinite value times a weight part that is zero is NaN where the weight
-  // itself is not: a split whose sums are not finite is done again one element
-  // at a time.
-  if (__ballot(!finite) != 0ull) scalar_split<D>(p, bhi, split, s0, s1, lane);
 }
 
 bool dense_ok(const dkv_segment& g) {
@@ -824,22 +916,20 @@ bool same_layout(const dkv_segment& a, const dkv_segment& b) {
          a.promoted == b.promoted && a.value_bits == b.value_bits && a.value_group == b.value_group;
 }
 
-template <int D, bool BF, int GP, int KBITS, bool MIXED>
+template <int D, bool BF, int GP, int KBITS, bool MIXED, bool PARTS = false>
 int launch_tiles(TileParams& p, hipStream_t s) {
   constexpr int TILE = KBITS == 8 ? 64 : 128;
-  typedef TileState<D, BF, GP, TILE> St;
+  typedef TileState<D, BF, GP, TILE, PARTS> St;
   const int kgroups = p.key_group >= TILE ? 1 : TILE / p.key_group;
   const int vgroups = (D + p.value_group - 1) / p.value_group;
   int o = 0;
-  p.kt = o; o += kgroups * (D * 8 + 16);
-  p.vt = o; o += vgroups * (TILE * 8 + 16);
-  p.pw = o; o += 16 * St::PASSES * St::kPRow;
-  p.sz = o; o += MIXED ? kgroups * D * 4 : 0;
-  p.q = o; o += MIXED ? GP * D * 2 : 0;
+  p.kt = p.vt = o; o += std::max(kgroups * (D * 8 + 16), vgroups * (TILE * 8 + 16));
+  p.pw = p.sz = o; o += std::max(16 * St::PASSES * St::kPRow, MIXED ? kgroups * D * 4 : 0);
+  p.q = o; o += MIXED || PARTS ? (PARTS ? 3 : 1) * GP * D * 2 : 0;
   p.wave_bytes = o;
   const int64_t workers = p.d.a.B * p.d.a.Hkv * p.splits;
   const dim3 grid((unsigned)((workers + kTileWaves - 1) / kTileWaves));
-  hipLaunchKernelGGL((decode_tiles<D, BF, GP, KBITS, MIXED, KBITS>), grid, dim3(64 * kTileWaves),
+  hipLaunchKernelGGL((decode_tiles<D, BF, GP, KBITS, MIXED, KBITS, PARTS>), grid, dim3(64 * kTileWaves),
                      (size_t)kTileWaves * o, s, p);
   return dkv_check_launch("dkv_decode_attention(tiles)");
 }
@@ -862,6 +952,31 @@ int launch_tiles_heads(TileParams& p, int bits, bool mixed, hipStream_t s) {
 }  // namespace
 
 namespace dkv {
+
+bool tiles_take_run(const dkv_decode_args& a, int group) {
+  if (a.fast_promoted > 0) return group == 16;
+  return a.q_dtype == a.cache_dtype && a.fast_key_bits == a.fast_value_bits && 128 / a.fast_value_group <= kMaxGroups &&
+         ((group >= 8 && a.fast_key_bits < 8) || a.B * a.Hkv * a.fast_count >= 2048);
+}
+
+int launch_tile_run(const DecodeParams& d, int first, int count, int splits, const TileLayout& g, hipStream_t s) {
+  const dkv_decode_args& a = d.a;
+  DKV_CHECK(a.B * a.Hkv * splits < (int64_t)1 << 31, DKV_ERR_UNSUPPORTED, "too many splits for one launch");
+  TileParams p;
+  p.d = d;
+  p.splits = splits;
+  p.packed_first = first;
+  p.n_packed = count;
+  p.key_group = g.key_group;
+  p.value_group = g.value_group;
+  p.promoted = g.promoted;
+  const bool mixed = g.promoted > 0, bf = a.cache_dtype == kBF16;
+  if (a.q_dtype != a.cache_dtype)  // (16 heads on Dart pages: tiles_take_run)
+    return bf ? launch_tiles<128, true, 16, 2, true, true>(p, s) : launch_tiles<128, false, 16, 2, true, true>(p, s);
+  if (a.D == 64)
+    return bf ? launch_tiles_heads<64, true>(p, g.bits, mixed, s) : launch_tiles_heads<64, false>(p, g.bits, mixed, s);
+  return bf ? launch_tiles_heads<128, true>(p, g.bits, mixed, s) : launch_tiles_heads<128, false>(p, g.bits, mixed, s);
+}
 
 int launch_tile_decode(const DecodeParams& d, hipStream_t stream, bool* taken) {
   *taken = false;
@@ -887,25 +1002,13 @@ int launch_tile_decode(const DecodeParams& d, hipStream_t stream, bool* taken) {
     else if (i != first + count || !same_layout(entry(first), g)) return DKV_OK;
     ++count;
   }
-  TileParams p;
-  p.d = d;
-  p.splits = d.splits;
-  p.packed_first = first;
-  p.n_packed = count;
-  // (without packed segments the layout is not used)
-  const dkv_segment* g = count ? &entry(first) : nullptr;
-  p.key_group = g ? g->key_group : 128;
-  p.value_group = g ? g->value_group : 64;
-  const bool mixed = g && g->key_kind == DKV_KEY_MIXED;
-  p.promoted = mixed ? g->promoted : 0;
-  const int bits = g ? g->value_bits : 2;
+  TileLayout l{2, 128, 64, 0};  // (without packed segments the layout is not used)
+  if (count) {
+    const dkv_segment& g = entry(first);
+    l = TileLayout{g.value_bits, g.key_group, g.value_group, g.key_kind == DKV_KEY_MIXED ? g.promoted : 0};
+  }
   *taken = true;
-  const bool bf = a.cache_dtype == kBF16;
-  if (a.D == 64)
-    return bf ? launch_tiles_heads<64, true>(p, bits, mixed, stream)
-              : launch_tiles_heads<64, false>(p, bits, mixed, stream);
-  return bf ? launch_tiles_heads<128, true>(p, bits, mixed, stream)
-            : launch_tiles_heads<128, false>(p, bits, mixed, stream);
+  return launch_tile_run(d, first, count, d.splits, l, stream);
 }
 
 }  // namespace dkv

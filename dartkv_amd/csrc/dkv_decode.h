@@ -38,6 +38,16 @@ int launch_uniform_decode(const dkv_decode_args& a, int first, int count, int kb
 // caches (decode_tiles.hip); *taken is false, and nothing is launched, when
 // they are not of the forms that kernel reads.
 int launch_tile_decode(const DecodeParams& d, hipStream_t stream, bool* taken);
+
+// Whether the tile kernel takes a call's page run instead of the page kernels
+// (the run is as dkv_decode_args guarantees), and its launch over `count`
+// packed entries from `first` on and the dense entries around them (d.n_total
+// in all, none skipped), writing `splits` records from d.split_offset on.
+struct TileLayout {
+  int bits, key_group, value_group, promoted;  // promoted 0: uniform pages
+};
+bool tiles_take_run(const dkv_decode_args& a, int group);
+int launch_tile_run(const DecodeParams& d, int first, int count, int splits, const TileLayout& g, hipStream_t stream);
 // LDS bytes of one wave of the uniform page kernel.
 size_t uniform_decode_wave_lds_bytes(int kb, int vb, int gv);
 

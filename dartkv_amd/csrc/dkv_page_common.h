@@ -212,6 +212,15 @@ __device__ __forceinline__ void lds_sync() {
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
+// LDS traffic of this wave before and after stays in program order.  A wave's
+// LDS operations execute in order, so what one lane writes another lane of the
+// wave reads after this without a wait; only LDS DMA (vector memory) needs
+// lds_sync before it overwrites what was read.
+__device__ __forceinline__ void lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 // Wait until at most n vector-memory operations of this wave are outstanding
 // (loads complete in issue order), and until all LDS traffic is done.
 // gfx9 s_waitcnt encoding: vmcnt[3:0] in bits 3:0, expcnt in 6:4 (7 = no

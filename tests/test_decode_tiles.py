@@ -122,3 +122,38 @@ def test_tile_kernel_keeps_infinite_dense_values(dtype):
     expected = torch.zeros(1, 6, 1, 64, dtype=torch.bool)
     expected[0, 3:, 0, 5] = True
     assert torch.equal(torch.isinf(out), expected) and not torch.isnan(out).any()
+
+
+@pytest.mark.parametrize("G,T,dtype,q_dtype,cfg", [
+    (16, 700, BF, BF, dict(promote_ratio=0.25)),                 # sixteen rows on Dart pages, dense pieces beside
+    (16, 900, FP, torch.float32, dict(promote_ratio=0.5)),       # a query of another type: three exact parts
+    (16, 900, BF, FP, dict(promote_ratio=0.125, value_group_size=16)),
+    (16, 1000, BF, torch.float64, dict(promote_ratio=0.25, hold_partial_pages=False)),  # a short page in the rest
+    (8, 900, BF, BF, dict(bits=4, promote_ratio=0.0)),           # uniform pages with eight rows
+    (8, 1000, FP, FP, dict(bits=8, promote_ratio=0.0, hold_partial_pages=False)),
+    (8, 800, BF, FP, dict(bits=2, promote_ratio=0.0)),           # ... and another query type: the page kernel
+    (8, 800, BF, BF, dict(bits=4, value_bits=2, promote_ratio=0.0)),
+])
+def test_page_runs_the_tile_kernel_takes(G, T, dtype, q_dtype, cfg):
+    """Full-page runs on their way through the page path's arguments (splits, events, dense rest, records)."""
+    import dartkv_amd as dart
+    from dartkv_amd import synthetic
+    from oracle import dart_oracle as O
+    cfg = dict(dict(bits=2, page_size=128, key_group_size=128, value_group_size=64, sink_tokens=32,
+                    hold_partial_pages=True, metadata_dtype=torch.float16), **cfg)
+    k, v, q = synthetic.outlier_kv(2, 2, T, 128, query_heads=2 * G, dtype=torch.float32, seed=T + G)
+    k, v, q = k.to(dtype), v.to(dtype), q.to(q_dtype)
+    oc, cache = O.OracleCache(O.OracleConfig(**cfg)), dart.DartKVCache(dart.DartKVCacheConfig(**cfg))
+    oc.append(k, v)
+    cache.append(k.to(DEV), v.to(DEV))
+    ref = O.streamed_attention(q, oc, return_fp32=True)[1]
+    out = torch.empty(2, 2 * G, 128, dtype=torch.float32, device=DEV)
+    print("case", G, T, dtype, q_dtype, cfg, flush=True)
+    events = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+    for e in events:
+        e.record()
+    got = dart.decode_attention(q.to(DEV), cache, out_f32=out, fast=True, fast_events=events)
+    torch.cuda.synchronize()
+    assert got.dtype == q_dtype and events[0].elapsed_time(events[1]) >= 0
+    tiles = G == 16 or (q_dtype == dtype and "value_bits" not in cfg and cfg["bits"] < 8)
+    assert _rel_err(out.unsqueeze(2), ref) <= (1e-5 if tiles else 2e-3)
