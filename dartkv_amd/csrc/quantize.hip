@@ -919,6 +919,36 @@ struct ColumnParams {
 
 constexpr int kColumnTokens = 128;
 
+// A lane's 64 tokens of its channels: the block's rows from a wave-uniform
+// base, the lane's offset in 32 bits.
+template <int SRC>
+__device__ __forceinline__ void load_columns(const ColumnParams& p, int64_t bh, int64_t page, int block, int half,
+                                             int c0, uint32_t (&w)[64]) {
+  constexpr int kSize = SRC == kF32 ? 4 : 2;
+  const uint8_t* base = (const uint8_t*)p.src +
+                        kSize * ((bh / p.H) * p.sb + (bh % p.H) * p.sh + (page * p.T + block * kColumnTokens) * p.st);
+  if ((block + 1) * kColumnTokens <= p.T) {
+    const uint32_t off = (uint32_t)kSize * (64u * half * (uint32_t)p.st + c0);
+#pragma unroll
+    for (int j = 0; j < 64; ++j) w[j] = *(const uint32_t*)(base + kSize * j * p.st + off);
+  } else {
+    const int last = p.T - 1 - block * kColumnTokens;
+#pragma unroll
+    for (int j = 0; j < 64; ++j) {
+      w[j] = *(const uint32_t*)(base + (uint32_t)kSize * ((uint32_t)min(64 * half + j, last) * (uint32_t)p.st + c0));
+      if (j % 8 == 7) __builtin_amdgcn_sched_barrier(0);  // eight addresses at a time
+    }
+  }
+}
+
+// Channel k of a loaded word.
+template <int SRC>
+__device__ __forceinline__ float column_elem(uint32_t w, int k) {
+  if (SRC == kF32) return __builtin_bit_cast(float, w);
+  if (SRC == kBF16) return __builtin_bit_cast(float, k ? w & 0xffff0000u : w << 16);
+  return (float)__builtin_bit_cast(_Float16, (uint16_t)(w >> (16 * k)));
+}
+
 template <int SRC, int BITS, int KG>
 __global__ void __launch_bounds__(kThreads, 4) quantize_key_columns(ColumnParams p) {
   constexpr int NCH = SRC == kF32 ? 1 : 2;
@@ -934,30 +964,11 @@ __global__ void __launch_bounds__(kThreads, 4) quantize_key_columns(ColumnParams
   const int64_t r1 = r0 / p.blocks, bh = r1 % p.bhs, page = r1 / p.bhs;
   const int c0 = (chunk * 32 + (lane & 31)) * NCH;
   const int t0 = block * kColumnTokens + 64 * half;
-  // the block's rows from a wave-uniform base; a lane's offset is 32 bits
-  constexpr int kSize = SRC == kF32 ? 4 : 2;
-  const uint8_t* base = (const uint8_t*)p.src +
-                        kSize * ((bh / p.H) * p.sb + (bh % p.H) * p.sh + (page * p.T + block * kColumnTokens) * p.st);
   uint32_t w[64];
-  if ((block + 1) * kColumnTokens <= p.T) {
-    const uint32_t off = (uint32_t)kSize * (64u * half * (uint32_t)p.st + c0);
-#pragma unroll
-    for (int j = 0; j < 64; ++j) w[j] = *(const uint32_t*)(base + kSize * j * p.st + off);
-  } else {
-    const int last = p.T - 1 - block * kColumnTokens;
-#pragma unroll
-    for (int j = 0; j < 64; ++j) {
-      w[j] = *(const uint32_t*)(base + (uint32_t)kSize * ((uint32_t)min(64 * half + j, last) * (uint32_t)p.st + c0));
-      if (j % 8 == 7) __builtin_amdgcn_sched_barrier(0);  // eight addresses at a time
-    }
-  }
+  load_columns<SRC>(p, bh, page, block, half, c0, w);
 #pragma unroll
   for (int k = 0; k < NCH; ++k) {
-    auto x = [&](int j) -> float {
-      if (SRC == kF32) return __builtin_bit_cast(float, w[j]);
-      if (SRC == kBF16) return __builtin_bit_cast(float, k ? w[j] & 0xffff0000u : w[j] << 16);
-      return (float)__builtin_bit_cast(_Float16, (uint16_t)(w[j] >> (16 * k)));
-    };
+    auto x = [&](int j) -> float { return column_elem<SRC>(w[j], k); };
     const int64_t channel = bh * p.D + c0 + k;
 #pragma unroll
     for (int s = 0; s < 64 / SG; ++s) {
@@ -1410,6 +1421,170 @@ __global__ void __launch_bounds__(kThreads) select_pages_and_rows(KeyParams k, i
   rows_vec_body<BITS, SRC, E>(p, lpg, row_shift, b % gx, b / gx, gx, gy);
 }
 
+// Dart pages of at most 128 tokens from the same registers, where the
+// single-pass kernel below does not apply (key groups of 32 and 64, head_dim
+// 64, fp32): one pass leaves each channel's score at the start of the page's
+// low-code region, key_select_pages chooses, a second pass reads the keys again
+// and writes the codes.  The tiled kernel's staging through LDS and its one
+// thread per channel took 50 µs a pass (mean over prefills of 16 x 8 x 4,096
+// tokens of head_dim 64, 8 x 8 x 4,096 with groups of 64, and two of one
+// sequence); these take 10 and 14 µs.  A prefill of 4 x 4 x 230 tokens with its
+// first decode 232 -> 196 µs.
+//
+// A score is the token mean in ATen's cascade order (channel_mean): each lane
+// sums its four runs of 16 tokens one by one, the runs are added in order over
+// both halves of the page, a short last run first.
+template <int SRC, bool SQUARES>
+__device__ __forceinline__ float column_mean(uint32_t (&w)[64], int k, int half, int T, bool magnitude, float center) {
+  float run[4], other[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    int left = T - 64 * half - 16 * q;
+    asm volatile("" : "+v"(left));  // its comparisons are made here, not kept for every run and channel
+    float acc = 0.f;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      asm volatile("" : "+v"(w[16 * q + j]));  // converted here
+      const float x = column_elem<SRC>(w[16 * q + j], k);
+      float term = magnitude ? fabsf(x) : x;
+      if (SQUARES) {
+        const float d = src_round<SRC>(__fsub_rn(x, center));
+        term = src_round<SRC>(__fmul_rn(d, d));
+      }
+      acc = __fadd_rn(acc, j < left ? term : 0.f);
+    }
+    run[q] = acc;
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) other[q] = __shfl_xor(run[q], 32, 64);
+  float sum = 0.f, rest = 0.f;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const float r = (q < 4) == (half == 0) ? run[q % 4] : other[q % 4];
+    if (16 * q + 16 <= T) sum = __fadd_rn(sum, r);
+    else if (16 * q < T) rest = r;
+  }
+  float acc = __fadd_rn(rest, sum);
+  acc = __fadd_rn(__fadd_rn(acc, 0.f), 0.f);  // the cascade's empty upper levels
+  return src_round<SRC>(__fdiv_rn(acc, (float)T));
+}
+
+struct DartColumnParams {
+  ColumnParams c;  // (bits 2)
+  int K, variance, source;  // promoted channels; where they come from (kIdx...)
+  uint8_t* high;
+  int32_t* idx;
+  const int32_t* given;
+  int64_t high_page_stride, idx_page_stride;
+};
+constexpr int kIdxChosen = 0, kIdxGiven = 1, kIdxAll = 2;
+
+template <int SRC>
+__global__ void __launch_bounds__(kThreads, 4) dart_column_scores(DartColumnParams p) {
+  constexpr int NCH = SRC == kF32 ? 1 : 2;
+  const ColumnParams& c = p.c;
+  const int64_t item = (int64_t)blockIdx.x * (kThreads / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (item >= c.items) return;
+  const int lane = threadIdx.x & 63, half = lane >> 5;
+  const int chunk = (int)(item % c.chunks);
+  const int64_t r = item / c.chunks, bh = r % c.bhs, page = r / c.bhs;
+  const int c0 = (chunk * 32 + (lane & 31)) * NCH;
+  uint32_t w[64];
+  load_columns<SRC>(c, bh, page, 0, half, c0, w);
+  float* score = (float*)(c.low + page * c.low_page_stride + bh * c.D * c.pk);
+#pragma unroll
+  for (int k = 0; k < NCH; ++k) {
+    float v = column_mean<SRC, false>(w, k, half, c.T, !p.variance, 0.f);
+    if (p.variance) v = column_mean<SRC, true>(w, k, half, c.T, false, v);  // mixed.py:159-160
+    if (half == 0) score[c0 + k] = v;
+  }
+}
+
+template <int SRC, int KG>
+__global__ void __launch_bounds__(kThreads, 4) dart_column_codes(DartColumnParams p) {
+  constexpr int NCH = SRC == kF32 ? 1 : 2;
+  constexpr int SG = KG < 64 ? KG : 64;  // tokens of a group in one lane
+  __shared__ int16_t slots[kThreads / 64][kSelectMaxD];
+  const ColumnParams& c = p.c;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t item = (int64_t)blockIdx.x * (kThreads / 64) + wave;
+  if (item >= c.items) return;
+  const int lane = threadIdx.x & 63, half = lane >> 5;
+  const int chunk = (int)(item % c.chunks);
+  const int64_t r = item / c.chunks, bh = r % c.bhs, page = r / c.bhs;
+  const int c0 = (chunk * 32 + (lane & 31)) * NCH, t0 = 64 * half;
+  uint32_t w[64];
+  load_columns<SRC>(c, bh, page, 0, half, c0, w);
+  // slot of each channel (-1: not promoted); the first piece's wave writes the indices it made
+  int16_t* slot = slots[wave];
+  for (int i = lane; i < c.D; i += 64) slot[i] = -1;
+  DeviceWave{lane}.sync();
+  int32_t* idx = (int32_t*)((char*)p.idx + page * p.idx_page_stride) + bh * p.K;
+  for (int j = lane; j < p.K; j += 64) {
+    const int ch = p.source == kIdxChosen ? idx[j] : p.source == kIdxAll ? j : p.given[(bh % c.H) * p.K + j];
+    if (ch >= 0 && ch < c.D) slot[ch] = (int16_t)j;
+    if (p.source != kIdxChosen && chunk == 0) idx[j] = ch;
+  }
+  DeviceWave{lane}.sync();
+#pragma unroll
+  for (int k = 0; k < NCH; ++k) {
+    auto x = [&](int j) -> float { return column_elem<SRC>(w[j], k); };
+    const int sl = slot[c0 + k];
+    const float qmax = sl >= 0 ? 15.f : 3.f, inv_qmax = sl >= 0 ? 1.0f / 15.0f : 1.0f / 3.0f;
+    const int64_t channel = bh * c.D + c0 + k;
+#pragma unroll
+    for (int s = 0; s < 64 / SG; ++s) {
+      float mn = x(s * SG), mx = mn;
+#pragma unroll
+      for (int j = 1; j < SG; ++j) {
+        mn = nmin(mn, x(s * SG + j));
+        mx = nmax(mx, x(s * SG + j));
+      }
+      if (KG == 128) {
+        mn = nmin(mn, __shfl_xor(mn, 32, 64));
+        mx = nmax(mx, __shfl_xor(mx, 32, 64));
+      }
+      const int g = (t0 + s * SG) / KG;
+      if (g >= c.G) continue;  // (both halves of a 128-token group agree)
+#pragma unroll
+      for (int j = 0; j < SG; ++j) asm volatile("" : "+v"(w[s * SG + j]));  // converted again below
+      const float sc = rows_group_scale<SRC>(mn, mx, qmax, inv_qmax);
+      const float y = __fdiv_rn(1.0f, sc);
+      if (KG < 128 || half == 0) {
+        flag_nonfinite(c.nonfinite, mn, mx);
+        dev_store_meta((char*)c.scale + page * c.scale_page_stride, channel * c.G + g, sc, c.meta_dtype);
+        dev_store_meta((char*)c.zero + page * c.zero_page_stride, channel * c.G + g, mn, c.meta_dtype);
+      }
+      constexpr int kWords = SG / 16;
+      uint32_t lo[kWords], hi[kWords];
+#pragma unroll
+      for (int d = 0; d < kWords; ++d) {
+        uint32_t plane[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+          float xs[4], q[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) xs[i] = x(s * SG + 16 * d + 4 * h + i);
+          chain_quotients4<SRC>(xs, mn, sc, y, q);
+          codes_to_planes2(q, h, plane);
+        }
+        lo[d] = pack2_low(plane);
+        hi[d] = pack2_high(plane);
+      }
+      const int at = (t0 + s * SG) / 4;
+      uint8_t* low = c.low + page * c.low_page_stride + channel * c.pk + at;
+      uint8_t* high = p.high + page * p.high_page_stride + (bh * p.K + sl) * c.pk + at;
+      if constexpr (kWords == 2) {
+        *(uint2*)low = make_uint2(lo[0], lo[1]);
+        if (sl >= 0) *(uint2*)high = make_uint2(hi[0], hi[1]);
+      } else {
+        *(uint4*)low = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+        if (sl >= 0) *(uint4*)high = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+      }
+    }
+  }
+}
+
 __host__ inline size_t key_tiled_smem(int D, int T, int G, int K, int row_bytes) {
   size_t o = ((size_t)T * key_tile_row_bytes(D) + 15) & ~(size_t)15;
   o += sizeof(float) * ((size_t)D + 2 * (size_t)D * G) + 2 * sizeof(int32_t) * D + sizeof(SelItem) * D;
@@ -1741,22 +1916,27 @@ extern "C" int dkv_quantize_key_pages(const dkv_key_pages_args* args, void* stre
                          ((int64_t)a.D * row_bytes) % 16 == 0 &&
                          (Kp == 0 || (((uintptr_t)a.high % 16) == 0 && (a.high_page_stride % 16) == 0 &&
                                       ((int64_t)Kp * row_bytes) % 16 == 0));
-  // uniform keys from registers; the single-pass kernel below keeps its shape
+  // keys from registers: uniform pages of any size, Dart pages of one block
+  // (selection needs a page's tokens in one wave); the single-pass kernel below keeps its shape
   // (one 128-token group per page of head_dim 128)
   const int row_piece = a.src_dtype == kF32 ? 32 : 64;  // channels of a 128-byte piece
-  const int col_store = std::min<int>(16, (int)std::min<int64_t>(a.group, 64) * (int)a.bits / 8);
-  const bool use_columns =
-      a.key_mode == DKV_KEY_UNIFORM && (a.group == 32 || a.group == 64 || a.group == 128) &&
+  const int col_store = std::min<int>(16, (int)std::min<int64_t>(a.group, 64) * (a.key_mode == DKV_KEY_MIXED ? 2 : (int)a.bits) / 8);
+  const bool columns_fit =
+      (a.group == 32 || a.group == 64 || a.group == 128) &&
       (a.src_dtype == kBF16 || a.src_dtype == kF16 || a.src_dtype == kF32) && a.sd == 1 && a.D % row_piece == 0 &&
       a.page_tokens < (1 << 28) && a.st >= 0 && a.st < (1 << 21) && ((uintptr_t)a.src % 4) == 0 &&
       (a.src_dtype == kF32 || (a.st % 2 == 0 && a.sb % 2 == 0 && a.sh % 2 == 0)) &&
       ((uintptr_t)a.low % col_store) == 0 && (a.low_page_stride % col_store) == 0 &&
       !(a.src_dtype != kF32 && a.D == kFastKeyD && a.page_tokens <= kFastKeyT && a.group == kFastKeyT);
-  if (use_columns) {
+  const bool use_columns = columns_fit && a.key_mode == DKV_KEY_UNIFORM;
+  const bool use_dart_columns =
+      columns_fit && a.key_mode == DKV_KEY_MIXED && a.page_tokens <= kColumnTokens && a.D <= kSelectMaxD &&
+      (Kp == 0 || (((uintptr_t)a.high % col_store) == 0 && (a.high_page_stride % col_store) == 0));
+  if (use_columns || use_dart_columns) {
     ColumnParams c;
     c.src = a.src;
     c.sb = a.sb; c.sh = a.sh; c.st = a.st;
-    c.H = (int)a.H; c.D = (int)a.D; c.T = (int)a.page_tokens; c.G = (int)k.G; c.pk = (int)k.pk;
+    c.H = (int)a.H; c.D = (int)a.D; c.T = (int)a.page_tokens; c.G = (int)k.G; c.pk = row_bytes;
     c.blocks = (int)((a.page_tokens + kColumnTokens - 1) / kColumnTokens);
     c.chunks = (int)(a.D / row_piece);
     c.bhs = a.B * a.H;
@@ -1769,6 +1949,33 @@ extern "C" int dkv_quantize_key_pages(const dkv_key_pages_args* args, void* stre
     const int64_t waves = kThreads / 64, wgs = (c.items + waves - 1) / waves;
     DKV_CHECK(wgs < (int64_t)1 << 31, DKV_ERR_UNSUPPORTED, "too many pages for one launch");
     const dim3 grid((unsigned)wgs);
+    if (use_dart_columns) {
+      DartColumnParams d;
+      d.c = c;
+      d.K = Kp;
+      d.variance = a.selection == DKV_SELECT_VARIANCE;
+      d.source = Kp == a.D ? kIdxAll : a.selection == DKV_SELECT_GIVEN ? kIdxGiven : kIdxChosen;
+      d.high = a.high;
+      d.idx = a.idx;
+      d.given = a.given_idx;
+      d.high_page_stride = a.high_page_stride;
+      d.idx_page_stride = a.idx_page_stride;
+#define DKV_DART(T)                                                                                             \
+  do {                                                                                                          \
+    if (Kp > 0 && d.source == kIdxChosen) {                                                                     \
+      hipLaunchKernelGGL((dart_column_scores<T>), grid, dim3(kThreads), 0, s, d);                               \
+      hipLaunchKernelGGL(key_select_pages, dim3((unsigned)(c.bhs * a.n_pages)), dim3(64), 0, s, k, row_bytes);  \
+    }                                                                                                           \
+    if (a.group == 32) hipLaunchKernelGGL((dart_column_codes<T, 32>), grid, dim3(kThreads), 0, s, d);           \
+    else if (a.group == 64) hipLaunchKernelGGL((dart_column_codes<T, 64>), grid, dim3(kThreads), 0, s, d);      \
+    else hipLaunchKernelGGL((dart_column_codes<T, 128>), grid, dim3(kThreads), 0, s, d);                        \
+  } while (0)
+      if (a.src_dtype == kBF16) DKV_DART(kBF16);
+      else if (a.src_dtype == kF16) DKV_DART(kF16);
+      else DKV_DART(kF32);
+#undef DKV_DART
+      return finish();
+    }
 #define DKV_COL(T, B)                                                                                           \
   do {                                                                                                          \
     if (a.group == 32) hipLaunchKernelGGL((quantize_key_columns<T, B, 32>), grid, dim3(kThreads), 0, s, c);     \

@@ -1,4 +1,4 @@
-"""Uniform keys quantized along tokens from registers (groups of 32, 64 and 128) and the eight-element dequantize kernel,
+"""Keys quantized along tokens from registers (groups of 32, 64 and 128; uniform and Dart pages) and the eight-element dequantize kernel,
 bit for bit against the oracle: every code width and source type, tokens that do not fill a group, a block or a page,
 strided sources, and the non-finite report."""
 
@@ -72,6 +72,34 @@ def test_uniform_pages_vs_oracle_from_a_strided_source(D, dtype, cfg):
                 assert _same(g, r)
             else:
                 assert all(_same(getattr(g, n), getattr(r, n)) for n in ("values", "scale", "zero_point"))
+
+
+@pytest.mark.parametrize("D,dtype,ratio,cfg", [
+    (64, BF, 0.25, dict(key_group_size=128)),                              # last page of 11 tokens: half a page each
+    (64, FP, 0.25, dict(key_group_size=32, sink_tokens=73)),               # 66 tokens
+    (64, FP, 0.5, dict(key_group_size=64, channel_selection="variance")),
+    (128, BF, 0.25, dict(key_group_size=64, channel_selection="variance", sink_tokens=73)),
+    (128, BF, 0.125, dict(key_group_size=32, page_size=100)),
+    (128, FP, 0.25, dict(key_group_size=64, page_size=16)),
+    (128, F32, 0.25, dict(key_group_size=128, channel_selection="variance")),
+    (96, F32, 0.25, dict(key_group_size=32, sink_tokens=60)),
+    (64, BF, 1.0, dict(key_group_size=64)),                                # every channel promoted
+])
+def test_dart_pages_vs_oracle_from_a_strided_source(D, dtype, ratio, cfg):
+    """Scores (both selections), the chosen channels in their order, low and high codes, scales and zero points."""
+    import dartkv_amd as dart
+    from oracle import dart_oracle as O
+    cfg = dict(cfg, bits=2, value_group_size=32, promote_ratio=ratio)
+    k, v = (_data((2, 523, 3, D), dtype, s).transpose(1, 2) for s in (3, 4))
+    oc, cache = O.OracleCache(O.OracleConfig(**cfg)), dart.DartKVCache(dart.DartKVCacheConfig(**cfg))
+    oc.append(k, v)
+    cache.append(k.to(DEV), v.to(DEV))
+    print("case", D, dtype, ratio, cfg, flush=True)
+    pairs = [(g, r) for g, r in zip(cache.iter_segments(), oc.segments()) if not isinstance(g[0], torch.Tensor)]
+    assert len(pairs) == (523 - cfg.get("sink_tokens", 0) + cfg.get("page_size", 128) - 1) // cfg.get("page_size", 128)
+    for (got, _), (ref, _) in pairs:
+        for name in ("low_values", "high_values", "channel_indices", "scale", "zero_point"):
+            assert _same(getattr(got, name), getattr(ref, name)), name
 
 
 @pytest.mark.parametrize("bad", [float("nan"), float("inf"), float("-inf")])
