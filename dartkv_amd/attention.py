@@ -291,6 +291,17 @@ def _fast_rows(plan) -> Tuple[int, ...]:
     return (1, 2, 4, 8, 16) if plan.fast_promoted else (1, 2, 4, 8)
 
 
+def _page_kernel_only(query: torch.Tensor, cache: DartKVCache, plan) -> bool:
+    """Whether the cache has pages that a page kernel takes and the tile kernel, which takes any row count up to
+    16, would leave to the general kernel: a query of another dtype, key and value codes of different widths,
+    value groups of 16, or entries beside the pages that are not dense."""
+    if plan.fast_count == 0 or not _fast_enabled():
+        return False
+    tiles = (query.dtype == cache.dtype and (plan.fast_promoted or plan.fast_key_bits == plan.fast_value_bits)
+             and plan.fast_value_group >= 32 and plan.rest_dense >= 0)
+    return not (tiles and (not plan.tail_is_pending or tail_segment(cache, with_dense_check=True)[1]))
+
+
 def _multi_token_attention(query: torch.Tensor, cache: DartKVCache, *, scale: Optional[float] = None,
                            out_f32: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Several query tokens per head over the packed cache.
@@ -299,24 +310,36 @@ def _multi_token_attention(query: torch.Tensor, cache: DartKVCache, *, scale: Op
     mask (attention.py:67-87), so token i of query head h is one more query
     row of h's KV group.  A [B, Hq, c, D] slice of the query read as a
     [B, Hq * c, D] query keeps that grouping (row h * c + i belongs to KV head
-    h // G), and the single-token HIP decode path runs it unchanged: the MFMA
-    page kernel while G * c fits its rows per KV head (8, or 16 on Dart pages:
-    the dequantized pages serve all rows of a launch), the general kernel up to
-    16.  ``out_f32`` ([B, Hq, Q, D] float32) receives the result before the cast.
+    h // G), and the single-token HIP decode path runs it unchanged.  A launch
+    takes 16 rows per KV head, the most of the kernels: the pages are unpacked
+    once per launch.  Where only the page kernel takes a cache's pages
+    (``_page_kernel_only``) it takes what that kernel has rows for.  Four
+    tokens, four heads per KV head: 102 -> 24 µs for 8 x 8 x 4,096 tokens with
+    key groups of 64 (four launches -> one), 64 -> 28 with uniform 4-bit pages
+    (two -> one), 728 -> 333 for 4 x 4 x 2,000 with groups of 40 (general
+    kernel).  ``out_f32`` ([B, Hq, Q, D] float32) receives the result before
+    the cast.
     """
     batch, kv_heads, head_dim = cache.shape[0], cache.shape[1], cache.shape[3]
     Hq, Q = query.shape[1], query.shape[-2]
     groups = Hq // kv_heads
     plan = cache.decode_plan(query.device)
-    rows = _fast_rows(plan) if plan.fast_count > 0 and _fast_enabled() else (1, 2, 4)
+    rows = _fast_rows(plan) if _page_kernel_only(query, cache, plan) else ()
     fits = [c for c in range(1, Q + 1) if groups * c in rows]  # token counts a page-kernel launch takes
     if out_f32 is not None and (out_f32.shape != (batch, Hq, Q, head_dim) or out_f32.dtype != torch.float32):
         raise ValueError("out_f32 must be a float32 [B, Hq, Q, D] tensor")
+
+    def tokens(left: int) -> int:  # of the next launch
+        return max((c for c in fits if c <= left), default=min(left, max(1, 16 // groups)))
+
+    if tokens(Q) == Q and (out_f32 is None or out_f32.is_contiguous()):  # one launch: its output is the result
+        o = decode_attention(query.reshape(batch, Hq * Q, head_dim), cache, scale=scale,
+                             out_f32=None if out_f32 is None else out_f32.view(batch, Hq * Q, head_dim))
+        return o.view(batch, Hq, Q, head_dim)
     out = torch.empty(batch, Hq, Q, head_dim, dtype=query.dtype, device=query.device)
     start = 0
     while start < Q:
-        left = [c for c in fits if c <= Q - start]
-        c = max(left) if left else min(Q - start, max(1, 16 // groups))
+        c = tokens(Q - start)
         q_rows = query[:, :, start:start + c].reshape(batch, Hq * c, head_dim)
         o32 = None if out_f32 is None else torch.empty(batch, Hq * c, head_dim, dtype=torch.float32,
                                                        device=query.device)

@@ -157,3 +157,44 @@ def test_page_runs_the_tile_kernel_takes(G, T, dtype, q_dtype, cfg):
     assert got.dtype == q_dtype and events[0].elapsed_time(events[1]) >= 0
     tiles = G == 16 or (q_dtype == dtype and "value_bits" not in cfg and cfg["bits"] < 8)
     assert _rel_err(out.unsqueeze(2), ref) <= (1e-5 if tiles else 2e-3)
+
+
+@pytest.mark.parametrize("G,Q,D,dtype,q_dtype,launches,cfg", [
+    (4, 4, 64, BF, BF, 1, dict(promote_ratio=0.25)),                 # no page run: sixteen rows in one launch
+    (3, 5, 128, FP, FP, 1, dict(key_group_size=64)),
+    (6, 3, 128, BF, BF, 2, dict(key_group_size=64, promote_ratio=0.25)),  # twelve rows, then six
+    (4, 3, 128, BF, BF, 1, dict(bits=4)),                            # page runs: rows the page kernels do not have
+    (2, 8, 128, FP, FP, 1, dict(bits=8)),
+    (1, 3, 128, BF, BF, 1, dict(promote_ratio=0.25)),
+    (16, 2, 128, BF, BF, 2, dict(bits=4)),
+    (4, 3, 128, BF, FP, 2, dict(promote_ratio=0.25)),                # pages only the page kernel takes: 8 + 4 rows
+    (4, 3, 128, BF, BF, 2, dict(bits=4, value_group_size=16)),
+    (4, 3, 128, FP, FP, 2, dict(bits=4, value_bits=2)),
+    (4, 3, 128, BF, BF, 2, dict(bits=4, value_local_tokens=70)),     # ... beside pages with a dense value window
+    (4, 4, 64, torch.float32, torch.float32, 1, dict(bits=4)),       # the general kernel
+])
+def test_query_tokens_share_launches(G, Q, D, dtype, q_dtype, launches, cfg, monkeypatch):
+    import dartkv_amd as dart
+    from dartkv_amd import attention, synthetic
+    from oracle import dart_oracle as O
+    cfg = dict(dict(bits=2, page_size=128, key_group_size=128, value_group_size=64, sink_tokens=32,
+                    hold_partial_pages=True, metadata_dtype=torch.float16), **cfg)
+    k, v, _ = synthetic.outlier_kv(2, 2, 700, D, query_heads=2, dtype=torch.float32, seed=G + Q)
+    q = torch.randn(2, Q, 2 * G, D, generator=torch.Generator().manual_seed(Q)).to(q_dtype).transpose(1, 2)
+    k, v = k.to(dtype), v.to(dtype)
+    oc, cache = O.OracleCache(O.OracleConfig(**cfg)), dart.DartKVCache(dart.DartKVCacheConfig(**cfg))
+    oc.append(k, v)
+    cache.append(k.to(DEV), v.to(DEV))
+    ref = O.streamed_attention(q, oc, return_fp32=True)[1]
+    print("case", G, Q, D, dtype, q_dtype, cfg, flush=True)
+    calls, decode = [], attention.decode_attention
+    monkeypatch.setattr(attention, "decode_attention", lambda *a, **kw: calls.append(0) or decode(*a, **kw))
+    plain = torch.empty(2, 2 * G, Q, D, dtype=torch.float32, device=DEV)
+    strided = torch.empty(2, Q, 2 * G, D, dtype=torch.float32, device=DEV).transpose(1, 2)
+    for out in (plain, strided):
+        got = attention._multi_token_attention(q.to(DEV), cache, out_f32=out)
+        torch.cuda.synchronize()
+        assert got.shape == out.shape and got.dtype == q_dtype and got.is_contiguous()
+        assert torch.equal(got.float(), out.to(q_dtype).float())
+        assert _rel_err(out, ref) <= (1e-5 if launches == 1 or G in (6, 16) else 2e-3)
+    assert len(calls) == 2 * launches
