@@ -304,6 +304,90 @@ __global__ void __launch_bounds__(kThreads) decode_merge(DecodeParams p) {
   }
 }
 
+// More records per query head: 1,024 threads, each summing every
+// n-th record of one channel, the first kMergeWideRegs of them loaded before
+// the weights are known; the weights are formed by all threads at once.  What
+// bounds it is one CU's chain of load rounds, so decode_merge's one pass over
+// the records by 128 threads grew with their number: for 8 query heads with
+// 256 records each 18 µs (the tile kernel before it 13), here 6.5; with 128
+// records 9.8 -> 5.3, with 64 6.2 -> 4.7.
+constexpr int kMergeWideThreads = 1024, kMergeWideRegs = 32, kMergeWideMaxSplits = 8192;
+
+__global__ void __launch_bounds__(kMergeWideThreads) decode_merge_wide(DecodeParams p) {
+  extern __shared__ float wsh[];  // [S] weights
+  __shared__ float part[kMergeWideThreads], wave_m[kMergeWideThreads / 64], wave_l[kMergeWideThreads / 64];
+  const int bq = blockIdx.x;  // b * Hq + hq
+  const dkv_decode_args& a = p.a;
+  const int S = p.split_stride, D = (int)a.D, tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int Dp = (D + 63) / 64 * 64, groups = kMergeWideThreads / Dp;
+  const int group = __builtin_amdgcn_readfirstlane(tid / Dp), c = tid - group * Dp;
+  const float* ws = (const float*)a.workspace + (int64_t)bq * S * (D + 2);
+  const bool sums = group < groups && c < D;
+  float r[kMergeWideRegs];
+  if (sums) {
+#pragma unroll
+    for (int i = 0; i < kMergeWideRegs; ++i) {
+      const int s = group + i * groups;
+      r[i] = s < S ? ws[(int64_t)s * (D + 2) + 2 + c] : 0.f;
+    }
+  }
+  float m = -INFINITY;
+  for (int s = tid; s < S; s += kMergeWideThreads) m = fmaxf(m, wsh[s] = ws[(int64_t)s * (D + 2)]);
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
+  if (lane == 0) wave_m[wave] = m;
+  __syncthreads();
+  float M = -INFINITY;
+#pragma unroll
+  for (int w = 0; w < kMergeWideThreads / 64; ++w) M = fmaxf(M, wave_m[w]);
+  float l = 0.f;
+  for (int s = tid; s < S; s += kMergeWideThreads) {
+    const float ms = wsh[s], w = ms == -INFINITY ? 0.f : expf(ms - M);
+    wsh[s] = w;
+    l += ws[(int64_t)s * (D + 2) + 1] * w;
+  }
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) l += __shfl_xor(l, off, 64);
+  if (lane == 0) wave_l[wave] = l;
+  __syncthreads();
+  if (sums) {
+    float o = 0.f;
+#pragma unroll
+    for (int i = 0; i < kMergeWideRegs; ++i)
+      if (group + i * groups < S) o += r[i] * wsh[group + i * groups];
+    for (int s = group + kMergeWideRegs * groups; s < S; s += groups) o += ws[(int64_t)s * (D + 2) + 2 + c] * wsh[s];
+    part[tid] = o;
+  }
+  __syncthreads();
+  if (tid < D) {
+    float o = 0.f, L = 0.f;
+    for (int g = 0; g < groups; ++g) o += part[g * Dp + tid];
+#pragma unroll
+    for (int w = 0; w < kMergeWideThreads / 64; ++w) L += wave_l[w];
+    o /= fmaxf(L, 1e-20f);
+    const int b = bq / (int)a.Hq, hq = bq % (int)a.Hq;
+    dev_store(a.out, (int64_t)b * a.out_sb + (int64_t)hq * a.out_sh + tid, o, (int)a.q_dtype);
+    if (a.out_f32) a.out_f32[(int64_t)bq * D + tid] = o;
+  }
+}
+
+// Merge p's records into the outputs.
+int launch_merge(const DecodeParams& p, hipStream_t s) {
+  const dkv_decode_args& a = p.a;
+  const int S = p.split_stride;
+  const dim3 grid((unsigned)(a.B * a.Hq));
+  // 24 to 32 records: 256 query heads 5.5 -> 4.5 µs; with 16 records or more
+  // heads than CUs (512 heads: 4.1 against 5.7) decode_merge is the faster
+  const bool wide = S > kMergeRegSplits || (S >= 24 && a.B * a.Hq <= 256);
+  if (wide && S <= kMergeWideMaxSplits && a.D <= kThreads) {
+    hipLaunchKernelGGL(decode_merge_wide, grid, dim3(kMergeWideThreads), (size_t)S * sizeof(float), s, p);
+  } else {
+    const int threads = (int)(a.D < 64 ? 64 : (a.D > kThreads ? kThreads : ((a.D + 63) / 64) * 64));
+    hipLaunchKernelGGL(decode_merge, grid, dim3(threads), (size_t)2 * S * sizeof(float), s, p);
+  }
+  return dkv_check_launch("dkv_decode_attention(merge)");
+}
+
 }  // namespace
 
 // Record a caller's timing event (if any) on the stream.
@@ -510,7 +594,6 @@ extern "C" int dkv_decode_attention(const dkv_decode_args* args, void* stream) {
     DKV_CHECK(a.D == kDenseDim && p.group <= max_group, DKV_ERR_UNSUPPORTED,
               "rest_dense_tokens needs head_dim %d and at most %d query heads per KV head", kDenseDim, max_group);
   }
-  const int merge_threads = (int)(a.D < 64 ? 64 : (a.D > kThreads ? kThreads : ((a.D + 63) / 64) * 64));
   bool run_done = false;
   if (fast_count > 0 && dkv::tiles_take_run(a, p.group)) {
     // The tile kernel takes the run: sixteen rows per KV head on Dart pages,
@@ -538,11 +621,7 @@ extern "C" int dkv_decode_attention(const dkv_decode_args* args, void* stream) {
     if (rc) return rc;
     rc = record_event(a.fast_events[1], s);
     if (rc) return rc;
-    if (all) {
-      hipLaunchKernelGGL(decode_merge, dim3((unsigned)(a.B * a.Hq)), dim3(merge_threads),
-                         (size_t)2 * splits * sizeof(float), s, t);
-      return dkv_check_launch("dkv_decode_attention(merge)");
-    }
+    if (all) return launch_merge(t, s);
     p.split_offset = splits;
     p.split_stride = t.split_stride;
     run_done = true;
@@ -572,10 +651,7 @@ extern "C" int dkv_decode_attention(const dkv_decode_args* args, void* stream) {
     if (rc) return rc;
     rc = record_event(a.fast_events[1], s);
     if (rc) return rc;
-    if (fuse) {
-      hipLaunchKernelGGL(decode_merge, dim3((unsigned)(a.B * a.Hq)), dim3(kThreads), 2 * stride * sizeof(float), s, p);
-      return dkv_check_launch("dkv_decode_attention(merge)");
-    }
+    if (fuse) return launch_merge(p, s);
   }
   if (dense_rest) {
     const int mg = p.group <= 1 ? 1 : p.group <= 2 ? 2 : p.group <= 4 ? 4 : 8;
@@ -626,7 +702,5 @@ extern "C" int dkv_decode_attention(const dkv_decode_args* args, void* stream) {
     rc = dkv_check_launch("dkv_decode_attention(split)");
     if (rc) return rc;
   }
-  hipLaunchKernelGGL(decode_merge, dim3((unsigned)(a.B * a.Hq)), dim3(merge_threads),
-                     (size_t)2 * p.split_stride * sizeof(float), s, p);
-  return dkv_check_launch("dkv_decode_attention(merge)");
+  return launch_merge(p, s);
 }

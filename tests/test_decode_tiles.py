@@ -198,3 +198,27 @@ def test_query_tokens_share_launches(G, Q, D, dtype, q_dtype, launches, cfg, mon
         assert torch.equal(got.float(), out.to(q_dtype).float())
         assert _rel_err(out, ref) <= (1e-5 if launches == 1 or G in (6, 16) else 2e-3)
     assert len(calls) == 2 * launches
+
+
+@pytest.mark.parametrize("D,pages,dtype", [
+    (128, 24, BF), (128, 33, BF), (64, 64, FP), (128, 300, BF),  # one record per page: the first, and past a thread's 32
+    (192, 40, torch.float32), (96, 30, BF), (256, 130, FP),      # thread groups that do not fill the workgroup
+])
+def test_merge_of_many_records(D, pages, dtype):
+    """One record per page, weights over many orders of magnitude and records of masked-out size."""
+    import dartkv_amd as dart
+    from oracle import dart_oracle as O
+    g = torch.Generator().manual_seed(pages + D)
+    T = 8 * pages
+    k, v, q = (torch.randn(1, 2, n, D, generator=g).to(dtype) for n in (T, T, 3))
+    k[:, :, : T // 2] *= 4.0
+    q = q.reshape(1, 6, 1, D)
+    cfg = dict(bits=4, page_size=8, key_group_size=8, value_group_size=32)
+    oc, cache = O.OracleCache(O.OracleConfig(**cfg)), dart.DartKVCache(dart.DartKVCacheConfig(**cfg))
+    oc.append(k, v)
+    cache.append(k.to(DEV), v.to(DEV))
+    ref = O.streamed_attention(q, oc, return_fp32=True)[1]
+    out = torch.empty(1, 6, D, dtype=torch.float32, device=DEV)
+    print("case", D, pages, dtype, flush=True)
+    dart.decode_attention(q.to(DEV), cache, out_f32=out, n_splits=pages)
+    assert _rel_err(out.unsqueeze(2), ref) <= 2e-5  # logits to about 100: 100 x 2^-24 relative in a weight
