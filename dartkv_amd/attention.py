@@ -287,7 +287,7 @@ def segment_attention(query: torch.Tensor, cache: DartKVCache, *, scale: Optiona
 
 
 def _fast_rows(plan) -> Tuple[int, ...]:
-    """Query rows per KV head the MFMA page kernels take: up to 16 on Dart pages, 8 on uniform pages."""
+    """Query rows per KV head of a page run's launch: 16 (tile kernel) on Dart pages beside the page kernels' up to 8."""
     return (1, 2, 4, 8, 16) if plan.fast_promoted else (1, 2, 4, 8)
 
 

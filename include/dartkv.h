@@ -276,10 +276,11 @@ typedef struct dkv_segment {
  * head_dim 128, Dart keys with fast_promoted promoted channels (a multiple of
  * 16, at most 64, one key group per page), 2-bit values in groups of
  * fast_value_group channels (a multiple of 16 dividing 128), fp16 metadata and a
- * bf16 or fp16 cache, every field 16-byte aligned, and Hq / Hkv of 1, 2, 4
- * or 8; the caller guarantees this (except the head ratio, which is checked).
- * Those pages are processed by the MFMA page kernel over `fast_splits` splits;
- * the other entries and the tail by the general kernel over `n_splits` splits.
+ * bf16 or fp16 cache, every field 16-byte aligned, and Hq / Hkv of 1, 2, 4,
+ * 8 or 16; the caller guarantees this (except the head ratio, which is checked).
+ * Those pages are processed by the MFMA page kernel (16 rows: the tile kernel)
+ * over `fast_splits` splits; the other entries and the tail by the tile or
+ * general kernel over `n_splits` splits.
  * With fast_promoted == 0 the run is instead uniform pages: keys quantized
  * with fast_key_bits bits along the tokens (one key group per page), values
  * with fast_value_bits bits along the channels in groups of fast_value_group
@@ -291,7 +292,7 @@ typedef struct dkv_segment {
  * outside the fast range and the tail are dense segments in the cache dtype
  * (bf16 or fp16) with 16-byte aligned rows and at most rest_dense_tokens
  * tokens each; then one wave per 32-token chunk handles them (head_dim 128, at
- * most 8 query heads per KV head, n_splits = number of those segments *
+ * most 8 query heads per KV head, 16 beside a Dart run, n_splits = number of those segments *
  * ceil(rest_dense_tokens / 32)).
  *
  * Checked guarantees: when segments_host is not NULL it holds the same
