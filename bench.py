@@ -646,7 +646,9 @@ def time_c5(args, bits: str, torch, dart, synthetic, stream) -> dict:
     ms_per_step = total_ms / args.steps
     gbs = nbytes * args.layers / (ms_per_step * 1e-3) / 1e9
     achieved = fast_bytes / (avg_kernel_ms * 1e-3) / 1e9 if avg_kernel_ms else None
-    kernel = "decode_pages_fast" if plan.fast_promoted else "decode_pages_uniform"
+    # (uniform runs that fill the device go to the tile kernel)
+    tiles = a.batch * a.kv_heads * plan.fast_count >= 2048
+    kernel = "decode_pages_fast" if plan.fast_promoted else "decode_tiles" if tiles else "decode_pages_uniform"
     tok_s = args.batch / (ms_per_step * 1e-3)
     multi = multi_token_leg(torch, dart, caches, a) if bits == "2b25" and not args.no_multi_token else None
     del caches, queries, step, events, plan
@@ -666,7 +668,7 @@ def time_c5(args, bits: str, torch, dart, synthetic, stream) -> dict:
             "bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4),
             "traffic": measured_traffic(kernel, "c5" if bits == "2b25" else f"c5_{bits}"),
-            "kernel": f"{kernel} (MFMA page kernel)",
+            "kernel": f"{kernel} (MFMA {'tile' if kernel == 'decode_tiles' else 'page'} kernel)",
             "algorithmic_bytes_per_launch": fast_bytes,
             "avg_kernel_us": round(avg_kernel_ms * 1e3, 2),
         },
@@ -676,7 +678,7 @@ def time_c5(args, bits: str, torch, dart, synthetic, stream) -> dict:
 
 def multi_token_leg(torch, dart, caches, a, steps: int = 3) -> dict:
     """Several query tokens per head over the resident C5 layer caches (fused_dart_attention with Q tokens:
-    each token one more query row of its KV group; the Dart page kernel takes 8 rows per KV head, so two
+    each token one more query row of its KV group; a launch takes 16 rows per KV head, so four
     tokens of a GQA-4 group share each page read), and one token of a GQA-8 query (8 query heads per KV
     head) over the same caches.  Microseconds per layer call (HIP events around `steps` passes over every
     layer after one untimed pass) and the ratio to one token."""
