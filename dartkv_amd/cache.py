@@ -578,11 +578,12 @@ class DartKVCache:
 
     def _materialize_all(self) -> Optional[Tuple[torch.Tensor, torch.Tensor]]:
         """The contents as dense tensors from one launch over the descriptor table (dkv_materialize), or None
-        where the segments are dequantized one by one: a cache on the host, Kitty value windows (the two
+        where the segments are dequantized one by one: a cache on the host, head_dims past 16,384 (the kernel's
+        channel table), Kitty value windows (the two
         tracks are not cut alike), and under capture a table that is not built yet (its upload cannot be
         captured)."""
         device, c = self._device, self.config
-        if device is None or device.type != "cuda" or c.value_local_tokens:
+        if device is None or device.type != "cuda" or c.value_local_tokens or self._shape[-1] > 16384:
             return None
         plan = self._decode_plan_cache
         ready = plan is not None and plan.version == self._sealed_version and plan.device == device
