@@ -222,3 +222,18 @@ def test_merge_of_many_records(D, pages, dtype):
     print("case", D, pages, dtype, flush=True)
     dart.decode_attention(q.to(DEV), cache, out_f32=out, n_splits=pages)
     assert _rel_err(out.unsqueeze(2), ref) <= 2e-5  # logits to about 100: 100 x 2^-24 relative in a weight
+
+
+@pytest.mark.parametrize("dtype,pad,skip", [(BF, 1, 0), (FP, 8, 4), (BF, 8, 0), (FP, 0, 1)])
+def test_query_alignment(dtype, pad, skip):
+    """Queries whose heads or base are off 16 bytes take the narrow loads, the same bits as a contiguous query."""
+    import dartkv_amd as dart
+    g = torch.Generator().manual_seed(3)
+    k, v = (torch.randn(2, 2, 300, 64, generator=g).to(dtype).to("cuda") for _ in range(2))
+    cache = dart.DartKVCache(dart.DartKVCacheConfig(promote_ratio=0.25, hold_partial_pages=True))
+    cache.append(k, v)
+    q = torch.randn(2, 6, 1, 64, generator=g).to(dtype).to("cuda")
+    flat = torch.zeros(skip + 2 * 6 * (64 + pad), dtype=dtype, device="cuda")
+    strided = flat[skip:].view(2, 6, 1, 64 + pad)[..., :64]
+    strided.copy_(q)
+    assert torch.equal(dart.decode_attention(strided, cache), dart.decode_attention(q, cache))
