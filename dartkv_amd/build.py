@@ -47,8 +47,8 @@ def command(output: str = LIB) -> list[str]:
 
 
 # Sources whose kernels must keep every value in registers: a spill to scratch
-# (private memory in HBM) would add memory traffic to the page kernels' loops.
-NO_SCRATCH = {"decode_fast.hip", "decode_uniform.hip"}
+# (private memory in HBM) would add memory traffic to the page and tile kernels' loops.
+NO_SCRATCH = {"decode_fast.hip", "decode_uniform.hip", "decode_tiles.hip"}
 
 
 def _run(cmd: list[str], verbose: bool) -> str:

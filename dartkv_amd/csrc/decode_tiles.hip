@@ -17,7 +17,7 @@
 // whose registers a larger tile would not leave room for).
 //
 // Bound by VALU issue and by the latency between a tile's steps at two waves
-// per SIMD (200-255 VGPRs), not by memory.  Against decode_split_general, which
+// per SIMD (140 to 256 VGPRs, no private memory: the build checks it), not by memory.  Against decode_split_general, which
 // spent about 100 VALU per element on scalar index arithmetic (one layer,
 // MI355X): 8 sequences x 4,096 tokens, 2-bit pages in groups of 64, fp16: 572
 // -> 19.8 µs; 8 x 8,011 tokens of Dart pages, six heads per KV head: 1,453 ->
@@ -169,6 +169,17 @@ struct Codes {
   static constexpr int kSpan = kShared ? 2 * NP : NP;             // positions of one load
 };
 
+// No value: a register that only one branch of a loop body loads would otherwise
+// hold its old contents through the whole body (at sixteen rows the kernel
+// spilled up to eight registers).
+template <class T>
+__device__ __forceinline__ void forget(T& x) { asm volatile("" : "=v"(x)); }
+template <class T, int N>
+__device__ __forceinline__ void forget(T (&x)[N]) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) forget(x[i]);
+}
+
 // Codes of K indices 0 .. NK - 1 of the lane into regs: index k's are at
 // base(k) (wave-uniform) + off(k) bytes; a shared load asks for the pair's
 // first index, and off adds the odd lane's step.
@@ -213,16 +224,20 @@ __device__ __forceinline__ uint32_t unshare(uint32_t x, uint32_t sel) { return p
 template <int NP>
 __device__ __forceinline__ uint32_t two_bit_bytes(uint32_t y) { return NP == 8 ? y : perm(y >> 4, y, 0x05040100u); }
 
-// Operand dwords of a pair of K indices at every position j, from 2-bit codes.
+// Operand dword w (a pair of K indices) at every position j, from 2-bit codes.
+// (The dwords of an operand are one vector from the start: gathered from an
+// array per pair, they went through private memory at head_dim 64 with up to
+// four heads per KV head; 16 x 16,384 tokens, 2-bit pages in groups of 64: 66.0
+// -> 44.0 µs.)
 template <int NP>
 __device__ __forceinline__ void lookup_pair(uint32_t y, uint32_t lo0, uint32_t hi0, uint32_t lo1, uint32_t hi1,
-                                            uint32_t m3, uint32_t sel2, uint32_t (&op)[NP]) {
+                                            uint32_t m3, uint32_t sel2, u32x4 (&op)[NP], int w) {
 #pragma unroll
   for (int j = 0; j < NP / 2; ++j) {
     const uint32_t e = ((y >> (2 * j)) & m3) | sel2;
     const uint32_t l = perm(lo1, lo0, e), h = perm(hi1, hi0, e);
-    op[j] = perm(h, l, 0x05010400u);
-    op[j + NP / 2] = perm(h, l, 0x07030602u);
+    op[j][w] = perm(h, l, 0x05010400u);
+    op[j + NP / 2][w] = perm(h, l, 0x07030602u);
   }
 }
 
@@ -239,7 +254,7 @@ __device__ __forceinline__ half2v codes16(uint32_t e) {
 // indices' scales and zero points, sel is the unshare selector.
 template <bool BF, int BITS, int NP>
 __device__ __forceinline__ void chain_pair(const uint32_t* codes, uint32_t s, uint32_t z, uint32_t sel,
-                                           uint32_t (&op)[NP]) {
+                                           u32x4 (&op)[NP], int w) {
   const half2v sv = __builtin_bit_cast(half2v, s), zv = __builtin_bit_cast(half2v, z);
   auto value = [&](half2v c) {
     const half2v prod = c * sv;  // -ffp-contract=off: one rounding each
@@ -250,10 +265,10 @@ __device__ __forceinline__ void chain_pair(const uint32_t* codes, uint32_t s, ui
     for (int q = 0; q < NP / 4; ++q) {  // four positions: bytes (k0, k1, k0, k1), two positions per byte
       const uint32_t y = NP == 8 ? perm(codes[1], codes[0], q ? 0x07030602u : 0x05010400u) : unshare(codes[0], sel);
       const uint32_t even = y & 0x0f0f0f0fu, odd = (y >> 4) & 0x0f0f0f0fu;
-      op[4 * q] = value(codes16<false>(even));
-      op[4 * q + 1] = value(codes16<false>(odd));
-      op[4 * q + 2] = value(codes16<true>(even));
-      op[4 * q + 3] = value(codes16<true>(odd));
+      op[4 * q][w] = value(codes16<false>(even));
+      op[4 * q + 1][w] = value(codes16<false>(odd));
+      op[4 * q + 2][w] = value(codes16<true>(even));
+      op[4 * q + 3][w] = value(codes16<true>(odd));
     }
   } else {
     static_assert(BITS == 8, "2-bit codes take the tables");
@@ -265,7 +280,7 @@ __device__ __forceinline__ void chain_pair(const uint32_t* codes, uint32_t s, ui
         // bytes (a_j, 0x64, b_j, 0x64): 1024 + code in fp16
         const uint32_t y = perm(b, a, j == 0 ? 0x0c040c00u : j == 1 ? 0x0c050c01u : j == 2 ? 0x0c060c02u : 0x0c070c03u);
         const half2v c = __builtin_bit_cast(half2v, y | 0x64006400u) - half2v{1024.0f16, 1024.0f16};
-        op[4 * q + j] = value(c);
+        op[4 * q + j][w] = value(c);
       }
     }
   }
@@ -341,26 +356,26 @@ struct TileState {
     return *(const u32x4*)((const uint16_t*)q + (part * GP + n % GP) * D + 32 * kb + 8 * kq);
   }
 
-  __device__ __forceinline__ void q_products(int kb, const uint32_t (&op)[4][NJ], float4v (&S)[NJ]) const {
+  __device__ __forceinline__ void q_products(int kb, const u32x4 (&op)[NJ], float4v (&S)[NJ]) const {
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) S[j] = mfma<BF>(qa[kb], u32x4{op[0][j], op[1][j], op[2][j], op[3][j]}, S[j]);
+    for (int j = 0; j < NJ; ++j) S[j] = mfma<BF>(qa[kb], op[j], S[j]);
     if constexpr (PARTS) {
 #pragma unroll
       for (int part = 1; part < 3; ++part) {
         const u32x4 a = q_part(part, kb);
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) S[j] = mfma<BF>(a, u32x4{op[0][j], op[1][j], op[2][j], op[3][j]}, S[j]);
+        for (int j = 0; j < NJ; ++j) S[j] = mfma<BF>(a, op[j], S[j]);
       }
     }
   }
 
   // Row 16 pass + r of the weights = part (16 pass + r) / GP of head r % GP.
-  __device__ __forceinline__ void p_products(int kb, const uint32_t (&op)[4][NC]) {
+  __device__ __forceinline__ void p_products(int kb, const u32x4 (&op)[NC]) {
 #pragma unroll
     for (int pass = 0; pass < PASSES; ++pass) {
       const u32x4 w = *(const u32x4*)(pw + (16 * pass + n) * kPRow + 64 * kb + 16 * kq);
 #pragma unroll
-      for (int j = 0; j < NC; ++j) O[j] = mfma<BF>(w, u32x4{op[0][j], op[1][j], op[2][j], op[3][j]}, O[j]);
+      for (int j = 0; j < NC; ++j) O[j] = mfma<BF>(w, op[j], O[j]);
     }
   }
 
@@ -621,6 +636,8 @@ __global__ void __launch_bounds__(64 * kTileWaves, 2) decode_tiles(TileParams p)
       const int g0 = t0 / kgroup, ng = min(Gp - g0, max(1, TILE / kgroup));
 #pragma unroll
       for (int m = 0; m < KIT; ++m) {
+        forget(ks[m]);
+        forget(kz[m]);
         if (m / KSTEP < ng) {
           const int step = 64 * (m % KSTEP) * Gp + g0 + m / KSTEP;
           ks[m] = gload<uint16_t>(t.ks + step, mul24(2 * lane, Gp));
@@ -643,6 +660,8 @@ __global__ void __launch_bounds__(64 * kTileWaves, 2) decode_tiles(TileParams p)
             vc, [&](int k) { return t.v + (t0 + 32 * (k >> 3) + (k & 7)) * vrow; }, [&](int) { return off; });
 #pragma unroll
         for (int m = 0; m < VIT; ++m) {
+          forget(vs[m]);
+          forget(vz[m]);
           if (m / VSTEP < Gv) {
             const int item = (t0 + 64 * (m % VSTEP)) * Gv + m / VSTEP;
             vs[m] = gload<uint16_t>(t.vs + item, mul24(2 * lane, Gv));
@@ -655,6 +674,8 @@ __global__ void __launch_bounds__(64 * kTileWaves, 2) decode_tiles(TileParams p)
             [&](int k) { return col + mul24(min(t0 + 32 * (k >> 3) + 8 * kq + (k & 7) + step, last), vrow); });
 #pragma unroll
         for (int m = 0; m < VIT; ++m) {
+          forget(vs[m]);
+          forget(vz[m]);
           if (m / VSTEP < Gv) {
             const uint32_t item = 2 * (mul24(min(t0 + lane + 64 * (m % VSTEP), last), Gv) + m / VSTEP);
             vs[m] = gload<uint16_t>(t.vs, item);
@@ -662,6 +683,18 @@ __global__ void __launch_bounds__(64 * kTileWaves, 2) decode_tiles(TileParams p)
           }
         }
       }
+    };
+    auto no_keys = [&] {
+      forget(kc);
+      forget(ks);
+      forget(kz);
+      forget(kidx);
+      forget(zidx);
+    };
+    auto no_values = [&] {
+      forget(vc);
+      forget(vs);
+      forget(vz);
     };
     const uint8_t* vtab = lds + p.vt + (NC * n / vgroup) * kTabV;
 
@@ -735,17 +768,17 @@ __global__ void __launch_bounds__(64 * kTileWaves, 2) decode_tiles(TileParams p)
       const uint8_t* ktab = lds + p.kt + lane_group * kTabK;
 #pragma unroll
       for (int kb = 0; kb < KB; ++kb) {
-        uint32_t op[4][NJ];
+        u32x4 op[NJ];
         const uint4* tab = (const uint4*)(ktab + (KBITS == 2 ? 8 : 4) * (32 * kb + 8 * kq));
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
           if constexpr (KBITS == 2) {
             const uint4 tt = tab[w];
-            lookup_pair<NJ>(two_bit_bytes<NJ>(unshare(kc[4 * kb + w], ksel)), tt.x, tt.y, tt.z, tt.w, m3, sel2, op[w]);
+            lookup_pair<NJ>(two_bit_bytes<NJ>(unshare(kc[4 * kb + w], ksel)), tt.x, tt.y, tt.z, tt.w, m3, sel2, op, w);
           } else {
             const uint4 tt = tab[w / 2];
             chain_pair<BF, KBITS, NJ>(&kc[KC::kPairRegs * (4 * kb + w)], w % 2 ? tt.z : tt.x, w % 2 ? tt.w : tt.y, ksel,
-                                      op[w]);
+                                      op, w);
           }
         }
         st.q_products(kb, op, S);
@@ -761,7 +794,7 @@ __global__ void __launch_bounds__(64 * kTileWaves, 2) decode_tiles(TileParams p)
           }
           // slots past the last one: zero query, zero scale and zero point
           const bool whole = 32 * block + 32 <= promoted;
-          uint32_t op[4][NJ];
+          u32x4 op[NJ];
           u32x4 qp[PARTS ? 3 : 1];
           const uint32_t* sz = (const uint32_t*)(lds + p.sz) + lane_group * D;
 #pragma unroll
@@ -788,17 +821,18 @@ __global__ void __launch_bounds__(64 * kTileWaves, 2) decode_tiles(TileParams p)
             for (int j = 0; j < NJ / 2; ++j) {
               const uint32_t e = ((j & 1 ? oddn : even) >> (4 * (j >> 1))) & 0x0f0f0f0fu;
               const half2v x = codes16<false>(e) * s, y = codes16<true>(e) * s;
-              op[w][j] = to_operand<BF>(x + z);
-              op[w][j + NJ / 2] = to_operand<BF>(y + z);
+              op[j][w] = to_operand<BF>(x + z);
+              op[j + NJ / 2][w] = to_operand<BF>(y + z);
             }
           }
 #pragma unroll
           for (int part = 0; part < (PARTS ? 3 : 1); ++part) {
 #pragma unroll
-            for (int j = 0; j < NJ; ++j) S[j] = mfma<BF>(qp[part], u32x4{op[0][j], op[1][j], op[2][j], op[3][j]}, S[j]);
+            for (int j = 0; j < NJ; ++j) S[j] = mfma<BF>(qp[part], op[j], S[j]);
           }
         }
       }
+      no_keys();
       if (live) load_keys(nxt, t0);
       lds_order();
       st.softmax(S, nt);
@@ -821,21 +855,22 @@ __global__ void __launch_bounds__(64 * kTileWaves, 2) decode_tiles(TileParams p)
       // ---- O += P V ----
 #pragma unroll
       for (int kb = 0; kb < VB; ++kb) {
-        uint32_t op[4][NC];
+        u32x4 op[NC];
         const uint4* tab = (const uint4*)(vtab + (VBITS == 2 ? 8 : 4) * (32 * kb + 8 * kq));
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
           if constexpr (VBITS == 2) {
             const uint4 tt = tab[w];
-            lookup_pair<NC>(two_bit_bytes<NC>(unshare(vc[4 * kb + w], vsel)), tt.x, tt.y, tt.z, tt.w, m3, sel2, op[w]);
+            lookup_pair<NC>(two_bit_bytes<NC>(unshare(vc[4 * kb + w], vsel)), tt.x, tt.y, tt.z, tt.w, m3, sel2, op, w);
           } else {
             const uint4 tt = tab[w / 2];
             chain_pair<BF, VBITS, NC>(&vc[VC::kPairRegs * (4 * kb + w)], w % 2 ? tt.z : tt.x, w % 2 ? tt.w : tt.y, vsel,
-                                      op[w]);
+                                      op, w);
           }
         }
         st.p_products(kb, op);
       }
+      no_values();
       if (live) load_values(nxt, t0);
       lds_order();
     }
