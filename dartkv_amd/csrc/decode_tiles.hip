@@ -41,11 +41,14 @@
 // their slots, 32 to a block.
 //
 // Arithmetic.  K and V hold the reference's dequantized values exactly (its
-// rounding chain), the query is exact in the operand type, and the softmax
-// weights stay fp32: a weight is the exact sum of three 16-bit parts (8 + 8 +
-// 8 bits for bf16; 11 + 11 + 2 for fp16), the parts of 4 heads take 12 of the
-// 16 rows of one MFMA (those of 8 heads two MFMAs, of 16 heads three), and their
-// products meet in the fp32 accumulators when the split ends.
+// rounding chain), the query is exact in the operand type, and a softmax weight
+// is the sum of three 16-bit parts: exact for bf16 (8 + 8 + 8 bits); for fp16
+// (11 + 11 + 2 bits, whose smallest step is fixed) within three steps of 2^-37
+// of the running maximum's weight, 2e-7 of the result over 8,192 tokens of one
+// split in the worst case, under the rounding of fp32 sums.  The parts of 4
+// heads take 12 of the 16 rows of one MFMA (those of 8 heads two MFMAs, of 16
+// heads three), and their products meet in the fp32 accumulators when the split
+// ends.
 #include <hip/hip_runtime.h>
 #include <math.h>
 
@@ -66,7 +69,13 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kTileWaves = 4;
 constexpr int kMaxGroups = 4;       // key groups per tile, value groups per token
-constexpr float kTileSlack = 5.5f;  // natural-log headroom before the running max moves (e^5.5 = 245)
+// Natural-log headroom of a weight before the running maximum moves, and the
+// power of two weights are scaled by.  fp16's range sets how small a part can
+// be: e^2.07 x 2^13 = 64,900 of 65,504.  (With 5.5 and 2^7, steps of 2^-31, the
+// error reached 1.7e-5 over 8,192 tokens of one split; with 0.68 and 2^15 the
+// maximum moved in most tiles: 1 to 2 % more time.)
+template <bool BF> constexpr float kTileSlack = BF ? 5.5f : 2.07f;
+template <bool BF> constexpr int kWeightExp = BF ? 0 : 13;
 
 struct TileParams {
   // This kernel's segments are numbered packed first: index i < n_packed is
@@ -211,6 +220,19 @@ __device__ __forceinline__ uint32_t swap_pair(uint32_t x) {
   return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0xb1, 0xf, 0xf, true);  // quad_perm 1, 0, 3, 2
 }
 
+// Maximum over the 16 lanes of a row.
+template <int CTRL>
+__device__ __forceinline__ float dpp_max(float x) {
+  const int y = __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true);
+  return fmaxf(x, __builtin_bit_cast(float, y));
+}
+__device__ __forceinline__ float max16(float x) {
+  x = dpp_max<0xb1>(x);   // lanes 1, 0, 3, 2 of each four
+  x = dpp_max<0x4e>(x);   // lanes 2, 3, 0, 1
+  x = dpp_max<0x141>(x);  // the other four of eight (row_half_mirror)
+  return dpp_max<0x140>(x);  // the other eight (row_mirror)
+}
+
 // Selector of unshare() for this lane: its own positions of (k0, k1) as bytes
 // (k0, k1, k0, k1), or (k0, k1, 0, 0) where a lane has one byte of each.
 template <int BYTES>
@@ -320,7 +342,7 @@ __device__ __forceinline__ uint32_t take_part(float x0, float x1, float& r0, flo
 // A pair of weight parts, none of them zero: an infinite value times a zero
 // part would be NaN where the weight itself is not zero (a zero weight keeps its
 // zero first part).  The smallest step, 2^-126 (bf16) or 2^-24 of weights
-// scaled by 2^7 (fp16), is below what the sums resolve.
+// scaled by 2^13 (fp16), is below what the sums resolve.
 template <bool BF>
 __device__ __forceinline__ uint32_t at_least_tiny(uint32_t x) {
   typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
@@ -370,13 +392,25 @@ struct TileState {
   }
 
   // Row 16 pass + r of the weights = part (16 pass + r) / GP of head r % GP.
-  __device__ __forceinline__ void p_products(int kb, const u32x4 (&op)[NC]) {
+  // A tile's products meet in T, which the logits no longer need, and are added
+  // to O once: straight into an O that a few tokens dominate, the small parts of
+  // the others' weights were rounded away (one dominant token, 8,191 of 2^-20 to
+  // 2^-29 of its weight in one split: error against 64 bits 2.8e-5).
+  __device__ __forceinline__ void p_products(int kb, const u32x4 (&op)[NC], float4v (&T)[NC]) {
 #pragma unroll
     for (int pass = 0; pass < PASSES; ++pass) {
       const u32x4 w = *(const u32x4*)(pw + (16 * pass + n) * kPRow + 64 * kb + 16 * kq);
 #pragma unroll
-      for (int j = 0; j < NC; ++j) O[j] = mfma<BF>(w, op[j], O[j]);
+      for (int j = 0; j < NC; ++j) T[j] = mfma<BF>(w, op[j], T[j]);
     }
+  }
+  __device__ __forceinline__ static void clear(float4v (&T)[NC]) {
+#pragma unroll
+    for (int j = 0; j < NC; ++j) T[j] = float4v{0.f, 0.f, 0.f, 0.f};
+  }
+  __device__ __forceinline__ void add_tile(const float4v (&T)[NC]) {
+#pragma unroll
+    for (int j = 0; j < NC; ++j) O[j] += T[j];
   }
 
   // Logits to weights in LDS, nt tokens of the tile valid.  A lane takes its
@@ -402,7 +436,7 @@ struct TileState {
         v *= scale;
         if (nt < TILE) v = NJ * n + start + u < nt ? v : -INFINITY;
         x[u][i] = v;
-        over |= v > m_run[i] + kTileSlack;
+        over |= v > m_run[i] + kTileSlack<BF>;
       }
     }
     if (__ballot(over) != 0ull) {
@@ -411,8 +445,7 @@ struct TileState {
         float mx = x[0][i];
 #pragma unroll
         for (int u = 1; u < U; ++u) mx = fmaxf(mx, x[u][i]);
-#pragma unroll
-        for (int off = 1; off < 16; off <<= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+        mx = max16(mx);
         if (GP == 4) mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
         if (GP <= 8) mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
         const float m_new = fmaxf(m_run[i], mx);
@@ -423,18 +456,21 @@ struct TileState {
         for (int j = 0; j < NC; ++j) O[j][i] *= alpha;
       }
     }
-    // weights (fp16 operands: times 2^7, undone in the record) and their parts;
+    // weights (fp16 operands: times 2^13, undone in the record) and their parts;
     // with 8 heads the last part takes two rows, half of it each
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int head = GP == 4 ? i : GP == 8 ? 4 * (kq & 1) + i : 4 * kq + i;
-      float w[U];
+      float w[U], sum = 0.f;  // (added to l once per tile, as O is)
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const float dlt = x[u][i] - m_run[i];
-        w[u] = __builtin_amdgcn_exp2f(BF ? dlt * kLog2e : __builtin_fmaf(dlt, kLog2e, 7.f));
-        l_part[i] += w[u];
+        w[u] = __builtin_amdgcn_exp2f(BF ? dlt * kLog2e : __builtin_fmaf(dlt, kLog2e, (float)kWeightExp<BF>));
+        sum += w[u];
+        // a weight below fp16's smallest step, but not zero, gets one (at_least_tiny)
+        if (!BF) w[u] = w[u] > 0.f ? fmaxf(w[u], 0x1p-24f) : w[u];
       }
+      l_part[i] += sum;
 #pragma unroll
       for (int k = 0; k < 3; ++k) {
         uint32_t part[U > 1 ? U / 2 : 1];
@@ -480,6 +516,8 @@ struct TileState {
     }
     softmax(S, nt);
     lds_order();
+    float4v T[NC];
+    clear(T);
 #pragma unroll 1
     for (int kb = 0; kb < VB; ++kb) {
       if (32 * kb >= nt) break;  // the weights of later tokens are zero
@@ -498,11 +536,12 @@ struct TileState {
 #pragma unroll
         for (int j = 0; j < NC; ++j) {
           const uint32_t sel = j % 2 ? 0x07060302u : 0x05040100u;
-          O[j] = mfma<BF>(w, u32x4{perm(r[1][j / 2], r[0][j / 2], sel), perm(r[3][j / 2], r[2][j / 2], sel),
-                                   perm(r[5][j / 2], r[4][j / 2], sel), perm(r[7][j / 2], r[6][j / 2], sel)}, O[j]);
+          T[j] = mfma<BF>(w, u32x4{perm(r[1][j / 2], r[0][j / 2], sel), perm(r[3][j / 2], r[2][j / 2], sel),
+                                   perm(r[5][j / 2], r[4][j / 2], sel), perm(r[7][j / 2], r[6][j / 2], sel)}, T[j]);
         }
       }
     }
+    add_tile(T);
     lds_order();
   }
 };
@@ -519,14 +558,18 @@ __global__ void __launch_bounds__(64 * kTileWaves, 2) decode_tiles(TileParams p)
   constexpr int KSTEP = D / 64, VSTEP = TILE / 64;       // table items of a lane per group
   constexpr int KIT = 2 * KSTEP, VIT = 2 * VSTEP;        // ... that wait in registers: two groups' (the others
                                                          // are loaded when their tables are made)
+  // Forms whose registers are full form the lane's coordinates anew for each
+  // tile: the addresses made from them would otherwise be kept from tile to tile
+  // and spilled (elsewhere this costs 2 %).
+  constexpr bool kRederive = D == 128 && ((GP == 16 && (MIXED || KBITS == 4)) || (GP == 8 && MIXED && !BF));
   constexpr int kTabK = D * 8 + 16, kTabV = TILE * 8 + 16;
   typedef Codes<KBITS, NJ> KC;
   typedef Codes<VBITS, NC> VC;
   const DecodeParams& d = p.d;
   const dkv_decode_args& a = d.a;
-  const int lane = threadIdx.x & 63;
+  int lane = threadIdx.x & 63;
   const int wave = uni(threadIdx.x >> 6);
-  const int n = lane & 15, kq = lane >> 4;
+  int n = lane & 15, kq = lane >> 4;
   const int worker = (int)blockIdx.x * kTileWaves + wave;
   const int Hkv = (int)a.Hkv, G = d.group;
   if (worker >= (int)a.B * Hkv * p.splits) return;
@@ -538,7 +581,7 @@ __global__ void __launch_bounds__(64 * kTileWaves, 2) decode_tiles(TileParams p)
   const int s1 = uni((int)(((int64_t)(split + 1) * d.n_total) / p.splits));
   const uint32_t m3 = in_sgpr(0x03030303u), sel2 = in_vgpr(0x04000400u);
   const uint32_t ksel = unshare_sel<KC::kBytes>(lane), vsel = unshare_sel<VC::kBytes>(lane);
-  const int odd = lane & 1;
+  int odd = lane & 1;
   const int kgroup = p.key_group, vgroup = p.value_group, promoted = p.promoted;
   const int Gv = groups_of(D, vgroup), vrow = Gv * vgroup * VBITS / 8;
 
@@ -709,6 +752,12 @@ __global__ void __launch_bounds__(64 * kTileWaves, 2) decode_tiles(TileParams p)
     }
 #pragma unroll 1
     while (live) {
+      if constexpr (kRederive) {
+        asm volatile("" : "+v"(lane));
+        n = st.n = lane & 15;
+        kq = st.kq = lane >> 4;
+        odd = lane & 1;
+      }
       const Packed cur = nxt;
       const int cur0 = t0, nt = min(TILE, cur.tokens - t0);
       t0 += TILE;
@@ -853,6 +902,8 @@ __global__ void __launch_bounds__(64 * kTileWaves, 2) decode_tiles(TileParams p)
       lds_order();
 
       // ---- O += P V ----
+      float4v T[NC];
+      St::clear(T);
 #pragma unroll
       for (int kb = 0; kb < VB; ++kb) {
         u32x4 op[NC];
@@ -868,8 +919,9 @@ __global__ void __launch_bounds__(64 * kTileWaves, 2) decode_tiles(TileParams p)
                                       op, w);
           }
         }
-        st.p_products(kb, op);
+        st.p_products(kb, op, T);
       }
+      st.add_tile(T);
       no_values();
       if (live) load_values(nxt, t0);
       lds_order();
@@ -910,7 +962,7 @@ __global__ void __launch_bounds__(64 * kTileWaves, 2) decode_tiles(TileParams p)
   }
 
   // ---- partial state ----
-  constexpr float unscale = BF ? 1.f : 0.0078125f;
+  constexpr float unscale = 1.f / (1 << kWeightExp<BF>);
   float* ws = (float*)a.workspace;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {

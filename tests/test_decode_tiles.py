@@ -237,3 +237,52 @@ def test_query_alignment(dtype, pad, skip):
     strided = flat[skip:].view(2, 6, 1, 64 + pad)[..., :64]
     strided.copy_(q)
     assert torch.equal(dart.decode_attention(strided, cache), dart.decode_attention(q, cache))
+
+
+def _peaked(G, D, T, dtype, gap):
+    """A cache whose first token holds almost all of the softmax weight of every query head, and a query: the other
+    tokens' logits lie ``gap`` to ``gap`` + 6 below.  Values are positive."""
+    import dartkv_amd as dart
+    g = torch.Generator().manual_seed(T + G)
+    k = 0.1 * torch.randn(1, 2, T, D, generator=g)
+    k[..., 0] = -torch.randint(0, 2, (T,), generator=g).float()  # two values: the codes keep them
+    k[:, :, 0, 0] = gap / 6.0
+    v = 0.5 + torch.rand(1, 2, T, D, generator=g)
+    q = 0.1 * torch.randn(1, 2 * G, 1, D, generator=g)
+    q[..., 0] = 6.0
+    cache = dart.DartKVCache(dart.DartKVCacheConfig(bits=2, page_size=128, key_group_size=64, value_group_size=32,
+                                                    hold_partial_pages=True))
+    return cache, k.to(dtype), v.to(dtype), q.to(dtype)
+
+
+@pytest.mark.parametrize("gap", [14.0, 18.0, 24.0])  # weights of 2^-20 to 2^-43
+@pytest.mark.parametrize("G,D,dtype", [(3, 64, FP), (7, 128, FP), (12, 64, FP), (16, 128, FP), (3, 64, BF), (12, 128, BF)])
+def test_small_weights_keep_their_bits(G, D, dtype, gap):
+    """8,191 negligible tokens in one split against 64 bits.  The split's 64 tiles are added to the result and to the sum
+    of the weights one by one, 2^-24 relative each at most: 128 x 2^-24 = 7.6e-6; fp16 weights add 2e-7, and fp32
+    logits 30 x 2^-24 of the 2^-7 that the negligible tokens hold."""
+    import dartkv_amd as dart
+    cache, k, v, q = _peaked(G, D, 8192, dtype, gap)
+    cache.append(k.to(DEV), v.to(DEV))
+    dk, dv = (t.cpu().double() for t in cache.get())
+    logits = torch.matmul(q.double().view(1, 2, G, D), dk.transpose(-1, -2))
+    ref = torch.matmul(torch.softmax(logits, -1), dv).view(1, 2 * G, 1, D)
+    out = torch.empty(1, 2 * G, D, dtype=torch.float32, device=DEV)
+    print("case", G, D, dtype, gap, flush=True)
+    dart.decode_attention(q.to(DEV), cache, scale=1.0, out_f32=out, fast=False, n_splits=1)
+    got = out.cpu().double().view(1, 2 * G, 1, D)
+    assert float(((got - ref).abs() / ref.abs()).max()) <= 7.8e-6
+
+
+@pytest.mark.parametrize("G,dtype", [(3, FP), (7, FP), (12, FP), (3, BF), (7, BF), (12, BF)])
+def test_infinite_value_of_a_small_weight(G, dtype):
+    """A held token with a weight of about 2^-50 and an infinite value gives an infinity, as fp32 weights do."""
+    import dartkv_amd as dart
+    cache, k, v, q = _peaked(G, 64, 300, dtype, 32.0)
+    v[0, 1, 299, 5] = float("inf")
+    cache.append(k.to(DEV), v.to(DEV))
+    print("case", G, dtype, flush=True)
+    out = dart.decode_attention(q.to(DEV), cache, scale=1.0, fast=False, n_splits=1).cpu()
+    expected = torch.zeros(1, 2 * G, 1, 64, dtype=torch.bool)
+    expected[0, G:, 0, 5] = True
+    assert torch.equal(torch.isinf(out), expected) and not torch.isnan(out).any()
