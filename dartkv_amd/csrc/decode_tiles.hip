@@ -344,11 +344,13 @@ __device__ __forceinline__ uint32_t take_part(float x0, float x1, float& r0, flo
 // zero first part).  The smallest step, 2^-126 (bf16) or 2^-24 of weights
 // scaled by 2^13 (fp16), is below what the sums resolve.
 template <bool BF>
-__device__ __forceinline__ uint32_t at_least_tiny(uint32_t x) {
+constexpr __device__ uint32_t tiny_part() { return BF ? 0x0080u : 0x0001u; }
+__device__ __forceinline__ uint32_t at_least(uint32_t x, uint32_t least) {
   typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
-  const uint16_t tiny = BF ? 0x0080 : 0x0001;
-  return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, x), u16x2{tiny, tiny}));
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, x), __builtin_bit_cast(u16x2, least)));
 }
+template <bool BF>
+__device__ __forceinline__ uint32_t at_least_tiny(uint32_t x) { return at_least(x, tiny_part<BF>() * 0x10001u); }
 
 // The softmax state and accumulators of a wave, and the steps both kinds of
 // tile share.  GP: query rows per KV head rounded up to 4, 8 or 16.  S[j] row 4
@@ -634,6 +636,15 @@ __global__ void __launch_bounds__(64 * kTileWaves, 2) decode_tiles(TileParams p)
       st.scale = ldexpf(st.scale, e);
 #pragma unroll
       for (int i = 0; i < 8 * KB; ++i) x[i] = ldexpf(x[i], -e);
+      // a part that is zero where the element is not gets the smallest step and
+      // the element's sign: an infinite key times a zero part would be NaN
+      uint32_t sign[4 * KB], least[4 * KB];
+#pragma unroll
+      for (int i = 0; i < 4 * KB; ++i) {
+        const uint32_t b0 = __builtin_bit_cast(uint32_t, x[2 * i]), b1 = __builtin_bit_cast(uint32_t, x[2 * i + 1]);
+        sign[i] = perm(b1, b0, 0x07060302u) & 0x80008000u;
+        least[i] = (x[2 * i] != 0.f ? tiny_part<BF>() : 0u) | (x[2 * i + 1] != 0.f ? tiny_part<BF>() << 16 : 0u);
+      }
 #pragma unroll
       for (int part = 0; part < 3; ++part) {
 #pragma unroll
@@ -646,6 +657,7 @@ __global__ void __launch_bounds__(64 * kTileWaves, 2) decode_tiles(TileParams p)
             row[w] = take_part<BF>(x0, x1, r0, r1);
             x0 = r0;
             x1 = r1;
+            row[w] = sign[4 * kb + w] | at_least(row[w] & 0x7fff7fffu, least[4 * kb + w]);
           }
           if (part == 0) st.qa[kb] = row;
           if (n < GP) *(u32x4*)(lds + p.q + 2 * ((part * GP + n) * D + 32 * kb + 8 * kq)) = row;

@@ -286,3 +286,26 @@ def test_infinite_value_of_a_small_weight(G, dtype):
     expected = torch.zeros(1, 2 * G, 1, 64, dtype=torch.bool)
     expected[0, G:, 0, 5] = True
     assert torch.equal(torch.isinf(out), expected) and not torch.isnan(out).any()
+
+
+@pytest.mark.parametrize("dtype,q_dtype", [(BF, torch.float32), (FP, torch.float32), (BF, FP)])
+def test_infinite_key_under_a_query_of_another_type(dtype, q_dtype):
+    """Sixteen rows on Dart pages, a held token with an infinite key channel whose query elements are short and
+    negative: its logit is minus infinity, its weight zero, and nothing is NaN."""
+    import dartkv_amd as dart
+    g = torch.Generator().manual_seed(5)
+    k, v = (torch.randn(1, 2, 300, 128, generator=g).to(dtype) for _ in range(2))
+    k[0, :, 299, 3] = float("inf")
+    q = torch.randn(1, 32, 1, 128, generator=g)
+    q[..., 3] = -0.5
+    q = q.to(q_dtype)
+    cache = dart.DartKVCache(dart.DartKVCacheConfig(promote_ratio=0.25, key_group_size=128, value_group_size=64,
+                                                    hold_partial_pages=True))
+    cache.append(k.to(DEV), v.to(DEV))
+    dk, dv = (t.cpu().double() for t in cache.get())
+    logits = torch.matmul(q.double().view(1, 2, 16, 128), dk.transpose(-1, -2)) / 128 ** 0.5
+    ref = torch.matmul(torch.softmax(logits, -1), dv).view(1, 32, 1, 128)
+    out = torch.empty(1, 32, 128, dtype=torch.float32, device=DEV)
+    print("case", dtype, q_dtype, flush=True)
+    dart.decode_attention(q.to(DEV), cache, out_f32=out)
+    assert _rel_err(out.unsqueeze(2), ref) <= 1e-5
