@@ -351,9 +351,6 @@ class _DecodePlan:
             self._chunks = torch.tensor(rows, dtype=torch.int32).reshape(len(rows), 3).to(self.device)
         return self._chunks
 
-    def chunks_ready(self) -> bool:
-        return self._chunks is not None or self.table is None
-
 
 class DartKVCache:
     """Append-only KV cache over HIP-quantized pages (reference cache.py:115-542).
@@ -579,15 +576,12 @@ class DartKVCache:
     def _materialize_all(self) -> Optional[Tuple[torch.Tensor, torch.Tensor]]:
         """The contents as dense tensors from one launch over the descriptor table (dkv_materialize), or None
         where the segments are dequantized one by one: a cache on the host, head_dims past 16,384 (the kernel's
-        channel table), Kitty value windows (the two
-        tracks are not cut alike), and under capture a table that is not built yet (its upload cannot be
-        captured)."""
+        channel table), Kitty value windows (the two tracks are not cut alike), and under graph capture (the table
+        lives as long as the plan, which the next sealed page replaces: a replay after it would read freed memory)."""
         device, c = self._device, self.config
         if device is None or device.type != "cuda" or c.value_local_tokens or self._shape[-1] > 16384:
             return None
-        plan = self._decode_plan_cache
-        ready = plan is not None and plan.version == self._sealed_version and plan.device == device
-        if not (ready and plan.chunks_ready()) and torch.cuda.is_current_stream_capturing():
+        if torch.cuda.is_current_stream_capturing():
             return None
         plan = self.decode_plan(device)
         B, H, D = self._shape

@@ -44,3 +44,41 @@ def test_get_equals_the_segments(T, D, dtype, cfg):
     bits = torch.int64 if dtype == F64 else torch.int32 if dtype == F32 else torch.int16
     assert torch.equal(got_k.view(bits), keys.contiguous().view(bits))
     assert torch.equal(got_v.view(bits), values.contiguous().view(bits))
+
+
+def test_captured_get_outlives_the_descriptor_table():
+    """A captured read-back keeps no pointer to the decode plan's table, which the next sealed page replaces: it replays
+    over the pages themselves, which stay where they are while the pool has room."""
+    import dartkv_amd as dart
+    g = torch.Generator().manual_seed(2)
+    k, v = (torch.randn(2, 2, 700, 128, generator=g).to(BF).to(DEV) for _ in range(2))
+    cache = dart.DartKVCache(dart.DartKVCacheConfig(promote_ratio=0.25, hold_partial_pages=True))
+    cache.append(k[..., :513, :], v[..., :513, :])
+    cache.append(k[..., 513:550, :], v[..., 513:550, :])
+    ref = [t.clone() for t in cache.get()]  # (the plan and its table are built)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        cache.get()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        assert cache._materialize_all() is None
+        got = cache.get()
+    for _ in range(3):
+        for t in got:
+            t.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(got, ref))
+
+    def storage():
+        return [t.data_ptr() for t in (cache._key_pool.tensors["low_values"], cache._value_pool.tensors["values"],
+                                       cache._tail_key, cache._tail_value)]
+    before, plan = storage(), cache.decode_plan(cache.device)
+    cache.append(k[..., 550:645, :], v[..., 550:645, :])
+    assert cache.decode_plan(cache.device) is not plan
+    if storage() == before:
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a[..., :512, :], b[..., :512, :]) for a, b in zip(got, ref))
