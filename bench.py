@@ -646,9 +646,9 @@ def time_c5(args, bits: str, torch, dart, synthetic, stream) -> dict:
     ms_per_step = total_ms / args.steps
     gbs = nbytes * args.layers / (ms_per_step * 1e-3) / 1e9
     achieved = fast_bytes / (avg_kernel_ms * 1e-3) / 1e9 if avg_kernel_ms else None
-    # (uniform runs that fill the device go to the tile kernel)
-    tiles = a.batch * a.kv_heads * plan.fast_count >= 2048
-    kernel = "decode_pages_fast" if plan.fast_promoted else "decode_tiles" if tiles else "decode_pages_uniform"
+    from dartkv_amd.attention import decode_route
+    run = decode_route(queries[0], caches[0], n_splits=splits)[0]
+    kernel = "decode_tiles" if run == "tiles" else "decode_pages_fast" if plan.fast_promoted else "decode_pages_uniform"
     tok_s = args.batch / (ms_per_step * 1e-3)
     multi = multi_token_leg(torch, dart, caches, a) if bits == "2b25" and not args.no_multi_token else None
     del caches, queries, step, events, plan

@@ -26,7 +26,7 @@ KEY_DENSE, KEY_UNIFORM, KEY_MIXED = 0, 1, 2
 VALUE_DENSE, VALUE_UNIFORM = 0, 1
 SELECT_MAGNITUDE, SELECT_VARIANCE, SELECT_GIVEN = 0, 1, 2
 
-ABI_VERSION = 14
+ABI_VERSION = 15
 
 _DTYPE_CODES = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2, torch.float64: 3}
 # element types the kernels read and write (sources, outputs, metadata)
@@ -106,6 +106,12 @@ class DecodeArgs(ctypes.Structure):
 
 assert ctypes.sizeof(Segment) == 160
 
+KERNEL_NONE, KERNEL_PAGES, KERNEL_TILES, KERNEL_DENSE, KERNEL_GENERAL = range(5)
+
+
+class DecodeKernels(ctypes.Structure):
+    _fields_ = [("run", ctypes.c_int64), ("rest", ctypes.c_int64), ("rest_units", ctypes.c_int64)]
+
 
 class MaterializeArgs(ctypes.Structure):
     _fields_ = [
@@ -148,6 +154,7 @@ EXPORTED = (
     "dkv_dequantize_rows",
     "dkv_dequantize_mixed", "dkv_decode_workspace_bytes", "dkv_decode_attention", "dkv_decode_attention_noalloc",
     "dkv_decode_scratch_bytes", "dkv_decode_prep", "dkv_copy_token_blocks", "dkv_materialize",
+    "dkv_decode_route",
 )
 
 _lib: Optional[ctypes.CDLL] = None
@@ -183,17 +190,25 @@ def load() -> ctypes.CDLL:
         lib.dkv_decode_scratch_bytes.argtypes = []
         lib.dkv_decode_scratch_bytes.restype = i64
         lib.dkv_decode_prep.argtypes = [ctypes.POINTER(DecodePrepArgs), vp]
+        lib.dkv_decode_route.argtypes = [ctypes.POINTER(DecodeArgs), ctypes.POINTER(DecodeKernels)]
         lib.dkv_materialize.argtypes = [ctypes.POINTER(MaterializeArgs), vp]
         lib.dkv_copy_token_blocks.argtypes = [ctypes.POINTER(CopyBlock), i64, vp]
         for name in ("dkv_quantize_rows", "dkv_quantize_row_blocks", "dkv_quantize_value_rows", "dkv_quantize_key_pages",
                      "dkv_dequantize_rows",
                      "dkv_dequantize_mixed", "dkv_decode_attention", "dkv_decode_attention_noalloc",
-                     "dkv_decode_prep", "dkv_copy_token_blocks", "dkv_materialize"):
+                     "dkv_decode_prep", "dkv_copy_token_blocks", "dkv_materialize", "dkv_decode_route"):
             getattr(lib, name).restype = ctypes.c_int
         if lib.dkv_abi_version() != ABI_VERSION:
             raise RuntimeError("libdartkv_hip.so ABI version mismatch; rebuild it")
         _lib = lib
     return _lib
+
+
+def decode_kernels(args: DecodeArgs) -> DecodeKernels:
+    """The kernels ``dkv_decode_attention`` would run ``args`` on (no GPU is needed)."""
+    out = DecodeKernels()
+    check(load().dkv_decode_route(args, out), "dkv_decode_route")
+    return out
 
 
 def check(rc: int, where: str) -> None:

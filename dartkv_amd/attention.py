@@ -162,27 +162,12 @@ def _call_layout(plan, cache: DartKVCache, q3: torch.Tensor, kv_heads: int, head
     return a, a.workspace_bytes
 
 
-def decode_attention(query: torch.Tensor, cache: DartKVCache, *, scale: Optional[float] = None,
-                     n_splits: Optional[int] = None, out_f32: Optional[torch.Tensor] = None,
-                     fast: Optional[bool] = None, fast_events=None, out: Optional[torch.Tensor] = None,
-                     static_scratch: bool = False) -> torch.Tensor:
-    """Single-token decode over the packed cache with the HIP split-K kernel.
-
-    ``query`` is [B, Hq, 1, D] (or [B, Hq, D]) on the cache's device.  Returns
-    [B, Hq, 1, D] in ``query.dtype``.  If ``out_f32`` ([B, Hq, D] fp32) is
-    given it receives the result before the final cast.  ``fast`` selects
-    the MFMA page kernel for the pages it supports (default: on unless the
-    environment sets DKV_FORCE_GENERAL=1, read at the first call); ``n_splits`` overrides the split
-    count of the page kernel (or of the general kernel when it does all work).
-    ``fast_events`` (two recorded ``torch.cuda.Event`` objects) are recorded
-    again right before and after the page kernel, to time it alone.  ``out``
-    ([B, Hq, 1, D] in ``query.dtype``) receives the result instead of a new
-    tensor.  ``static_scratch`` keeps the split records in the library's static
-    device scratch (``dkv_decode_attention_noalloc``) instead of a workspace
-    tensor, so with ``out`` given the call allocates nothing.
-    """
+def _prepare_call(query: torch.Tensor, cache: DartKVCache, scale: Optional[float], n_splits: Optional[int],
+                  fast: Optional[bool], static_scratch: bool):
+    """A decode call's checked parts: the query as [B, Hq, D], the plan, the tail's descriptor, and the call's layout
+    (argument template, workspace bytes)."""
     _lib.require_device(query)
-    batch, kv_heads, head_dim = _check_query(query, cache)
+    _, kv_heads, head_dim = _check_query(query, cache)
     # q3: the query as [B, Hq, D] (a [B, Hq, 1, D] query is read through its own strides 0, 1 and 3)
     q3 = query.reshape(query.shape[0], query.shape[1], query.shape[-1]) if query.ndim == 4 and query.shape[2] != 1 \
         else query
@@ -207,7 +192,44 @@ def decode_attention(query: torch.Tensor, cache: DartKVCache, *, scale: Optional
     if layout is None:
         layout = plan.call_layouts[key] = _call_layout(plan, cache, q3, kv_heads, head_dim, tail, use_fast, dense_ok,
                                                        n_splits, factor)
-    template, ws_bytes = layout
+    return q3, plan, tail, layout
+
+
+def decode_route(query: torch.Tensor, cache: DartKVCache, *, scale: Optional[float] = None,
+                 n_splits: Optional[int] = None, fast: Optional[bool] = None) -> Tuple[str, str]:
+    """The kernels ``decode_attention`` runs these arguments on: one for the page run, one for the other entries
+    ("none", "pages", "tiles", "dense" or "general")."""
+    _, _, tail, (template, _) = _prepare_call(query, cache, scale, n_splits, fast, False)
+    a = _lib.DecodeArgs.from_buffer_copy(template)
+    a.tail = tail
+    kernels = _lib.decode_kernels(a)
+    names = ("none", "pages", "tiles", "dense", "general")
+    return names[kernels.run], names[kernels.rest]
+
+
+def decode_attention(query: torch.Tensor, cache: DartKVCache, *, scale: Optional[float] = None,
+                     n_splits: Optional[int] = None, out_f32: Optional[torch.Tensor] = None,
+                     fast: Optional[bool] = None, fast_events=None, out: Optional[torch.Tensor] = None,
+                     static_scratch: bool = False) -> torch.Tensor:
+    """Single-token decode over the packed cache with the HIP split-K kernel.
+
+    ``query`` is [B, Hq, 1, D] (or [B, Hq, D]) on the cache's device.  Returns
+    [B, Hq, 1, D] in ``query.dtype``.  If ``out_f32`` ([B, Hq, D] fp32) is
+    given it receives the result before the final cast.  ``fast`` selects
+    the page run's kernels for the pages they support (default: on unless the
+    environment sets DKV_FORCE_GENERAL=1, read at the first call; off, all
+    entries go to the tile kernel, or to the general kernel where that does not
+    read them: ``decode_route``); ``n_splits`` overrides the split count of the
+    page run (or of the kernel that does all work).
+    ``fast_events`` (two recorded ``torch.cuda.Event`` objects) are recorded
+    again right before and after the page kernel, to time it alone.  ``out``
+    ([B, Hq, 1, D] in ``query.dtype``) receives the result instead of a new
+    tensor.  ``static_scratch`` keeps the split records in the library's static
+    device scratch (``dkv_decode_attention_noalloc``) instead of a workspace
+    tensor, so with ``out`` given the call allocates nothing.
+    """
+    q3, plan, tail, (template, ws_bytes) = _prepare_call(query, cache, scale, n_splits, fast, static_scratch)
+    batch, Hq, head_dim, device = q3.shape[0], q3.shape[1], q3.shape[-1], query.device
     if out is None:
         out = torch.empty(batch, Hq, 1, head_dim, dtype=query.dtype, device=query.device)
     elif out.shape != (batch, Hq, 1, head_dim) or out.dtype != query.dtype or out.device != query.device \

@@ -515,6 +515,42 @@ static int check_segments(const dkv_decode_args& a, int64_t fast_count, bool den
   return DKV_OK;
 }
 
+// The launch parameters of the entries outside the page run.
+static DecodeParams rest_params(const dkv_decode_args& a) {
+  const bool run = a.fast_count > 0;
+  DecodeParams p;
+  p.a = a;
+  p.group = (int)(a.Hq / a.Hkv);
+  p.n_total = (int)(a.n_segments - (run ? a.fast_count : 0) + (a.tail.tokens > 0 ? 1 : 0));
+  p.splits = p.n_total > 0 ? (int)a.n_splits : 0;
+  p.split_offset = run ? (int)a.fast_splits : 0;
+  p.split_stride = p.split_offset + p.splits;
+  p.skip_first = run ? (int)a.fast_first : 0;
+  p.skip_count = run ? (int)a.fast_count : 0;
+  return p;
+}
+
+extern "C" int dkv_decode_route(const dkv_decode_args* args, dkv_decode_kernels* out) {
+  DKV_CHECK(args != nullptr && out != nullptr, DKV_ERR_INVALID, "args or out is NULL");
+  const dkv_decode_args& a = *args;
+  DKV_CHECK(a.Hkv > 0 && a.Hq > 0 && a.Hq % a.Hkv == 0, DKV_ERR_INVALID, "bad decode shape");
+  DKV_CHECK(a.n_segments >= 0 && (a.fast_count <= 0 || (a.fast_first >= 0 && a.fast_first + a.fast_count <= a.n_segments)),
+            DKV_ERR_INVALID, "fast page range outside the descriptor table");
+  const DecodeParams p = rest_params(a);
+  dkv::TileRest tiles;
+  out->run = a.fast_count <= 0 ? DKV_KERNEL_NONE
+             : dkv::tiles_take_run(a, p.group) ? DKV_KERNEL_TILES : DKV_KERNEL_PAGES;
+  out->rest_units = p.n_total;
+  if (p.n_total == 0) {
+    out->rest = DKV_KERNEL_NONE;
+  } else if (a.rest_dense_tokens > 0) {
+    out->rest = out->run == DKV_KERNEL_TILES ? DKV_KERNEL_TILES : DKV_KERNEL_DENSE;
+  } else {
+    out->rest = dkv::tiles_take_rest(p, &tiles) ? DKV_KERNEL_TILES : DKV_KERNEL_GENERAL;
+  }
+  return DKV_OK;
+}
+
 extern "C" int dkv_decode_attention(const dkv_decode_args* args, void* stream) {
   DKV_CHECK(args != nullptr, DKV_ERR_INVALID, "args is NULL");
   dkv_decode_args a = *args;
@@ -573,15 +609,7 @@ extern "C" int dkv_decode_attention(const dkv_decode_args* args, void* stream) {
     if (rc != DKV_OK) return rc;
   }
   hipStream_t s = (hipStream_t)stream;
-  DecodeParams p;
-  p.a = a;
-  p.group = (int)(a.Hq / a.Hkv);
-  p.n_total = (int)rest;
-  p.splits = (int)general_splits;
-  p.split_offset = (int)fast_splits;
-  p.split_stride = (int)stride;
-  p.skip_first = fast_count > 0 ? (int)a.fast_first : 0;
-  p.skip_count = fast_count > 0 ? (int)fast_count : 0;
+  DecodeParams p = rest_params(a);
   const bool dense_rest = rest > 0 && a.rest_dense_tokens > 0;
   const int64_t chunks = dense_rest ? (a.rest_dense_tokens + kDenseChunk - 1) / kDenseChunk : 0;
   if (dense_rest) {
@@ -689,16 +717,16 @@ extern "C" int dkv_decode_attention(const dkv_decode_args* args, void* stream) {
     int rc = dkv_check_launch("dkv_decode_attention(dense)");
     if (rc) return rc;
   } else if (general_splits > 0) {
-    bool taken = false;
-    int rc = dkv::launch_tile_decode(p, s, &taken);
-    if (rc) return rc;
     const dim3 grid((unsigned)general_splits, (unsigned)a.Hkv, (unsigned)a.B);
-    if (taken) {
-    } else if (p.group <= 1) hipLaunchKernelGGL(decode_split_general<1>, grid, dim3(kThreads), 0, s, p);
+    dkv::TileRest tiles;
+    int rc = DKV_OK;
+    if (dkv::tiles_take_rest(p, &tiles)) rc = dkv::launch_tile_run(p, tiles.first, tiles.count, p.splits, tiles.layout, s);
+    else if (p.group <= 1) hipLaunchKernelGGL(decode_split_general<1>, grid, dim3(kThreads), 0, s, p);
     else if (p.group <= 2) hipLaunchKernelGGL(decode_split_general<2>, grid, dim3(kThreads), 0, s, p);
     else if (p.group <= 4) hipLaunchKernelGGL(decode_split_general<4>, grid, dim3(kThreads), 0, s, p);
     else if (p.group <= 8) hipLaunchKernelGGL(decode_split_general<8>, grid, dim3(kThreads), 0, s, p);
     else hipLaunchKernelGGL(decode_split_general<16>, grid, dim3(kThreads), 0, s, p);
+    if (rc) return rc;
     rc = dkv_check_launch("dkv_decode_attention(split)");
     if (rc) return rc;
   }

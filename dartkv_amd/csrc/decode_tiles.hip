@@ -1094,37 +1094,35 @@ int launch_tile_run(const DecodeParams& d, int first, int count, int splits, con
   return bf ? launch_tiles_heads<128, true>(p, g.bits, mixed, s) : launch_tiles_heads<128, false>(p, g.bits, mixed, s);
 }
 
-int launch_tile_decode(const DecodeParams& d, hipStream_t stream, bool* taken) {
-  *taken = false;
+bool tiles_take_rest(const DecodeParams& d, TileRest* rest) {
   const dkv_decode_args& a = d.a;
   if ((a.cache_dtype != kBF16 && a.cache_dtype != kF16) || a.q_dtype != a.cache_dtype || a.meta_dtype != kF16)
-    return DKV_OK;
-  if ((a.D != 64 && a.D != 128) || d.group > 16 || (a.n_segments > 0 && a.segments_host == nullptr)) return DKV_OK;
-  if (a.B * a.Hkv * d.splits >= (int64_t)1 << 31) return DKV_OK;
+    return false;
+  if ((a.D != 64 && a.D != 128) || d.group > 16 || (a.n_segments > 0 && a.segments_host == nullptr)) return false;
+  if (a.B * a.Hkv * d.splits >= (int64_t)1 << 31) return false;
   const int n_rest = (int)a.n_segments - d.skip_count;
   auto entry = [&](int i) -> const dkv_segment& {
     return i >= n_rest ? a.tail : a.segments_host[i < d.skip_first ? i : i + d.skip_count];
   };
   // one run of packed segments of one layout, everything else dense
-  int first = 0, count = 0;
+  *rest = TileRest{0, 0, TileLayout{2, 128, 64, 0}};  // (without packed segments the layout is not used)
   for (int i = 0; i < d.n_total; ++i) {
     const dkv_segment& g = entry(i);
     if (g.key_kind == DKV_KEY_DENSE) {
-      if (!dense_ok(g)) return DKV_OK;
+      if (!dense_ok(g)) return false;
       continue;
     }
-    if (i >= n_rest || !packed_ok(g, (int)a.D)) return DKV_OK;
-    if (count == 0) first = i;
-    else if (i != first + count || !same_layout(entry(first), g)) return DKV_OK;
-    ++count;
+    if (i >= n_rest || !packed_ok(g, (int)a.D)) return false;
+    if (rest->count == 0) {
+      rest->first = i;
+      rest->layout =
+          TileLayout{g.value_bits, g.key_group, g.value_group, g.key_kind == DKV_KEY_MIXED ? g.promoted : 0};
+    } else if (i != rest->first + rest->count || !same_layout(entry(rest->first), g)) {
+      return false;
+    }
+    ++rest->count;
   }
-  TileLayout l{2, 128, 64, 0};  // (without packed segments the layout is not used)
-  if (count) {
-    const dkv_segment& g = entry(first);
-    l = TileLayout{g.value_bits, g.key_group, g.value_group, g.key_kind == DKV_KEY_MIXED ? g.promoted : 0};
-  }
-  *taken = true;
-  return launch_tile_run(d, first, count, d.splits, l, stream);
+  return true;
 }
 
 }  // namespace dkv

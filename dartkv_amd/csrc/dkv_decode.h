@@ -34,11 +34,6 @@ int launch_fast_decode(const dkv_decode_args& a, int first, int count, int np, i
 int uniform_decode_max_loads(int kb, int vb, int gv);
 int launch_uniform_decode(const dkv_decode_args& a, int first, int count, int kb, int vb, int vg, int splits,
                           int split_stride, hipStream_t stream, const FusedRest* fused = nullptr);
-// The segments of a decode call outside the page kernels' run, for 16-bit
-// caches (decode_tiles.hip); *taken is false, and nothing is launched, when
-// they are not of the forms that kernel reads.
-int launch_tile_decode(const DecodeParams& d, hipStream_t stream, bool* taken);
-
 // Whether the tile kernel takes a call's page run instead of the page kernels
 // (the run is as dkv_decode_args guarantees), and its launch over `count`
 // packed entries from `first` on and the dense entries around them (d.n_total
@@ -48,6 +43,15 @@ struct TileLayout {
 };
 bool tiles_take_run(const dkv_decode_args& a, int group);
 int launch_tile_run(const DecodeParams& d, int first, int count, int splits, const TileLayout& g, hipStream_t stream);
+
+// Whether the tile kernel reads the segments of a decode call outside the page
+// kernels' run (checked on the host copies of the descriptors): `count` packed
+// ones of one layout from entry `first` of the rest on, the others dense.
+struct TileRest {
+  int first, count;
+  TileLayout layout;
+};
+bool tiles_take_rest(const DecodeParams& d, TileRest* rest);
 // LDS bytes of one wave of the uniform page kernel.
 size_t uniform_decode_wave_lds_bytes(int kb, int vb, int gv);
 

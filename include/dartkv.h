@@ -52,7 +52,7 @@ extern "C" {
 /* Thread-local description of the last error on this thread. */
 const char* dkv_last_error(void);
 
-/* ABI version (13); bumps when a struct or an entry point below changes. */
+/* ABI version (15); bumps when a struct or an entry point below changes. */
 int dkv_abi_version(void);
 
 /*
@@ -405,6 +405,23 @@ typedef struct dkv_decode_prep_args {
 int dkv_decode_prep(const dkv_decode_prep_args* args, void* stream);
 
 int64_t dkv_decode_workspace_bytes(int64_t B, int64_t Hq, int64_t D, int64_t n_splits);
+
+/*
+ * The kernels dkv_decode_attention would run a call on (host only; device
+ * pointers, workspace and n_splits need not be set): `run` for the page run,
+ * `rest` for the other entries and the tail, and the number of pieces the
+ * rest's work comes in (more splits than that leave some empty).
+ */
+#define DKV_KERNEL_NONE 0
+#define DKV_KERNEL_PAGES 1   /* the page kernels */
+#define DKV_KERNEL_TILES 2   /* the tile kernel */
+#define DKV_KERNEL_DENSE 3   /* the dense chunks */
+#define DKV_KERNEL_GENERAL 4 /* the general kernel */
+typedef struct dkv_decode_kernels {
+  int64_t run, rest, rest_units;
+} dkv_decode_kernels;
+
+int dkv_decode_route(const dkv_decode_args* args, dkv_decode_kernels* out);
 
 int dkv_decode_attention(const dkv_decode_args* args, void* stream);
 

@@ -20,7 +20,12 @@ def _rel_err(a, b):
     return float(((a - b).abs().amax(-1) / b.abs().amax(-1).clamp_min(1e-30)).max())
 
 
-def _run(B, Hkv, G, D, T, dtype, cfg, updates=(), n_splits=None):
+def _route(q, cache, **options):
+    from dartkv_amd.attention import decode_route
+    return decode_route(q.to(DEV), cache, **options)
+
+
+def _run(B, Hkv, G, D, T, dtype, cfg, updates=(), n_splits=None, kernel="tiles"):
     import dartkv_amd as dart
     from dartkv_amd import synthetic
     from oracle import dart_oracle as O
@@ -37,6 +42,7 @@ def _run(B, Hkv, G, D, T, dtype, cfg, updates=(), n_splits=None):
     ref = O.streamed_attention(q, oc, return_fp32=True)[1]
     out = torch.empty(B, Hkv * G, D, dtype=torch.float32, device=DEV)
     print("case", B, Hkv, G, D, T, dtype, cfg, n_splits, flush=True)
+    assert _route(q, cache, fast=False, n_splits=n_splits) == ("none", kernel)
     dart.decode_attention(q.to(DEV), cache, out_f32=out, fast=False, n_splits=n_splits)
     torch.cuda.synchronize()
     return _rel_err(out.unsqueeze(2), ref)
@@ -80,6 +86,18 @@ def test_tile_kernel_vs_oracle(G, D, T, dtype, cfg):
     assert _run(2, 2, G, D, T, dtype, cfg) <= 1e-5
 
 
+@pytest.mark.parametrize("G,D,T,dtype,cfg", [
+    (4, 96, 400, BF, dict(key_group_size=64, value_group_size=32)),          # head_dim
+    (4, 128, 400, torch.float32, dict(key_group_size=64)),                   # cache type
+    (4, 128, 400, BF, dict(metadata_dtype=BF)),
+    (4, 128, 400, FP, dict(page_size=80, key_group_size=40)),
+    (4, 128, 400, FP, dict(value_group_size=16)),                            # eight value groups
+    (4, 64, 400, BF, dict(bits=4, value_bits=2)),
+])
+def test_what_the_tile_kernel_leaves_to_the_general_kernel(G, D, T, dtype, cfg):
+    assert _run(2, 2, G, D, T, dtype, cfg, kernel="general") <= 1e-5
+
+
 @pytest.mark.parametrize("n_splits", [1, 2, 5, 64])
 def test_tile_kernel_split_counts(n_splits):
     """Splits that hold several pages, a page and the dense pieces, or nothing but a dense piece."""
@@ -100,6 +118,7 @@ def test_rest_of_a_page_run_takes_the_tile_kernel():
     cache.append(k.to(DEV), v.to(DEV))
     ref = O.streamed_attention(q, oc, return_fp32=True)[1]
     out = torch.empty(2, 16, 128, dtype=torch.float32, device=DEV)
+    assert _route(q, cache) == ("pages", "tiles")
     dart.decode_attention(q.to(DEV), cache, out_f32=out)
     torch.cuda.synchronize()
     assert _rel_err(out.unsqueeze(2), ref) <= 2e-3
@@ -117,6 +136,7 @@ def test_tile_kernel_keeps_infinite_dense_values(dtype):
     cache = dart.DartKVCache(dart.DartKVCacheConfig(bits=4, page_size=128, key_group_size=64, value_group_size=64,
                                                     hold_partial_pages=True))
     cache.append(k.to(DEV), v.to(DEV))
+    assert _route(q, cache) == ("none", "tiles")
     out = dart.fused_dart_attention(q.to(DEV), cache).cpu()
     torch.cuda.synchronize()
     expected = torch.zeros(1, 6, 1, 64, dtype=torch.bool)
@@ -156,6 +176,10 @@ def test_page_runs_the_tile_kernel_takes(G, T, dtype, q_dtype, cfg):
     torch.cuda.synchronize()
     assert got.dtype == q_dtype and events[0].elapsed_time(events[1]) >= 0
     tiles = G == 16 or (q_dtype == dtype and "value_bits" not in cfg and cfg["bits"] < 8)
+    rest = "tiles" if q_dtype == dtype else "general"
+    if cfg["hold_partial_pages"]:
+        rest = "tiles" if tiles else "dense"
+    assert _route(q, cache, fast=True) == ("tiles" if tiles else "pages", rest)
     assert _rel_err(out.unsqueeze(2), ref) <= (1e-5 if tiles else 2e-3)
 
 
@@ -269,6 +293,7 @@ def test_small_weights_keep_their_bits(G, D, dtype, gap):
     ref = torch.matmul(torch.softmax(logits, -1), dv).view(1, 2 * G, 1, D)
     out = torch.empty(1, 2 * G, D, dtype=torch.float32, device=DEV)
     print("case", G, D, dtype, gap, flush=True)
+    assert _route(q, cache, fast=False, n_splits=1) == ("none", "tiles")
     dart.decode_attention(q.to(DEV), cache, scale=1.0, out_f32=out, fast=False, n_splits=1)
     got = out.cpu().double().view(1, 2 * G, 1, D)
     assert float(((got - ref).abs() / ref.abs()).max()) <= 7.8e-6
@@ -282,6 +307,7 @@ def test_infinite_value_of_a_small_weight(G, dtype):
     v[0, 1, 299, 5] = float("inf")
     cache.append(k.to(DEV), v.to(DEV))
     print("case", G, dtype, flush=True)
+    assert _route(q, cache, fast=False, n_splits=1) == ("none", "tiles")
     out = dart.decode_attention(q.to(DEV), cache, scale=1.0, fast=False, n_splits=1).cpu()
     expected = torch.zeros(1, 2 * G, 1, 64, dtype=torch.bool)
     expected[0, G:, 0, 5] = True
@@ -307,5 +333,6 @@ def test_infinite_key_under_a_query_of_another_type(dtype, q_dtype):
     ref = torch.matmul(torch.softmax(logits, -1), dv).view(1, 32, 1, 128)
     out = torch.empty(1, 32, 128, dtype=torch.float32, device=DEV)
     print("case", dtype, q_dtype, flush=True)
+    assert _route(q, cache) == ("tiles", "tiles")
     dart.decode_attention(q.to(DEV), cache, out_f32=out)
     assert _rel_err(out.unsqueeze(2), ref) <= 1e-5
