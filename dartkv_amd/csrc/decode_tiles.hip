@@ -101,10 +101,11 @@ __device__ __forceinline__ const_segment& rest_entry(const DecodeParams& p, int 
 // Global loads from a wave-uniform base and a 32-bit lane offset (the
 // addresses come out of memory, so without the address space they would be
 // flat loads, which also count as LDS traffic).
-template <class T>
+template <class T, int ALIGN = alignof(T)>
 __device__ __forceinline__ T gload(const void* base, uint32_t off) {
+  typedef T aligned_t __attribute__((aligned(ALIGN)));
   typedef __attribute__((address_space(1))) const uint8_t gbyte;
-  typedef __attribute__((address_space(1))) const T gtype;
+  typedef __attribute__((address_space(1))) const aligned_t gtype;
   return *(gtype*)((gbyte*)(uintptr_t)base + off);
 }
 
@@ -200,10 +201,11 @@ __device__ __forceinline__ void load_codes(uint32_t (&regs)[N], Base base, Off o
   for (int p = 0; p < NK / 2; ++p) {
     const uint8_t* a = base(2 * p);
     const uint32_t oa = off(2 * p);
+    // (a shared load is aligned to one lane's codes only: value rows of an odd number of them)
     if constexpr (C::kBytes == 1) {
-      regs[p] = gload<uint16_t>(a, oa);
+      regs[p] = gload<uint16_t, 1>(a, oa);
     } else if constexpr (C::kBytes == 2) {
-      regs[p] = gload<uint32_t>(a, oa);
+      regs[p] = gload<uint32_t, 2>(a, oa);
     } else if constexpr (C::kBytes == 4) {
       regs[2 * p] = gload<uint32_t>(a, oa);
       regs[2 * p + 1] = gload<uint32_t>(base(2 * p + 1), off(2 * p + 1));
@@ -1010,9 +1012,13 @@ bool dense_ok(const dkv_segment& g) {
          g.value[0] % 16 == 0 && (2 * g.value_bh[0]) % 16 == 0;
 }
 
-// Whether the tile kernel reads this packed segment (host).
+// Whether the tile kernel reads this packed segment (host).  The bounds on its
+// tokens and groups (a page of any size in use has far smaller ones) keep the
+// kernel's 32-bit offsets in range: a key row is at most 2^17 bytes, a segment's
+// values at most 2^28.
 bool packed_ok(const dkv_segment& g, int D) {
-  if (g.tokens < 1 || g.tokens > (1 << 16) || g.value_kind != DKV_VALUE_UNIFORM) return false;
+  if (g.tokens < 1 || g.tokens > (1 << 16) || g.key_group > (1 << 16) || g.value_group > (1 << 12)) return false;
+  if (g.value_kind != DKV_VALUE_UNIFORM) return false;
   if (g.key_kind != DKV_KEY_MIXED && g.key_kind != DKV_KEY_UNIFORM) return false;
   const bool mixed = g.key_kind == DKV_KEY_MIXED;
   const int bits = mixed ? 2 : g.key_bits;

@@ -72,6 +72,10 @@ def test_rest_by_call(call, route):
     (dict(bits=8, vgroup=32), "tiles"), (dict(bits=4, vgroup=200), "tiles"),
     (dict(kgroup=48), "general"), (dict(kgroup=192), "general"), (dict(vgroup=16), "general"),
     (dict(bits=4, value_bits=2), "general"), (dict(key="dart", promoted=0), "general"),
+    # sizes whose byte offsets would leave 32 bits (or 24, where they are factors)
+    (dict(kgroup=1 << 16), "tiles"), (dict(kgroup=1 << 17), "general"), (dict(kgroup=1 << 27, bits=4), "general"),
+    (dict(bits=8, vgroup=4096), "tiles"), (dict(bits=8, vgroup=1 << 15, tokens=1 << 16), "general"),
+    (dict(tokens=1 << 16), "tiles"), (dict(tokens=(1 << 16) + 1), "general"),
 ])
 def test_rest_by_page_layout(page, route):
     assert _route(_args([_page(**page)] * 2)) == ("none", route)

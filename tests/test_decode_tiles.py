@@ -67,6 +67,10 @@ def _run(B, Hkv, G, D, T, dtype, cfg, updates=(), n_splits=None, kernel="tiles")
     (4, 64, 500, FP, dict(key_group_size=256, value_group_size=16)),
     (7, 128, 500, BF, dict(bits=4, key_group_size=64, value_group_size=48)),
     (2, 64, 500, BF, dict(bits=4, key_group_size=32, value_group_size=64)),
+    # value rows of 42 and 18 bytes: off the shared loads' width
+    (4, 128, 500, BF, dict(value_group_size=56)),
+    (3, 128, 500, FP, dict(promote_ratio=0.25, value_group_size=56)),
+    (4, 64, 500, BF, dict(value_group_size=24)),
     (4, 128, 500, FP, dict(bits=8, key_group_size=64, value_group_size=128)),
     (12, 64, 500, BF, dict(bits=8, key_group_size=32, value_group_size=32)),
     # segments that are not one full tile: short pages, pages of 256 tokens (two and four tiles), partial pages
