@@ -287,7 +287,8 @@ __global__ void __launch_bounds__(kThreads) decode_merge(DecodeParams p) {
     const float lw = l * w;
     float L = 0.f;
     for (int s = 0; s < S; ++s) L += __shfl(lw, s, 64);
-    if (tid == 0) den[0] = fmaxf(L, 1e-20f);
+    const bool none = M == -INFINITY && __ballot(l == kNoWeight) != 0ull;
+    if (tid == 0) den[0] = none ? NAN : fmaxf(L, 1e-20f);
   }
   __syncthreads();
   if (tid < D) {
@@ -365,6 +366,10 @@ __global__ void __launch_bounds__(kMergeWideThreads) decode_merge_wide(DecodePar
 #pragma unroll
     for (int w = 0; w < kMergeWideThreads / 64; ++w) L += wave_l[w];
     o /= fmaxf(L, 1e-20f);
+    if (M == -INFINITY) {
+      for (int s = 0; s < S; ++s)
+        if (ws[(int64_t)s * (D + 2) + 1] == kNoWeight) o = NAN;
+    }
     const int b = bq / (int)a.Hq, hq = bq % (int)a.Hq;
     dev_store(a.out, (int64_t)b * a.out_sb + (int64_t)hq * a.out_sh + tid, o, (int)a.q_dtype);
     if (a.out_f32) a.out_f32[(int64_t)bq * D + tid] = o;
@@ -546,7 +551,9 @@ extern "C" int dkv_decode_route(const dkv_decode_args* args, dkv_decode_kernels*
   } else if (a.rest_dense_tokens > 0) {
     out->rest = out->run == DKV_KERNEL_TILES ? DKV_KERNEL_TILES : DKV_KERNEL_DENSE;
   } else {
-    out->rest = dkv::tiles_take_rest(p, &tiles) ? DKV_KERNEL_TILES : DKV_KERNEL_GENERAL;
+    const bool taken = dkv::tiles_take_rest(p, &tiles);
+    out->rest = taken ? DKV_KERNEL_TILES : DKV_KERNEL_GENERAL;
+    if (taken) out->rest_units = tiles.items;
   }
   return DKV_OK;
 }
@@ -635,8 +642,9 @@ extern "C" int dkv_decode_attention(const dkv_decode_args* args, void* stream) {
     DecodeParams t = p;
     t.skip_first = t.skip_count = 0;
     const bool all = rest == 0 || dense_rest;  // the dense pieces ride in the same launch
-    t.n_total = (int)(all ? a.n_segments + (a.tail.tokens > 0 ? 1 : 0) : fast_count);
-    // one page per split: one dense piece per split too (there is a record for each)
+    const int n_dense = all ? (int)rest : 0;
+    t.n_total = dkv::tile_items((int)fast_count, n_dense, a.rest_dense_tokens);
+    // one page per split: one dense piece per split too (there are records for smaller ones)
     const int splits = (int)(fast_splits >= fast_count ? t.n_total : fast_splits);
     t.split_offset = 0;
     if (all) t.split_stride = splits;
@@ -645,7 +653,7 @@ extern "C" int dkv_decode_attention(const dkv_decode_args* args, void* stream) {
     if (rc) return rc;
     const dkv::TileLayout layout{a.fast_promoted > 0 ? 2 : (int)a.fast_key_bits, 128, (int)a.fast_value_group,
                                  (int)a.fast_promoted};
-    rc = dkv::launch_tile_run(t, (int)a.fast_first, (int)fast_count, splits, layout, s);
+    rc = dkv::launch_tile_run(t, (int)a.fast_first, (int)fast_count, n_dense, splits, layout, s);
     if (rc) return rc;
     rc = record_event(a.fast_events[1], s);
     if (rc) return rc;
@@ -720,8 +728,11 @@ extern "C" int dkv_decode_attention(const dkv_decode_args* args, void* stream) {
     const dim3 grid((unsigned)general_splits, (unsigned)a.Hkv, (unsigned)a.B);
     dkv::TileRest tiles;
     int rc = DKV_OK;
-    if (dkv::tiles_take_rest(p, &tiles)) rc = dkv::launch_tile_run(p, tiles.first, tiles.count, p.splits, tiles.layout, s);
-    else if (p.group <= 1) hipLaunchKernelGGL(decode_split_general<1>, grid, dim3(kThreads), 0, s, p);
+    if (dkv::tiles_take_rest(p, &tiles)) {
+      DecodeParams t = p;
+      t.n_total = tiles.items;
+      rc = dkv::launch_tile_run(t, tiles.first, tiles.count, tiles.n_dense, p.splits, tiles.layout, s);
+    } else if (p.group <= 1) hipLaunchKernelGGL(decode_split_general<1>, grid, dim3(kThreads), 0, s, p);
     else if (p.group <= 2) hipLaunchKernelGGL(decode_split_general<2>, grid, dim3(kThreads), 0, s, p);
     else if (p.group <= 4) hipLaunchKernelGGL(decode_split_general<4>, grid, dim3(kThreads), 0, s, p);
     else if (p.group <= 8) hipLaunchKernelGGL(decode_split_general<8>, grid, dim3(kThreads), 0, s, p);

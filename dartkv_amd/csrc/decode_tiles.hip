@@ -68,6 +68,7 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kTileWaves = 4;
+constexpr int kPiece = 128;         // tokens of a dense work item
 constexpr int kMaxGroups = 4;       // key groups per tile, value groups per token
 // Natural-log headroom of a weight before the running maximum moves, and the
 // power of two weights are scaled by.  fp16's range sets how small a part can
@@ -78,11 +79,15 @@ template <bool BF> constexpr float kTileSlack = BF ? 5.5f : 2.07f;
 template <bool BF> constexpr int kWeightExp = BF ? 0 : 13;
 
 struct TileParams {
-  // This kernel's segments are numbered packed first: index i < n_packed is
-  // rest entry packed_first + i, then come the dense entries in order (rest
-  // entries: the descriptors outside the page kernels' run, then the tail).
+  // This kernel's work items (d.n_total of them, dealt to the splits in order)
+  // are the packed segments, item i < n_packed being rest entry packed_first + i,
+  // then the dense entries' pieces of kPiece tokens: the first piece of each
+  // entry, then the second ones (rest entries: the descriptors outside the page
+  // kernels' run, then the tail).  A piece is the work of a page, so a long
+  // dense window spreads over the splits: as one item, a window of 4,096 tokens
+  // beside 64 uniform pages of one sequence kept its wave busy for 142 µs.
   DecodeParams d;
-  int packed_first, n_packed, splits;
+  int packed_first, n_packed, n_dense, splits;
   // what every packed segment shares
   int key_group, value_group, promoted;
   // LDS of one wave (bytes): the key tables, and after Q K the value tables in
@@ -466,9 +471,10 @@ struct TileState {
     for (int i = 0; i < 4; ++i) {
       const int head = GP == 4 ? i : GP == 8 ? 4 * (kq & 1) + i : 4 * kq + i;
       float w[U], sum = 0.f;  // (added to l once per tile, as O is)
+      const float m_safe = m_run[i] == -INFINITY ? 0.f : m_run[i];  // (no token with a logit above it yet)
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        const float dlt = x[u][i] - m_run[i];
+        const float dlt = x[u][i] - m_safe;
         w[u] = __builtin_amdgcn_exp2f(BF ? dlt * kLog2e : __builtin_fmaf(dlt, kLog2e, (float)kWeightExp<BF>));
         sum += w[u];
         // a weight below fp16's smallest step, but not zero, gets one (at_least_tiny)
@@ -565,7 +571,7 @@ __global__ void __launch_bounds__(64 * kTileWaves, 2) decode_tiles(TileParams p)
   // Forms whose registers are full form the lane's coordinates anew for each
   // tile: the addresses made from them would otherwise be kept from tile to tile
   // and spilled (elsewhere this costs 2 %).
-  constexpr bool kRederive = D == 128 && ((GP == 16 && (MIXED || KBITS == 4)) || (GP == 8 && MIXED && !BF));
+  constexpr bool kRederive = D == 128 && GP >= 8 && (MIXED || (GP == 16 && KBITS == 4));
   constexpr int kTabK = D * 8 + 16, kTabV = TILE * 8 + 16;
   typedef Codes<KBITS, NJ> KC;
   typedef Codes<VBITS, NC> VC;
@@ -942,11 +948,13 @@ __global__ void __launch_bounds__(64 * kTileWaves, 2) decode_tiles(TileParams p)
     }
   }
 
-  // ---- dense segments ----
+  // ---- dense pieces ----
+  bool seen = s0 < min(s1, p.n_packed);  // the split has tokens
   const int n_rest = (int)a.n_segments - d.skip_count;
 #pragma unroll 1
   for (int i = max(s0, p.n_packed); i < s1; ++i) {
-    const int j = i - p.n_packed, e = uni(j < p.packed_first ? j : j + p.n_packed);
+    const int j = i - p.n_packed, piece = uni(j / p.n_dense), entry = uni(j % p.n_dense);
+    const int e = entry < p.packed_first ? entry : entry + p.n_packed;
     int tokens;
     uint64_t k, v;
     bool dense = true;
@@ -965,7 +973,11 @@ __global__ void __launch_bounds__(64 * kTileWaves, 2) decode_tiles(TileParams p)
       k = a.tail.key[0] + (uint64_t)(2 * bh * a.tail.key_bh[0]);
       v = a.tail.value[0] + (uint64_t)(2 * bh * a.tail.value_bh[0]);
     }
-    tokens = uni(tokens);
+    const int first = piece * kPiece;
+    tokens = uni(min(tokens - first, kPiece));
+    k += (uint64_t)first * (2 * D);
+    v += (uint64_t)first * (2 * D);
+    seen |= tokens > 0;
     if (!dense) {  // (a caller that passed no host copy of the descriptors to check): a NaN record
       st.m_run[0] = st.m_run[1] = st.m_run[2] = st.m_run[3] = NAN;
       tokens = 0;
@@ -991,7 +1003,7 @@ __global__ void __launch_bounds__(64 * kTileWaves, 2) decode_tiles(TileParams p)
     const bool writes = head < G && (GP == 4 ? kq == 0 : GP == 8 ? kq < 2 : true);
     if (writes && n == 0) {
       rec[0] = st.m_run[i];
-      rec[1] = l * unscale;
+      rec[1] = seen && st.m_run[i] == -INFINITY ? kNoWeight : l * unscale;
     }
     float o[NC];
 #pragma unroll
@@ -1081,7 +1093,12 @@ bool tiles_take_run(const dkv_decode_args& a, int group) {
          ((group >= 8 && a.fast_key_bits < 8) || a.B * a.Hkv * a.fast_count >= 2048);
 }
 
-int launch_tile_run(const DecodeParams& d, int first, int count, int splits, const TileLayout& g, hipStream_t s) {
+int tile_items(int count, int n_dense, int64_t dense_tokens) {
+  return (int)std::min<int64_t>(INT32_MAX, count + n_dense * ((dense_tokens + kPiece - 1) / kPiece));
+}
+
+int launch_tile_run(const DecodeParams& d, int first, int count, int n_dense, int splits, const TileLayout& g,
+                    hipStream_t s) {
   const dkv_decode_args& a = d.a;
   DKV_CHECK(a.B * a.Hkv * splits < (int64_t)1 << 31, DKV_ERR_UNSUPPORTED, "too many splits for one launch");
   TileParams p;
@@ -1089,6 +1106,7 @@ int launch_tile_run(const DecodeParams& d, int first, int count, int splits, con
   p.splits = splits;
   p.packed_first = first;
   p.n_packed = count;
+  p.n_dense = n_dense;
   p.key_group = g.key_group;
   p.value_group = g.value_group;
   p.promoted = g.promoted;
@@ -1111,11 +1129,13 @@ bool tiles_take_rest(const DecodeParams& d, TileRest* rest) {
     return i >= n_rest ? a.tail : a.segments_host[i < d.skip_first ? i : i + d.skip_count];
   };
   // one run of packed segments of one layout, everything else dense
-  *rest = TileRest{0, 0, TileLayout{2, 128, 64, 0}};  // (without packed segments the layout is not used)
+  int most = 0;  // tokens of a dense entry
+  *rest = TileRest{0, 0, 0, 0, TileLayout{2, 128, 64, 0}};  // (without packed segments the layout is not used)
   for (int i = 0; i < d.n_total; ++i) {
     const dkv_segment& g = entry(i);
     if (g.key_kind == DKV_KEY_DENSE) {
       if (!dense_ok(g)) return false;
+      most = std::max(most, g.tokens);
       continue;
     }
     if (i >= n_rest || !packed_ok(g, (int)a.D)) return false;
@@ -1128,6 +1148,8 @@ bool tiles_take_rest(const DecodeParams& d, TileRest* rest) {
     }
     ++rest->count;
   }
+  rest->n_dense = d.n_total - rest->count;
+  rest->items = tile_items(rest->count, rest->n_dense, most);
   return true;
 }
 

@@ -36,19 +36,23 @@ int launch_uniform_decode(const dkv_decode_args& a, int first, int count, int kb
                           int split_stride, hipStream_t stream, const FusedRest* fused = nullptr);
 // Whether the tile kernel takes a call's page run instead of the page kernels
 // (the run is as dkv_decode_args guarantees), and its launch over `count`
-// packed entries from `first` on and the dense entries around them (d.n_total
-// in all, none skipped), writing `splits` records from d.split_offset on.
+// packed entries from `first` on and the n_dense dense entries around them (none
+// skipped), writing `splits` records from d.split_offset on.  d.n_total is the
+// number of work items: tile_items of those and of the most tokens that a dense
+// entry holds.
 struct TileLayout {
   int bits, key_group, value_group, promoted;  // promoted 0: uniform pages
 };
 bool tiles_take_run(const dkv_decode_args& a, int group);
-int launch_tile_run(const DecodeParams& d, int first, int count, int splits, const TileLayout& g, hipStream_t stream);
+int tile_items(int count, int n_dense, int64_t dense_tokens);
+int launch_tile_run(const DecodeParams& d, int first, int count, int n_dense, int splits, const TileLayout& g,
+                    hipStream_t stream);
 
 // Whether the tile kernel reads the segments of a decode call outside the page
 // kernels' run (checked on the host copies of the descriptors): `count` packed
 // ones of one layout from entry `first` of the rest on, the others dense.
 struct TileRest {
-  int first, count;
+  int first, count, n_dense, items;
   TileLayout layout;
 };
 bool tiles_take_rest(const DecodeParams& d, TileRest* rest);

@@ -263,6 +263,11 @@ __device__ __forceinline__ void dense_chunk(const DecodeParams& p, int chunks, i
   }
 }
 
+// The weight sum of a record whose split has tokens, all of them with a logit of
+// minus infinity (its maximum is minus infinity too): it adds nothing beside
+// other records, and alone it makes the result NaN, as softmax does.
+constexpr float kNoWeight = -1.f;
+
 // Combine the split records of query heads kvh * G + h (h < G) of batch b with
 // the log-sum-exp rule, then out = acc / max(sum, 1e-20) (attention.py:86).
 // Same arithmetic and summation order for every thread count: per head, the
@@ -297,8 +302,12 @@ __device__ __forceinline__ void merge_heads(const DecodeParams& p, int b, int hq
     const float* w = wgt + tid * S;
     const float* l = lsum + tid * S;
     float L = 0.f;
-    for (int s = 0; s < S; ++s) L += l[s] * w[s];
-    den[tid] = fmaxf(L, 1e-20f);
+    bool none = false;
+    for (int s = 0; s < S; ++s) {
+      L += l[s] * w[s];
+      none |= l[s] == kNoWeight;
+    }
+    den[tid] = mx[tid] == -INFINITY && none ? NAN : fmaxf(L, 1e-20f);
   }
   sync();
   for (int i = tid; i < G * D; i += nt) {

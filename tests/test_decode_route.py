@@ -99,3 +99,16 @@ def test_page_runs():
     assert _route(_args([dart16] * 4 + [_page(key="dart", promoted=32, tokens=40)], run=(0, 4))) == ("pages", "tiles")
     other = _page(bits=4, value_bits=2)
     assert _route(_args([other] * 64, B=64, G=8, run=(0, 64))) == ("pages", "none")  # two code widths
+
+
+def test_dense_entries_come_in_pieces():
+    """Work items of the tile kernel: the packed segments, and 128-token pieces of the longest dense entry for each."""
+    pages = [_page(kgroup=64)] * 5
+
+    def units(a):
+        return _lib.decode_kernels(a).rest_units
+    assert units(_args(pages)) == 5
+    assert units(_args([_dense(32)] + pages, tail=_dense(128))) == 5 + 2
+    assert units(_args([_dense(32)] + pages, tail=_dense(129))) == 5 + 2 * 2
+    assert units(_args([_dense(1 << 19)], tail=_dense(1))) == 2 * (1 << 12)
+    assert units(_args([_dense(4000)] + pages, dtype=F32)) == 6  # the general kernel takes whole segments

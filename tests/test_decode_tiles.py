@@ -340,3 +340,58 @@ def test_infinite_key_under_a_query_of_another_type(dtype, q_dtype):
     assert _route(q, cache) == ("tiles", "tiles")
     dart.decode_attention(q.to(DEV), cache, out_f32=out)
     assert _rel_err(out.unsqueeze(2), ref) <= 1e-5
+
+
+@pytest.mark.parametrize("G,T,dtype,n_splits,fast,cfg", [
+    (6, 1400, BF, None, None, dict(promote_ratio=0.25, sink_tokens=300, local_tokens=500)),
+    (6, 1400, FP, 3, None, dict(promote_ratio=0.25, sink_tokens=129, local_tokens=257)),   # pieces of one token
+    (3, 1000, FP, 64, False, dict(key_group_size=64, local_tokens=700)),
+    (4, 900, BF, None, False, dict(key_group_size=64, sink_tokens=900)),                   # dense pieces only
+    (16, 1700, BF, None, True, dict(promote_ratio=0.25, local_tokens=600)),                # beside a page run
+    (16, 1700, FP, 2, True, dict(promote_ratio=0.25, local_tokens=600, sink_tokens=256)),
+    (8, 1700, BF, None, True, dict(bits=4, local_tokens=600)),
+    (8, 1700, FP, 5, True, dict(bits=2, local_tokens=384, sink_tokens=0)),
+])
+def test_long_dense_windows_in_pieces(G, T, dtype, n_splits, fast, cfg):
+    import dartkv_amd as dart
+    from dartkv_amd import synthetic
+    from oracle import dart_oracle as O
+    cfg = dict(dict(bits=2, page_size=128, key_group_size=128, value_group_size=64, sink_tokens=32,
+                    hold_partial_pages=True, metadata_dtype=torch.float16), **cfg)
+    k, v, q = synthetic.outlier_kv(2, 2, T, 128, query_heads=2 * G, dtype=dtype, seed=T + G)
+    oc, cache = O.OracleCache(O.OracleConfig(**cfg)), dart.DartKVCache(dart.DartKVCacheConfig(**cfg))
+    oc.append(k, v)
+    cache.append(k.to(DEV), v.to(DEV))
+    ref = O.streamed_attention(q, oc, return_fp32=True)[1]
+    out = torch.empty(2, 2 * G, 128, dtype=torch.float32, device=DEV)
+    print("case", G, T, dtype, n_splits, fast, cfg, flush=True)
+    run, rest = _route(q, cache, n_splits=n_splits, fast=fast)
+    assert rest == "tiles" and run == ("tiles" if fast else "none")
+    dart.decode_attention(q.to(DEV), cache, out_f32=out, n_splits=n_splits, fast=fast)
+    assert _rel_err(out.unsqueeze(2), ref) <= 1e-5
+
+
+@pytest.mark.parametrize("dtype", [BF, FP])
+@pytest.mark.parametrize("n_splits", [None, 1, 40])
+def test_logits_of_minus_infinity(dtype, n_splits):
+    """Tokens with a logit of minus infinity have no weight, also where they are a whole piece and split of their own;
+    where every token is one, the result is NaN."""
+    import dartkv_amd as dart
+    g = torch.Generator().manual_seed(9)
+    k, v = (torch.randn(1, 2, 260, 64, generator=g).to(dtype) for _ in range(2))
+    q = torch.randn(1, 6, 1, 64, generator=g).to(dtype)
+    q[..., 7] = 1.0
+    k[..., 256:, 7] = float("-inf")
+    cfg = dict(bits=2, page_size=128, key_group_size=64, value_group_size=32, sink_tokens=400, hold_partial_pages=True)
+    for first in (0, 256):
+        cache = dart.DartKVCache(dart.DartKVCacheConfig(**cfg))
+        cache.append(k[..., first:, :].to(DEV), v[..., first:, :].to(DEV))
+        assert _route(q, cache, n_splits=n_splits) == ("none", "tiles")
+        print("case", dtype, n_splits, first, flush=True)
+        got = dart.decode_attention(q.to(DEV), cache, n_splits=n_splits).cpu().double()
+        logits = torch.matmul(q.double().view(1, 2, 3, 64), k[..., first:, :].double().transpose(-1, -2)) / 8.0
+        ref = torch.matmul(torch.softmax(logits, -1), v[..., first:, :].double()).view(1, 6, 1, 64)
+        if first:
+            assert torch.isnan(ref).all() and torch.isnan(got).all()
+        else:
+            assert float((got - ref).norm() / ref.norm()) <= (4e-3 if dtype == BF else 5e-4)  # the output's rounding
