@@ -58,7 +58,7 @@ def default_splits(batch: int, kv_heads: int, n_segments: int, target: int = 409
 
 # Workers of the tile kernel (16-bit caches outside the page kernels' forms): one wave each, 2,048 resident.
 # Measured with 64 (batch, kv head) pairs x 62 pages, six heads per KV head: 36.5 µs with 2,048 waves, 42.7 with
-# 4,096 and 44.8 with 1,024; 128 pairs x 256 pages: 188, 194 and 291.
+# 4,096 and 44.8 with 1,024; 128 pairs x 256 pages: 188, 194 and 291.  The general kernel keeps its 4,096.
 TILE_WORKERS = 2048
 
 
@@ -137,10 +137,7 @@ def _call_layout(plan, cache: DartKVCache, q3: torch.Tensor, kv_heads: int, head
         fast_splits = max(1, min(fast_splits, units))
         splits = rest * -(-dense_tokens // 32) if dense_tokens else (max(1, min(rest, 4)) if rest else 0)
     else:
-        fast_splits = 0
-        tiles = cache.dtype in (torch.bfloat16, torch.float16) and head_dim in (64, 128)
-        splits = n_splits or default_splits(batch, kv_heads, rest, TILE_WORKERS if tiles else 4096)
-        splits = max(1, min(splits, max(1, rest)))
+        fast_splits = splits = 0
     a = _lib.DecodeArgs()
     a.q_dtype = _lib.dtype_code(q3.dtype)
     a.q_sb, a.q_sh = q3.stride(0), q3.stride(1)
@@ -151,6 +148,15 @@ def _call_layout(plan, cache: DartKVCache, q3: torch.Tensor, kv_heads: int, head
     a.cache_dtype = _lib.dtype_code(cache.dtype)
     a.meta_dtype = _lib.dtype_code(cache.config.metadata_dtype)
     a.scale = float(factor)
+    if not fast_count:
+        a.tail = tail
+        kernels = _lib.decode_kernels(a)
+        units = max(1, kernels.rest_units)
+        target = TILE_WORKERS if kernels.rest == _lib.KERNEL_TILES else 4096
+        splits = max(1, min(n_splits or default_splits(batch, kv_heads, units, target), units))
+        if splits > rest:  # (pieces of long dense windows: no more records than the static scratch holds)
+            scratch = _lib.load().dkv_decode_scratch_bytes()
+            splits = max(rest, min(splits, scratch // _lib.load().dkv_decode_workspace_bytes(batch, Hq, head_dim, 1)))
     a.n_splits = splits
     a.workspace_bytes = _lib.load().dkv_decode_workspace_bytes(batch, Hq, head_dim, splits + fast_splits)
     if fast_count:

@@ -395,3 +395,22 @@ def test_logits_of_minus_infinity(dtype, n_splits):
             assert torch.isnan(ref).all() and torch.isnan(got).all()
         else:
             assert float((got - ref).norm() / ref.norm()) <= (4e-3 if dtype == BF else 5e-4)  # the output's rounding
+
+
+@pytest.mark.parametrize("dtype,q_dtype,cfg,kernel,splits", [
+    (BF, BF, dict(key_group_size=64), "tiles", 16),
+    (BF, torch.float32, dict(key_group_size=64), "general", 32),
+    (BF, BF, dict(key_group_size=64, metadata_dtype=BF), "general", 32),
+    (FP, FP, dict(page_size=80, key_group_size=40), "general", 32),
+    (FP, FP, dict(key_group_size=64, sink_tokens=4000), "tiles", 16),  # pieces of one dense segment
+])
+def test_split_counts_of_the_kernel_that_runs(dtype, q_dtype, cfg, kernel, splits):
+    """2,048 waves of the tile kernel, 4,096 workgroups of the general kernel (128 batch-head pairs)."""
+    import dartkv_amd as dart
+    from dartkv_amd.attention import _prepare_call
+    k = torch.randn(16, 8, 4000, 64, device=DEV).to(dtype)
+    cache = dart.DartKVCache(dart.DartKVCacheConfig(bits=2, value_group_size=32, hold_partial_pages=True, **cfg))
+    cache.append(k, k)
+    q = torch.randn(16, 8, 1, 64, device=DEV).to(q_dtype)
+    assert _route(q, cache) == ("none", kernel)
+    assert _prepare_call(q, cache, None, None, None, False)[3][0].n_splits == splits
