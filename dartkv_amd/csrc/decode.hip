@@ -111,7 +111,7 @@ __global__ void __launch_bounds__(kThreads) decode_split_general(DecodeParams p)
           }
         } else {
           for (int c = 0; c < D; ++c) {
-            const float kv = key_value(seg, bh, c, t, D, seg.key_kind == DKV_KEY_MIXED ? inv_s[c] : -1, cache_dt, meta);
+            const float kv = key_value(seg, bh, c, t, D, inv_s, cache_dt, meta);
             DKV_FOR_HEAD(h) logit[h] = fmaf(q_s[h * D + c], kv, logit[h]);
           }
         }

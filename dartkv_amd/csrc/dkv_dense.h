@@ -83,23 +83,53 @@ __device__ __forceinline__ PackedElem value_code(const dkv_segment& s, int64_t b
 }
 
 // The same elements of a segment of any kind, dequantized with the reference's
-// chain, as fp32.
-__device__ __forceinline__ float key_value(const dkv_segment& s, int64_t bh, int c, int t, int D, int slot,
+// chain, as fp32.  Written out for the general decode kernel's loops: through
+// PackedElem above it ran 4 % longer (16 x 16,000 tokens: 4,635 -> 4,824 µs).
+// inv: slot of each channel among the promoted ones of a Dart page.
+__device__ __forceinline__ float key_value(const dkv_segment& s, int64_t bh, int c, int t, int D, const int32_t* inv,
                                            int cache_dt, int meta) {
-  if (s.key_kind == DKV_KEY_DENSE)
+  if (s.key_kind == DKV_KEY_DENSE) {
     return dev_load((const void*)s.key[0], bh * s.key_bh[0] + (int64_t)t * D + c, cache_dt);
-  const PackedElem e = key_code(s, bh, c, t, D, slot);
-  return dev_dequant(e.code, dev_load_meta(e.scale, bh * s.key_bh[3] + e.at, meta),
-                     dev_load_meta(e.zero, bh * s.key_bh[4] + e.at, meta), meta, cache_dt);
+  }
+  const int kg = s.key_group;
+  const int G = (s.tokens + kg - 1) / kg;
+  const int g = t / kg;
+  uint32_t code;
+  if (s.key_kind == DKV_KEY_UNIFORM) {
+    const int per_byte = 8 / s.key_bits;
+    const int pk = (G * kg + per_byte - 1) / per_byte;
+    const uint8_t byte = ((const uint8_t*)s.key[0])[bh * s.key_bh[0] + (int64_t)c * pk + t / per_byte];
+    code = (byte >> ((t % per_byte) * s.key_bits)) & ((1u << s.key_bits) - 1u);
+  } else {
+    const int nb = (kg + 3) / 4;
+    const int w = t % kg;
+    const uint8_t lo = ((const uint8_t*)s.key[0])[bh * s.key_bh[0] + ((int64_t)c * G + g) * nb + w / 4];
+    code = (lo >> ((w % 4) * 2)) & 3u;
+    const int slot = inv[c];
+    if (slot >= 0) {
+      const uint8_t hi = ((const uint8_t*)s.key[1])[bh * s.key_bh[1] + ((int64_t)slot * G + g) * nb + w / 4];
+      code |= ((hi >> ((w % 4) * 2)) & 3u) << 2;
+    }
+  }
+  const int64_t mi = (int64_t)c * G + g;
+  return dev_dequant(code, dev_load_meta((const void*)s.key[3], bh * s.key_bh[3] + mi, meta),
+                     dev_load_meta((const void*)s.key[4], bh * s.key_bh[4] + mi, meta), meta, cache_dt);
 }
 
 __device__ __forceinline__ float value_value(const dkv_segment& s, int64_t bh, int t, int c, int D, int cache_dt,
                                              int meta) {
-  if (s.value_kind == DKV_VALUE_DENSE)
+  if (s.value_kind == DKV_VALUE_DENSE) {
     return dev_load((const void*)s.value[0], bh * s.value_bh[0] + (int64_t)t * D + c, cache_dt);
-  const PackedElem e = value_code(s, bh, t, c, D);
-  return dev_dequant(e.code, dev_load_meta(e.scale, bh * s.value_bh[1] + e.at, meta),
-                     dev_load_meta(e.zero, bh * s.value_bh[2] + e.at, meta), meta, cache_dt);
+  }
+  const int vg = s.value_group;
+  const int Gv = (D + vg - 1) / vg;
+  const int per_byte = 8 / s.value_bits;
+  const int pv = (Gv * vg + per_byte - 1) / per_byte;
+  const uint8_t byte = ((const uint8_t*)s.value[0])[bh * s.value_bh[0] + (int64_t)t * pv + c / per_byte];
+  const uint32_t code = (byte >> ((c % per_byte) * s.value_bits)) & ((1u << s.value_bits) - 1u);
+  const int64_t mi = (int64_t)t * Gv + c / vg;
+  return dev_dequant(code, dev_load_meta((const void*)s.value[1], bh * s.value_bh[1] + mi, meta),
+                     dev_load_meta((const void*)s.value[2], bh * s.value_bh[2] + mi, meta), meta, cache_dt);
 }
 
 constexpr int kDenseWaves = 4;
