@@ -168,45 +168,17 @@ def _call_layout(plan, cache: DartKVCache, q3: torch.Tensor, kv_heads: int, head
     return a, a.workspace_bytes
 
 
-def _prepare_call(query: torch.Tensor, cache: DartKVCache, scale: Optional[float], n_splits: Optional[int],
-                  fast: Optional[bool], static_scratch: bool):
-    """A decode call's checked parts: the query as [B, Hq, D], the plan, the tail's descriptor, and the call's layout
-    (argument template, workspace bytes)."""
-    _lib.require_device(query)
-    _, kv_heads, head_dim = _check_query(query, cache)
-    # q3: the query as [B, Hq, D] (a [B, Hq, 1, D] query is read through its own strides 0, 1 and 3)
-    q3 = query.reshape(query.shape[0], query.shape[1], query.shape[-1]) if query.ndim == 4 and query.shape[2] != 1 \
-        else query
-    if q3.stride(-1) != 1:
-        q3 = q3.contiguous()
-    device = query.device
-    if device != cache.device:
-        raise ValueError("query and cache must be on the same device")
-    factor = scale if scale is not None else 1.0 / math.sqrt(head_dim)
-    plan = cache.decode_plan(device)
-    if plan.tail_is_pending:
-        tail, dense_ok = tail_segment(cache, with_dense_check=True)
-    else:
-        tail, dense_ok = _NO_TAIL, True
-    Hq = q3.shape[1]
-    use_fast = ((_fast_enabled() if fast is None else fast) and plan.fast_count > 0
-                and Hq // kv_heads in _fast_rows(plan))
-    chunks = -(-max(plan.rest_dense, tail.tokens) // 32)
-    key = (Hq, q3.dtype, q3.stride(0), q3.stride(1), use_fast, n_splits, factor, static_scratch, tail.tokens > 0,
-           dense_ok, chunks)
-    layout = plan.call_layouts.get(key)
-    if layout is None:
-        layout = plan.call_layouts[key] = _call_layout(plan, cache, q3, kv_heads, head_dim, tail, use_fast, dense_ok,
-                                                       n_splits, factor)
-    return q3, plan, tail, layout
-
-
-def decode_route(query: torch.Tensor, cache: DartKVCache, *, scale: Optional[float] = None,
-                 n_splits: Optional[int] = None, fast: Optional[bool] = None) -> Tuple[str, str]:
+def decode_route(query: torch.Tensor, cache: DartKVCache, *, n_splits: Optional[int] = None,
+                 fast: Optional[bool] = None) -> Tuple[str, str]:
     """The kernels ``decode_attention`` runs these arguments on: one for the page run, one for the other entries
     ("none", "pages", "tiles", "dense" or "general")."""
-    _, _, tail, (template, _) = _prepare_call(query, cache, scale, n_splits, fast, False)
-    a = _lib.DecodeArgs.from_buffer_copy(template)
+    plan = cache.decode_plan(query.device)
+    kv_heads, head_dim = cache.shape[1], cache.shape[3]
+    q3 = query.reshape(query.shape[0], query.shape[1], head_dim)
+    tail, dense_ok = tail_segment(cache, with_dense_check=True) if plan.tail_is_pending else (_NO_TAIL, True)
+    use_fast = ((_fast_enabled() if fast is None else fast) and plan.fast_count > 0
+                and q3.shape[1] // kv_heads in _fast_rows(plan))
+    a, _ = _call_layout(plan, cache, q3, kv_heads, head_dim, tail, use_fast, dense_ok, n_splits, 1.0)
     a.tail = tail
     kernels = _lib.decode_kernels(a)
     names = ("none", "pages", "tiles", "dense", "general")
@@ -234,8 +206,33 @@ def decode_attention(query: torch.Tensor, cache: DartKVCache, *, scale: Optional
     device scratch (``dkv_decode_attention_noalloc``) instead of a workspace
     tensor, so with ``out`` given the call allocates nothing.
     """
-    q3, plan, tail, (template, ws_bytes) = _prepare_call(query, cache, scale, n_splits, fast, static_scratch)
-    batch, Hq, head_dim, device = q3.shape[0], q3.shape[1], q3.shape[-1], query.device
+    _lib.require_device(query)
+    batch, kv_heads, head_dim = _check_query(query, cache)
+    # q3: the query as [B, Hq, D] (a [B, Hq, 1, D] query is read through its own strides 0, 1 and 3)
+    q3 = query.reshape(query.shape[0], query.shape[1], query.shape[-1]) if query.ndim == 4 and query.shape[2] != 1 \
+        else query
+    if q3.stride(-1) != 1:
+        q3 = q3.contiguous()
+    device = query.device
+    if device != cache.device:
+        raise ValueError("query and cache must be on the same device")
+    factor = scale if scale is not None else 1.0 / math.sqrt(head_dim)
+    plan = cache.decode_plan(device)
+    if plan.tail_is_pending:
+        tail, dense_ok = tail_segment(cache, with_dense_check=True)
+    else:
+        tail, dense_ok = _NO_TAIL, True
+    Hq = q3.shape[1]
+    use_fast = ((_fast_enabled() if fast is None else fast) and plan.fast_count > 0
+                and Hq // kv_heads in _fast_rows(plan))
+    chunks = -(-max(plan.rest_dense, tail.tokens) // 32)
+    key = (Hq, q3.dtype, q3.stride(0), q3.stride(1), use_fast, n_splits, factor, static_scratch, tail.tokens > 0,
+           dense_ok, chunks)
+    layout = plan.call_layouts.get(key)
+    if layout is None:
+        layout = plan.call_layouts[key] = _call_layout(plan, cache, q3, kv_heads, head_dim, tail, use_fast, dense_ok,
+                                                       n_splits, factor)
+    template, ws_bytes = layout
     if out is None:
         out = torch.empty(batch, Hq, 1, head_dim, dtype=query.dtype, device=query.device)
     elif out.shape != (batch, Hq, 1, head_dim) or out.dtype != query.dtype or out.device != query.device \

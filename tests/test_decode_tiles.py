@@ -407,10 +407,11 @@ def test_logits_of_minus_infinity(dtype, n_splits):
 def test_split_counts_of_the_kernel_that_runs(dtype, q_dtype, cfg, kernel, splits):
     """2,048 waves of the tile kernel, 4,096 workgroups of the general kernel (128 batch-head pairs)."""
     import dartkv_amd as dart
-    from dartkv_amd.attention import _prepare_call
     k = torch.randn(16, 8, 4000, 64, device=DEV).to(dtype)
     cache = dart.DartKVCache(dart.DartKVCacheConfig(bits=2, value_group_size=32, hold_partial_pages=True, **cfg))
     cache.append(k, k)
     q = torch.randn(16, 8, 1, 64, device=DEV).to(q_dtype)
     assert _route(q, cache) == ("none", kernel)
-    assert _prepare_call(q, cache, None, None, None, False)[3][0].n_splits == splits
+    dart.decode_attention(q, cache)
+    (template, _), = cache.decode_plan(q.device).call_layouts.values()
+    assert template.n_splits == splits
