@@ -631,14 +631,6 @@ extern "C" int dkv_decode_attention(const dkv_decode_args* args, void* stream) {
   }
   bool run_done = false;
   if (fast_count > 0 && dkv::tiles_take_run(a, p.group)) {
-    // The tile kernel takes the run: sixteen rows per KV head on Dart pages,
-    // and uniform pages of one width where the launch fills the device or has
-    // eight rows (one layer with its merge, MI355X, tile against page kernel: sixteen
-    // rows, 8 x 8 heads x 64 pages: 38 against 71 µs; 16 x 8 x 256 pages at 2 bits: 119
-    // against 172 µs; 16 x 8 x 128 pages at 4 bits, four rows: 94 against 99, eight rows:
-    // 105 against 127 µs, at 8 bits 148 against 156; one sequence x 8 heads x 8 pages:
-    // four rows at 2 bits 15.6 against 14.3 µs, eight rows at 2 bits 14.7 against 17.8,
-    // at 8 bits 19.1 against 17.9).
     DecodeParams t = p;
     t.skip_first = t.skip_count = 0;
     const bool all = rest == 0 || dense_rest;  // the dense pieces ride in the same launch

@@ -1088,10 +1088,32 @@ int launch_tiles_heads(TileParams& p, int bits, bool mixed, hipStream_t s) {
 
 namespace dkv {
 
+// Both sides measured, one layer with its merge (tile | page kernel, MI355X):
+// * Dart pages, sixteen rows (the page kernel has no such form any more): 8 x 8
+//   heads x 64 pages 38 | 71 µs.  Up to eight rows they stay with the page kernel.
+// * Uniform pages of one code width, eight rows: 16 x 8 heads x 128 pages 102 |
+//   128 µs at 4 bits, x 64 pages 43 | 69 at 2 bits, 86 | 113 at 8 bits; one
+//   sequence x 8 pages at 2 bits 14.1 | 17.5, at 8 bits 19.1 | 17.9.
+// * Fewer rows, where the launch fills the device.  The page kernel's work grows
+//   with the rows, the tile kernel's hardly does, and its bf16 rounding chain
+//   is the dearer one.  2 bits: one row, 16 x 8 x 64 pages 40 | 48, but 16 pages
+//   (every wave has one, and the dense pieces start a second round of waves) 23 |
+//   21; four rows 25 | 26.  4 bits: value groups of 32 channels 26 | 30 and up to
+//   1.5 times there; else fp16 with two rows 46 | 48, four rows 46 | 50, bf16 with
+//   four rows 55 | 51.  8 bits: bf16 with two rows 84 | 86, with one 83 | 81;
+//   fp16 with four rows 78 | 75, but 24 pages 36 | 40.
 bool tiles_take_run(const dkv_decode_args& a, int group) {
   if (a.fast_promoted > 0) return group == 16;
-  return a.q_dtype == a.cache_dtype && a.fast_key_bits == a.fast_value_bits && 128 / a.fast_value_group <= kMaxGroups &&
-         ((group >= 8 && a.fast_key_bits < 8) || a.B * a.Hkv * a.fast_count >= 2048);
+  if (a.q_dtype != a.cache_dtype || a.fast_key_bits != a.fast_value_bits || 128 / a.fast_value_group > kMaxGroups)
+    return false;
+  const int64_t pages = a.B * a.Hkv * a.fast_count, bits = a.fast_key_bits;
+  constexpr int64_t kFull = 2048;  // waves the device holds
+  if (group >= 8) return bits < 8 || pages >= kFull;
+  if (pages < kFull) return false;
+  const bool bf = a.cache_dtype == kBF16, more = pages > kFull;
+  if (bits == 2) return group == 4 || more;
+  if (bits == 4) return a.fast_value_group == 32 || (!bf && (group == 4 || (group == 2 && more)));
+  return group >= 2 && (bf || pages <= kFull * 3 / 2);
 }
 
 int tile_items(int count, int n_dense, int64_t dense_tokens) {

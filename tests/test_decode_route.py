@@ -112,3 +112,18 @@ def test_dense_entries_come_in_pieces():
     assert units(_args([_dense(32)] + pages, tail=_dense(129))) == 5 + 2 * 2
     assert units(_args([_dense(1 << 19)], tail=_dense(1))) == 2 * (1 << 12)
     assert units(_args([_dense(4000)] + pages, dtype=F32)) == 6  # the general kernel takes whole segments
+
+
+@pytest.mark.parametrize("bits,dtype,G,pages,vgroup,run", [
+    # eight rows: 2 and 4 bits always, 8 bits where the launch fills the device (2,048 pages of all heads)
+    (2, BF, 8, 1, 64, "tiles"), (4, FP, 8, 1, 128, "tiles"), (8, BF, 8, 255, 64, "pages"), (8, FP, 8, 256, 64, "tiles"),
+    (2, BF, 4, 255, 64, "pages"), (2, FP, 4, 256, 64, "tiles"), (2, BF, 2, 256, 64, "pages"), (2, BF, 1, 257, 128, "tiles"),
+    (4, BF, 4, 4096, 64, "pages"), (4, BF, 1, 256, 32, "tiles"), (4, BF, 1, 255, 32, "pages"),
+    (4, FP, 4, 256, 64, "tiles"), (4, FP, 2, 256, 64, "pages"), (4, FP, 2, 257, 128, "tiles"), (4, FP, 1, 999, 64, "pages"),
+    (8, BF, 2, 256, 64, "tiles"), (8, BF, 1, 999, 64, "pages"), (8, FP, 4, 384, 64, "tiles"), (8, FP, 4, 385, 64, "pages"),
+    (8, FP, 1, 256, 64, "pages"),
+    (2, BF, 8, 999, 16, "pages"),  # eight value groups: the page kernel only
+])
+def test_uniform_page_runs(bits, dtype, G, pages, vgroup, run):
+    a = _args([_page(bits=bits, vgroup=vgroup)] * pages, B=1, H=8, G=G, dtype=dtype, run=(0, pages))
+    assert _route(a) == (run, "none")
