@@ -562,9 +562,12 @@ class DartKVCache:
     def get(self) -> Tuple[torch.Tensor, torch.Tensor]:
         if self._seen_tokens == 0:
             raise RuntimeError("DartKVCache is empty; call update() before get()")
-        dense = self._materialize_all()
-        if dense is not None:
-            return dense
+        for segment in self._keys:
+            if not isinstance(segment, torch.Tensor):  # packed pages
+                dense = self._materialize_all()
+                if dense is not None:
+                    return dense
+                break
         keys = [_materialize(s) for s in self._keys]
         values = [_materialize(s) for s in self._values]
         if self._pending_key is not None:
