@@ -16,6 +16,7 @@ from . import _lib
 from .finite import drain, nonfinite_flags
 
 _SUPPORTED_BITS = (2, 4, 8)
+_METADATA_DTYPES = (torch.float16, torch.bfloat16, torch.float32, torch.float64)
 
 
 def _validate_bits(bits: int) -> None:
@@ -26,7 +27,7 @@ def _validate_bits(bits: int) -> None:
 def _metadata_dtype(data: torch.Tensor, requested: Optional[torch.dtype]) -> torch.dtype:
     """reference quantization.py:48-53."""
     if requested is not None:
-        if requested not in (torch.float16, torch.bfloat16, torch.float32, torch.float64):
+        if requested not in _METADATA_DTYPES:
             raise TypeError(f"metadata dtype must be floating point, got {requested}")
         return requested
     return data.dtype if data.dtype in (torch.float16, torch.bfloat16) else torch.float32
@@ -162,7 +163,7 @@ def quantize(
     # the kernels report non-finite values themselves; checked ahead where another error would come first
     # or none of their launches runs
     ahead = (bad_axis or data.device.type != "cuda" or data.dtype not in _lib.FLOAT_DTYPES or data.numel() == 0
-             or torch.cuda.is_current_stream_capturing())
+             or metadata_dtype not in (None, *_METADATA_DTYPES) or torch.cuda.is_current_stream_capturing())
     if ahead:
         _check_finite(data, message)
     if bad_axis:

@@ -112,3 +112,16 @@ def test_quantize_rejects_non_finite_values(bad, axis):
         dart.quantize(x.to(DEV), bits=4, group_size=64, axis=axis)
     x[1, 1, 129, 63] = 0.0
     dart.quantize(x.to(DEV), bits=4, group_size=64, axis=axis)  # the report is cleared
+
+
+def test_non_finite_input_is_reported_before_a_bad_metadata_type():
+    """The reference's order of checks (non-finite values first, src/dart/quantization.py:159-160): both faults at once raise ValueError."""
+    import dartkv_amd as dart
+    x = torch.ones(4, 64, device="cuda")
+    x[1, 3] = float("nan")
+    with pytest.raises(ValueError, match="finite"):
+        dart.quantize(x, bits=4, group_size=32, metadata_dtype=torch.int8)
+    with pytest.raises(TypeError, match="metadata dtype"):
+        dart.quantize(torch.ones(4, 64, device="cuda"), bits=4, group_size=32, metadata_dtype=torch.int8)
+    with pytest.raises(ValueError, match="finite"):
+        dart.quantize(x, bits=4, group_size=32)
