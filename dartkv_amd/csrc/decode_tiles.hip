@@ -1090,18 +1090,24 @@ namespace dkv {
 
 // Both sides measured, one layer with its merge (tile | page kernel, MI355X):
 // * Dart pages, sixteen rows (the page kernel has no such form any more): 8 x 8
-//   heads x 64 pages 38 | 71 µs.  Up to eight rows they stay with the page kernel.
-// * Uniform pages of one code width, eight rows: 16 x 8 heads x 128 pages 102 |
-//   128 µs at 4 bits, x 64 pages 43 | 69 at 2 bits, 86 | 113 at 8 bits; one
-//   sequence x 8 pages at 2 bits 14.1 | 17.5, at 8 bits 19.1 | 17.9.
+//   heads x 64 pages 37 | 71 µs.  Up to four rows the page kernel, whose staged
+//   pages serve every row, is the faster everywhere: four rows, 64 x 8 x 255
+//   pages 524 | 424, 16 x 8 x 64 51 | 40, one sequence x 8 pages 15.1 | 12.2; one
+//   row 521 | 393, 50 | 36, 14.8 | 12.9.  Eight rows are even (582 | 532, 55 | 53,
+//   15.1 | 16.6) and stay with it.
+// * Uniform pages of one code width, eight rows: 16 x 8 heads x 128 pages 104 |
+//   127 µs at 4 bits, 69 | 122 at 2 bits, 151 | 191 at 8 bits; one sequence x 8
+//   pages at 2 bits 14.1 | 17.5, at 8 bits 19.1 | 17.9.
 // * Fewer rows, where the launch fills the device.  The page kernel's work grows
-//   with the rows, the tile kernel's hardly does, and its bf16 rounding chain
-//   is the dearer one.  2 bits: one row, 16 x 8 x 64 pages 40 | 48, but 16 pages
-//   (every wave has one, and the dense pieces start a second round of waves) 23 |
-//   21; four rows 25 | 26.  4 bits: value groups of 32 channels 26 | 30 and up to
-//   1.5 times there; else fp16 with two rows 46 | 48, four rows 46 | 50, bf16 with
-//   four rows 55 | 51.  8 bits: bf16 with two rows 84 | 86, with one 83 | 81;
-//   fp16 with four rows 78 | 75, but 24 pages 36 | 40.
+//   with the rows, the tile kernel's hardly does; its bf16 rounding chain is the
+//   dearer one, and a launch pays for its prologue.  2 bits: one row, 64 x 8 x
+//   255 pages 400 | 637, 16 x 8 x 64 40 | 48, but 16 pages (every wave has one, and
+//   the dense pieces start a second round of waves) 23 | 21.  4 bits in value
+//   groups of 32 channels: 676 | 1,036, 26 | 30; else fp16 with one row 494 | 624,
+//   50 | 52, but 32 pages 31 | 30; bf16 with four rows 608 | 675, 16 x 8 x 128
+//   pages 95 | 98, but 64 pages 55 | 54, with one row 590 | 651, but 16 x 8 x 128
+//   93 | 90.  8 bits: bf16 with two rows 938 | 1,075, 84 | 87, with one 934 |
+//   1,041, but 64 pages 83 | 82; fp16 with four rows 913 | 871, but 24 pages 36 | 40.
 bool tiles_take_run(const dkv_decode_args& a, int group) {
   if (a.fast_promoted > 0) return group == 16;
   if (a.q_dtype != a.cache_dtype || a.fast_key_bits != a.fast_value_bits || 128 / a.fast_value_group > kMaxGroups)
@@ -1112,8 +1118,11 @@ bool tiles_take_run(const dkv_decode_args& a, int group) {
   if (pages < kFull) return false;
   const bool bf = a.cache_dtype == kBF16, more = pages > kFull;
   if (bits == 2) return group == 4 || more;
-  if (bits == 4) return a.fast_value_group == 32 || (!bf && (group == 4 || (group == 2 && more)));
-  return group >= 2 && (bf || pages <= kFull * 3 / 2);
+  if (bits == 4 && a.fast_value_group == 32) return true;
+  if (bits == 4 && bf) return pages >= (group == 4 ? 8 : 32) * kFull;
+  if (bits == 4) return group == 4 || (group == 2 && more) || pages >= 4 * kFull;
+  if (bf) return group >= 2 || pages >= 16 * kFull;
+  return group >= 2 && pages <= kFull * 3 / 2;
 }
 
 int tile_items(int count, int n_dense, int64_t dense_tokens) {

@@ -118,10 +118,12 @@ def test_dense_entries_come_in_pieces():
     # eight rows: 2 and 4 bits always, 8 bits where the launch fills the device (2,048 pages of all heads)
     (2, BF, 8, 1, 64, "tiles"), (4, FP, 8, 1, 128, "tiles"), (8, BF, 8, 255, 64, "pages"), (8, FP, 8, 256, 64, "tiles"),
     (2, BF, 4, 255, 64, "pages"), (2, FP, 4, 256, 64, "tiles"), (2, BF, 2, 256, 64, "pages"), (2, BF, 1, 257, 128, "tiles"),
-    (4, BF, 4, 4096, 64, "pages"), (4, BF, 1, 256, 32, "tiles"), (4, BF, 1, 255, 32, "pages"),
-    (4, FP, 4, 256, 64, "tiles"), (4, FP, 2, 256, 64, "pages"), (4, FP, 2, 257, 128, "tiles"), (4, FP, 1, 999, 64, "pages"),
-    (8, BF, 2, 256, 64, "tiles"), (8, BF, 1, 999, 64, "pages"), (8, FP, 4, 384, 64, "tiles"), (8, FP, 4, 385, 64, "pages"),
-    (8, FP, 1, 256, 64, "pages"),
+    (4, BF, 4, 2047, 64, "pages"), (4, BF, 4, 2048, 64, "tiles"), (4, BF, 2, 8191, 64, "pages"), (4, BF, 1, 8192, 128, "tiles"),
+    (4, BF, 1, 256, 32, "tiles"), (4, BF, 1, 255, 32, "pages"),
+    (4, FP, 4, 256, 64, "tiles"), (4, FP, 2, 256, 64, "pages"), (4, FP, 2, 257, 128, "tiles"),
+    (4, FP, 1, 1023, 64, "pages"), (4, FP, 1, 1024, 64, "tiles"),
+    (8, BF, 2, 256, 64, "tiles"), (8, BF, 1, 4095, 64, "pages"), (8, BF, 1, 4096, 64, "tiles"),
+    (8, FP, 4, 384, 64, "tiles"), (8, FP, 4, 385, 64, "pages"), (8, FP, 1, 256, 64, "pages"),
     (2, BF, 8, 999, 16, "pages"),  # eight value groups: the page kernel only
 ])
 def test_uniform_page_runs(bits, dtype, G, pages, vgroup, run):
