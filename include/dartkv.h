@@ -278,7 +278,8 @@ typedef struct dkv_segment {
  * fast_value_group channels (a multiple of 16 dividing 128), fp16 metadata and a
  * bf16 or fp16 cache, every field 16-byte aligned, and Hq / Hkv of 1, 2, 4,
  * 8 or 16; the caller guarantees this (except the head ratio, which is checked).
- * Those pages are processed by the MFMA page kernel (16 rows: the tile kernel)
+ * Those pages are processed by the MFMA page kernel (16 rows, and uniform runs
+ * that it is faster on: the tile kernel)
  * over `fast_splits` splits; the other entries and the tail by the tile or
  * general kernel over `n_splits` splits.
  * With fast_promoted == 0 the run is instead uniform pages: keys quantized
