@@ -1,9 +1,10 @@
 """The tile decode kernel (16-bit caches outside the page kernels' forms) against the oracle, at the edges of its
 tiles and of its dispatch.
 
-Its weights stay fp32 and its products are exact, so its error is that of fp32 logits and sums: a logit of size L
-carries about L 2^-24 (L below 50 here: 3e-6 relative in its weight) and the sums over at most 1,200 tokens the
-same order, under the 1e-5 that fp32 caches are held to.
+Its weights are fp32 (three 16-bit parts; in fp16 within three steps of 2^-37 of the largest) and its products exact,
+so its error is that of fp32 logits and sums: a logit of size L carries about L 2^-24 (L below 50 here: 3e-6 relative
+in its weight) and the sums over at most 1,700 tokens the same order, under the 1e-5 that fp32 caches are held to;
+test_small_weights_keep_their_bits has the long sums.
 """
 
 import pytest
