@@ -12,16 +12,17 @@
 // pieces beside them.  What it does not take (fp32 and float64 caches, other
 // metadata, odd group sizes) stays with decode_split_general.
 //
-// One wave owns one split, a contiguous range of segments of one (batch, kv
-// head), and walks it in tiles of TILE tokens (128, or 64 with 8-bit codes,
+// One wave owns one split, a contiguous range of work items (packed segments,
+// pieces of dense ones) of one (batch, kv head), and walks it in tiles of TILE tokens (128, or 64 with 8-bit codes,
 // whose registers a larger tile would not leave room for).
 //
 // Bound by VALU issue and by the latency between a tile's steps at two waves
-// per SIMD (140 to 256 VGPRs, no private memory: the build checks it), not by memory.  Against decode_split_general, which
-// spent about 100 VALU per element on scalar index arithmetic (one layer,
-// MI355X): 8 sequences x 4,096 tokens, 2-bit pages in groups of 64, fp16: 572
-// -> 19.8 µs; 8 x 8,011 tokens of Dart pages, six heads per KV head: 1,453 ->
-// 32.3 µs; 16 x 4,000 tokens of head_dim 64: 841 -> 29.1 µs.
+// per SIMD (three in a few forms; 151 to 256 VGPRs, no private memory: the build
+// checks it), not by memory.  Against decode_split_general, which spent about
+// 100 VALU per element on scalar index arithmetic (one layer, MI355X): 8
+// sequences x 4,096 tokens, 2-bit pages in groups of 64, fp16: 572 -> 19.8 µs; 8
+// x 8,011 tokens of Dart pages, six heads per KV head: 1,456 -> 32.9 µs; 16 x
+// 4,000 tokens of head_dim 64: 841 -> 24.5 µs.
 //
 // Layout.  Both products run on v_mfma_f32_16x16x32 with the query heads in
 // the 16 rows.  Codes are packed along tokens for keys and along channels for
