@@ -562,12 +562,13 @@ class DartKVCache:
     def get(self) -> Tuple[torch.Tensor, torch.Tensor]:
         if self._seen_tokens == 0:
             raise RuntimeError("DartKVCache is empty; call update() before get()")
-        for segment in self._keys:
-            if not isinstance(segment, torch.Tensor):  # packed pages
-                dense = self._materialize_all()
-                if dense is not None:
-                    return dense
-                break
+        # small dense pieces alone take two copies (61,440 elements of keys 10.1 against 12.4 µs, 1,228,800 elements
+        # 15.0 against 12.8, 33 million 165 against 48)
+        B, H, D = self._shape
+        if B * H * D * self._seen_tokens >= 1 << 20 or not all(isinstance(s, torch.Tensor) for s in self._keys):
+            dense = self._materialize_all()
+            if dense is not None:
+                return dense
         keys = [_materialize(s) for s in self._keys]
         values = [_materialize(s) for s in self._values]
         if self._pending_key is not None:

@@ -84,11 +84,13 @@ def test_captured_get_outlives_the_descriptor_table():
         assert all(torch.equal(a[..., :512, :], b[..., :512, :]) for a, b in zip(got, ref))
 
 
-def test_get_of_dense_pieces_alone():
+@pytest.mark.parametrize("T,table", [(90, False), (8191, False), (8192, True)])
+def test_get_of_dense_pieces_alone(T, table):
+    """Two copies for few elements, the one-launch kernel over a descriptor table for 2^20 and more."""
     import dartkv_amd as dart
-    k = torch.randn(1, 2, 90, 64, device=DEV).to(BF)
-    cache = dart.DartKVCache(dart.DartKVCacheConfig(sink_tokens=32, hold_partial_pages=True))
+    k = torch.randn(1, 2, T, 64, device=DEV).to(BF)
+    cache = dart.DartKVCache(dart.DartKVCacheConfig(sink_tokens=32, page_size=10000, hold_partial_pages=True))
     cache.append(k, -k)
     got_k, got_v = cache.get()
     assert torch.equal(got_k, k) and torch.equal(got_v, -k) and got_k.data_ptr() != k.data_ptr()
-    assert cache._decode_plan_cache is None  # no descriptor table is made for it
+    assert (cache._decode_plan_cache is not None) == table
